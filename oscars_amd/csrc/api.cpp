@@ -60,7 +60,7 @@ hipError_t om_launch_lw_wave(const om::LwArgs* A, int mixed, hipStream_t s);
 hipError_t om_launch_omega_from_ev(const double* e, long n, double* om, double qe, double hbar, hipStream_t s);
 hipError_t om_launch_level_stats(const int* level, const unsigned char* conv, long n, unsigned long long* out,
                                  hipStream_t s);
-hipError_t om_launch_pd_point(const om::PdArgs* A, int mixed, int split, hipStream_t s);
+hipError_t om_launch_pd_point(const om::PdArgs* A, int mixed, hipStream_t s);
 hipError_t om_launch_finalize(const om::FinArgs* F, hipStream_t s);
 hipError_t om_launch_state_reset(const om::State* st, long npts, hipStream_t s);
 hipError_t om_launch_count_active(const om::State* st, long npts, int* out, hipStream_t s);
@@ -1312,7 +1312,7 @@ int power_density(om_context* ctx, int ip, const double* obs_xyz, long n_obs, co
         A.La = La;
         A.Lb = Lb;
         ctx->timer.begin(ctx->stream);
-        check(om_launch_pd_point(&A, mix ? 1 : 0, ctx->split, ctx->stream), "pd_point");
+        check(om_launch_pd_point(&A, mix ? 1 : 0, ctx->stream), "pd_point");
         ctx->timer.end(ctx->stream);
         Ldone = Lb;
         if (Lb >= stop_ext) break;

@@ -28,8 +28,8 @@
 //                     accumulation stay FP64 in both: with packed FP32
 //                     disabled, v_fma_f32 and v_fma_f64 issue at the same rate
 //                     on gfx950, so FP32 would cost accuracy and save nothing.
-//   pd_point_kernel   power density, one lane = one observation point, a level's
-//                     samples split over the S waves of a workgroup.  FP64
+//   pd_wave_kernel    power density, the lanes of a wave split between
+//                     observation points and a level's samples.  FP64
 //                     variant: the reference's operations; mixed variant:
 //                     reciprocal square root and reciprocal refined by Newton
 //                     steps instead of the square root and quotients, with an
@@ -359,10 +359,12 @@ __global__ void __launch_bounds__(64 * S) lw_tile_kernel(LwArgs A, long n_tiles_
 }
 
 // ---------------------------------------------------------------- power density
-// One workgroup of S waves per 64 observation points (lane = point): wave w
-// sums the contiguous slice [ns*w/S, ns*(w+1)/S) of each level, the rows being
-// wave-uniform (scalar loads); the slices' partial sums are added in wave order
-// through LDS, so all waves hold the same totals and stop decisions.
+// Bound by the issue of the terms' instructions (FP64: ~112 per term, a square
+// root, a reciprocal and two quotients the most of them; mixed ~65).  The lanes
+// of a wave are split between points and the samples of a level
+// (pd_wave_kernel): one lane per point with the samples shared by the 8 waves of
+// a workgroup left most SIMDs idle on ordinary maps (51 x 51: 41 workgroups,
+// 0.43 ms where a wave per point takes 0.08 ms).
 //
 // MIXED = false: the reference's operations for each term (IEEE square root
 // and quotients).  MIXED = true: N = R / |R| from a Newton-refined reciprocal
@@ -418,7 +420,8 @@ __device__ __forceinline__ void pd_term(const PdArgs& A, V3 obs, V3 nrm, const d
   if (!MIXED) {
     double r2 = mag2(R);
     double m = sqrt(r2);
-    V3 N1 = v3(R.x / m, R.y / m, R.z / m);
+    double im = 1.0 / m;  // correctly rounded, so div_by gives the IEEE quotients
+    V3 N1 = v3(div_by(R.x, m, im), div_by(R.y, m, im), div_by(R.z, m, im));
     // src/OSCARSSR.cc:2908: a surface without normals takes N1.normal as 1
     double ndn = A.has_normal ? dot(N1, nrm) : 1.0;
     V3 Num = cross(N1, cross(sub(N1, B), Ac));
@@ -532,104 +535,80 @@ __device__ __forceinline__ V3 pd_normal(const PdArgs& A, long pc) {
                    : v3(A.normal[0], A.normal[1], A.normal[2]);
 }
 
-template <int S>
-struct PdLds {
-  double ps[S][64];
-  double ts[S][64];
-  double qs[S][64];
-  double xm[S][64];
-};
-
-template <bool MIXED, int S>
-__global__ void __launch_bounds__(64 * S) pd_point_kernel(PdArgs A) {
-  __shared__ PdLds<S> sh;
-  const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
-  long g = (long) blockIdx.x * 64 + lane;
-  bool valid;
-  long p;
-  if (A.list) {  // compacted: the points still active at this level
-    valid = g < A.n_list;
-    p = valid ? (long) A.list[g] : 0;
-  } else {
-    valid = g < A.npts;
-    p = g;
+// P x R points per wave: 64 / P lanes per group of R points (small maps, later
+// levels, the mixed path's FP64 recheck).  Lane j of a group sums samples j,
+// j + 64/P, ... of each level for its R points, from rows loaded one step ahead,
+// and the lanes' partial sums are combined by a butterfly in a fixed order, so
+// every lane of the group holds the same totals and takes the same decisions.
+template <bool MIXED, int P, int R>
+__global__ void __launch_bounds__(64) pd_wave_kernel(PdArgs A) {
+  constexpr int Q = 64 / P;
+  const int lane = threadIdx.x;
+  const int q0 = lane / P;
+  V3 obs[R], nrm[R];
+  PdPoint q[R];
+  long pc[R];
+  bool active[R], mine[R], done[R];
+  bool any = false;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const long g = ((long) blockIdx.x * R + r) * P + lane % P;
+    const bool valid = g < (A.list ? A.n_list : A.npts);
+    pc[r] = A.list ? (long) A.list[valid ? g : 0] : (valid ? g : 0);
+    obs[r] = v3(A.obs[3 * pc[r]], A.obs[3 * pc[r] + 1], A.obs[3 * pc[r] + 2]);
+    nrm[r] = pd_normal(A, pc[r]);
+    q[r] = pd_load<MIXED>(A, pc[r]);
+    active[r] = valid && !A.st.conv[pc[r]] && q[r].lev == A.La - 1;
+    mine[r] = active[r];
+    done[r] = false;
+    any = any || active[r];
   }
-  long pc = valid ? p : 0;
-  V3 obs = v3(A.obs[3 * pc], A.obs[3 * pc + 1], A.obs[3 * pc + 2]);
-  V3 nrm = pd_normal(A, pc);
-  PdPoint q = pd_load<MIXED>(A, pc);
-  bool active = valid && !A.st.conv[pc] && q.lev == A.La - 1;
-  for (int L = A.La; L <= A.Lb; ++L) {
-    if (S > 1 ? !__syncthreads_or(active) : !__any(active)) break;
+  for (int L = A.La; L <= A.Lb && __any(any); ++L) {
     const double* __restrict__ rows = A.lv.rows[L];
-    long ns = 1L << L;
-    long i0 = ns * w / S, i1 = ns * (w + 1) / S;
-    double ps = 0, tsum = 0, qsum = 0, xmin = 2.0;
-    for (long i = i0; i < i1; ++i) pd_term<MIXED>(A, obs, nrm, rows + 10 * i, ps, tsum, qsum, xmin);
-    if (S > 1) {
-      sh.ps[w][lane] = ps;
-      if (MIXED) {
-        sh.ts[w][lane] = tsum;
-        sh.qs[w][lane] = qsum;
-        sh.xm[w][lane] = xmin;
-      }
-      __syncthreads();
-      ps = 0;
-      tsum = 0;
-      qsum = 0;
-      xmin = 2.0;
-      for (int v = 0; v < S; ++v) {
-        long j0 = ns * v / S, j1 = ns * (v + 1) / S;
-        if (j1 <= j0) continue;
-        ps += sh.ps[v][lane];
+    const long ns = 1L << L;
+    double ps[R], tsum[R], qsum[R], xmin[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      ps[r] = tsum[r] = qsum[r] = 0;
+      xmin[r] = 2.0;
+    }
+    double cur[10], nxt[10];
+    const long i0 = q0 < ns ? q0 : 0;
+#pragma unroll
+    for (int k = 0; k < 10; ++k) nxt[k] = rows[10 * i0 + k];
+    for (long i = q0; i < ns; i += Q) {
+#pragma unroll
+      for (int k = 0; k < 10; ++k) cur[k] = nxt[k];
+      const long in = i + Q < ns ? i + Q : i;
+#pragma unroll
+      for (int k = 0; k < 10; ++k) nxt[k] = rows[10 * in + k];
+#pragma unroll
+      for (int r = 0; r < R; ++r) pd_term<MIXED>(A, obs[r], nrm[r], cur, ps[r], tsum[r], qsum[r], xmin[r]);
+    }
+    any = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      for (int off = 32; off >= P; off >>= 1) {
+        ps[r] += __shfl_xor(ps[r], off);
         if (MIXED) {
-          tsum += sh.ts[v][lane];
-          qsum += sh.qs[v][lane];
-          xmin = fmin(xmin, sh.xm[v][lane]);
+          tsum[r] += __shfl_xor(tsum[r], off);
+          qsum[r] += __shfl_xor(qsum[r], off);
+          xmin[r] = fmin(xmin[r], __shfl_xor(xmin[r], off));
         }
       }
-      // the next level's __syncthreads_or keeps these reads ahead of its writes
-    }
-    if (active && pd_level_end<MIXED>(A, L, ps, tsum, qsum, xmin, q)) {
-      A.st.conv[pc] = 1;
-      active = false;
-    }
-  }
-  if (w == 0 && valid && q.lev >= A.La) pd_store<MIXED>(A, pc, q);
-}
-
-// One wave per listed point (few points left, or the mixed path's FP64
-// recheck): lane j sums samples j, j + 64, ... of each level, and the lanes'
-// partial sums are combined by a butterfly in a fixed order, so every lane
-// holds the same total and takes the same decision.
-template <bool MIXED>
-__global__ void __launch_bounds__(64) pd_wave_kernel(PdArgs A) {
-  const int lane = threadIdx.x;
-  long pc = A.list[blockIdx.x];
-  V3 obs = v3(A.obs[3 * pc], A.obs[3 * pc + 1], A.obs[3 * pc + 2]);
-  V3 nrm = pd_normal(A, pc);
-  PdPoint q = pd_load<MIXED>(A, pc);
-  if (A.st.conv[pc] || q.lev != A.La - 1) return;
-  for (int L = A.La; L <= A.Lb; ++L) {
-    const double* __restrict__ rows = A.lv.rows[L];
-    long ns = 1L << L;
-    double ps = 0, tsum = 0, qsum = 0, xmin = 2.0;
-    for (long i = lane; i < ns; i += 64) pd_term<MIXED>(A, obs, nrm, rows + 10 * i, ps, tsum, qsum, xmin);
-    for (int off = 32; off > 0; off >>= 1) {
-      ps += __shfl_xor(ps, off);
-      if (MIXED) {
-        tsum += __shfl_xor(tsum, off);
-        qsum += __shfl_xor(qsum, off);
-        xmin = fmin(xmin, __shfl_xor(xmin, off));
+      if (active[r] && pd_level_end<MIXED>(A, L, ps[r], tsum[r], qsum[r], xmin[r], q[r])) {
+        done[r] = true;
+        active[r] = false;
       }
-    }
-    if (pd_level_end<MIXED>(A, L, ps, tsum, qsum, xmin, q)) {
-      if (lane == 0) A.st.conv[pc] = 1;
-      break;
+      any = any || active[r];
     }
   }
-  if (lane == 0 && q.lev >= A.La) pd_store<MIXED>(A, pc, q);
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (q0 == 0 && mine[r]) {
+      if (done[r]) A.st.conv[pc[r]] = 1;
+      if (q[r].lev >= A.La) pd_store<MIXED>(A, pc[r], q[r]);
+    }
 }
 
 // ---------------------------------------------------------------- power density on STL triangles
@@ -1276,37 +1255,27 @@ extern "C" hipError_t om_launch_tile_list(const om::State* st, long n_obs, long 
   return hipGetLastError();
 }
 
-// Power density: S waves per 64 points, chosen so that the grid holds about
-// 8192 waves (at least 8 per SIMD) unless split > 0 names S; a list of at most
-// kPdWaveListMax points runs one wave per point.
-constexpr long kPdWaveListMax = 8192;
-extern "C" hipError_t om_launch_pd_point(const om::PdArgs* A, int mixed, int split, hipStream_t s) {
-  if (A->list && A->n_list <= kPdWaveListMax && split <= 0) {  // few points: one wave each
-    if (mixed) hipLaunchKernelGGL(om::pd_wave_kernel<true>, dim3((unsigned) A->n_list), dim3(64), 0, s, *A);
-    else hipLaunchKernelGGL(om::pd_wave_kernel<false>, dim3((unsigned) A->n_list), dim3(64), 0, s, *A);
-    return hipGetLastError();
-  }
-  long groups = ((A->list ? A->n_list : A->npts) + 63) / 64;
-  if (split <= 0) {
-    split = 1;
-    while (split < 8 && groups * split < 8192) split *= 2;
-  }
-  dim3 g((unsigned) groups);
-  if (mixed) {
-    switch (split) {
-      case 1: hipLaunchKernelGGL((om::pd_point_kernel<true, 1>), g, dim3(64), 0, s, *A); break;
-      case 2: hipLaunchKernelGGL((om::pd_point_kernel<true, 2>), g, dim3(128), 0, s, *A); break;
-      case 4: hipLaunchKernelGGL((om::pd_point_kernel<true, 4>), g, dim3(256), 0, s, *A); break;
-      default: hipLaunchKernelGGL((om::pd_point_kernel<true, 8>), g, dim3(512), 0, s, *A); break;
-    }
-  } else {
-    switch (split) {
-      case 1: hipLaunchKernelGGL((om::pd_point_kernel<false, 1>), g, dim3(64), 0, s, *A); break;
-      case 2: hipLaunchKernelGGL((om::pd_point_kernel<false, 2>), g, dim3(128), 0, s, *A); break;
-      case 4: hipLaunchKernelGGL((om::pd_point_kernel<false, 4>), g, dim3(256), 0, s, *A); break;
-      default: hipLaunchKernelGGL((om::pd_point_kernel<false, 8>), g, dim3(512), 0, s, *A); break;
-    }
-  }
+template <int P, int R>
+static void launch_pd_wave(const om::PdArgs* A, int mixed, hipStream_t s) {
+  const long n = A->list ? A->n_list : A->npts;
+  dim3 g((unsigned) ((n + P * R - 1) / (P * R)));
+  if (mixed) hipLaunchKernelGGL((om::pd_wave_kernel<true, P, R>), g, dim3(64), 0, s, *A);
+  else hipLaunchKernelGGL((om::pd_wave_kernel<false, P, R>), g, dim3(64), 0, s, *A);
+}
+
+// Power density: a wave per point while that leaves SIMDs to fill, then fewer
+// lanes per point, so that more of a loaded row's lanes share its address, and
+// for the largest maps two points per lane.  Measured (1 point per wave / 2 / 8
+// as 4 x 2; FP64, planar magnet at +-5 mm): 2601 points 77 / 96 / 175 us, 5625
+// points 136 / 133 / 180, 22801 points 398 / 389 / 405, 40401 points 687 / 632 /
+// 655, 160801 points 2.71 / 2.34 / 2.22 ms; the mixed terms on an EPU's 40401
+// and 160801 points 389 / 318 / 303 us and 1.40 / 1.10 / 0.88 ms.
+constexpr long kPdOneMax = 4096, kPdTwoMax = 32768;
+extern "C" hipError_t om_launch_pd_point(const om::PdArgs* A, int mixed, hipStream_t s) {
+  const long n = A->list ? A->n_list : A->npts;
+  if (n <= kPdOneMax) launch_pd_wave<1, 1>(A, mixed, s);
+  else if (n <= kPdTwoMax) launch_pd_wave<2, 1>(A, mixed, s);
+  else launch_pd_wave<4, 2>(A, mixed, s);
   return hipGetLastError();
 }
 
