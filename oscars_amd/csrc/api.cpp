@@ -33,7 +33,9 @@ hipError_t om_launch_lw_batch(const om::BatchArgs* A, int mixed, int n_groups, h
 hipError_t om_scratch_setup(int device, void** ptr, size_t* bytes);
 hipError_t om_launch_lw_batch_stages(const om::BatchArgs* A, int mixed, int n_groups, int stages, hipStream_t s);
 hipError_t om_launch_rk4(const om::FieldDev* F, const om::FieldDev* F0_host, int nfields, om::TrajDesc* desc,
-                         int np, double* t, double* p, hipStream_t s, int nefields);
+                         int np, double* t, double* p, hipStream_t s, int nefields, int* shot);
+int om_shoot_steps(const om::FieldDev* F0_host, int nfields);
+hipError_t om_launch_shoot(const om::ShootArgs* A, const om::FieldDev* F0_host, hipStream_t s);
 hipError_t om_launch_knot_finish(double* p, long total, hipStream_t s);
 hipError_t om_launch_field_points(const om::FieldDev* F, int nf, const double* xyz, long n, double t, double* out,
                                   hipStream_t s);
@@ -258,6 +260,20 @@ struct om_context {
   std::vector<om_particle> parts;
   std::vector<LevelCache> levels;
   DevBuf<om::FieldDev> d_fields;
+  // segmented integration (shoot.hip): chains of the current particles, none
+  // (nblocks 0) where the steps are taken in order
+  struct Shoot {
+    int nchains = 0, nblocks = 0;
+    std::vector<om::ShootChain> chain;
+    std::vector<int> block_chain, flags;
+    DevBuf<om::ShootChain> d_chain;
+    DevBuf<int> d_block_chain, d_flags;  // flags: done, arrived per chain; joins agree, 2 per workgroup
+    DevBuf<double> maps;
+    PinnedStage stage;
+    void release() {
+      d_chain.release(); d_block_chain.release(); d_flags.release(); maps.release(); stage.release();
+    }
+  } shoot;
   std::vector<DevBuf<double>> grid_bufs;
   // work buffers
   DevBuf<double> d_obs, d_omega, d_sum, d_err, d_lastmag, d_prec, d_out, d_outcomp, d_oute;
@@ -349,6 +365,7 @@ struct om_context {
   ~om_context() {
     batch.release();
     adj.release();
+    shoot.release();
     free_levels();
     for (auto& g : grid_bufs) g.release();
     d_desc.release(); d_t.release(); d_p.release(); d_ypp.release(); d_u.release(); d_fields.release();
@@ -729,13 +746,92 @@ void finish_outputs(om_context* ctx, om::FinArgs& F, long npts, double* out_valu
   }
 }
 
+// Chains of the resident descriptors for the segmented integration, and its
+// workspace.  Chains shorter than kShootMinSteps, and particles with electric
+// fields (their sqrt(1 - beta^2) leaves no room for estimates off the energy
+// shell), are stepped in order.
+constexpr long kShootMinSteps = 1500;
+// Workgroups in all, shared by the chains (at least one each): one per CU, so
+// that the launches of several contexts can be resident at once.
+constexpr long kShootBlocks = 256;
+
+void shoot_setup(om_context* ctx, int np) {
+  auto& S = ctx->shoot;
+  S.nchains = S.nblocks = 0;
+  long longest = 0, total = 0;
+  for (int i = 0; i < np; ++i) {
+    longest = std::max(longest, std::max(ctx->desc[i].nf, ctx->desc[i].nb));
+    total += ctx->desc[i].nf + ctx->desc[i].nb;
+  }
+  if (ctx->nefields > 0 || longest < kShootMinSteps) return;
+  om::FieldDev none;
+  std::memset(&none, 0, sizeof(none));
+  const long per_step = 8L * om::kShootWaves;  // segments of a workgroup
+  long steps = om_shoot_steps(ctx->nfields > 0 ? &ctx->fields_host[0] : &none, ctx->nfields);
+  const long spare = std::max(1L, kShootBlocks - 2L * np);
+  steps = std::max(steps, (total + per_step * spare - 1) / (per_step * spare));
+  S.chain.clear();
+  S.block_chain.clear();
+  for (int i = 0; i < np; ++i)
+    for (int dir = 0; dir < 2; ++dir) {
+      om::ShootChain C;
+      C.ip = i;
+      C.dir = dir;
+      C.n = dir ? ctx->desc[i].nb : ctx->desc[i].nf;
+      C.block0 = (int) S.block_chain.size();
+      const bool one = 2L * np >= kShootBlocks;  // a workgroup each
+      C.nblock = C.n < 1 ? 0 : one ? 1 : (int) ((C.n + per_step * steps - 1) / (per_step * steps));
+      C.steps = C.nblock ? (int) ((C.n + per_step * C.nblock - 1) / (per_step * C.nblock)) : 1;
+      S.block_chain.insert(S.block_chain.end(), C.nblock, (int) S.chain.size());
+      S.chain.push_back(C);
+    }
+  S.nchains = (int) S.chain.size();
+  S.nblocks = (int) S.block_chain.size();
+  S.maps.ensure(84 * (size_t) S.nblocks);
+  S.flags.assign(2 * (size_t) S.nchains + 2 * (size_t) S.nblocks, 0);
+  // the lists in one staging buffer: it is rewritten only after its copies have run
+  const size_t cb = S.chain.size() * sizeof(om::ShootChain), bb = S.block_chain.size() * sizeof(int),
+               fb = S.flags.size() * sizeof(int);
+  S.d_chain.ensure(S.chain.size());
+  S.d_block_chain.ensure(S.block_chain.size());
+  S.d_flags.ensure(S.flags.size());
+  char* h = static_cast<char*>(S.stage.get(cb + bb + fb));
+  std::memcpy(h, S.chain.data(), cb);
+  std::memcpy(h + cb, S.block_chain.data(), bb);
+  std::memcpy(h + cb + bb, S.flags.data(), fb);
+  check(hipMemcpyAsync(S.d_chain.p, h, cb, hipMemcpyHostToDevice, ctx->stream), "upload");
+  check(hipMemcpyAsync(S.d_block_chain.p, h + cb, bb, hipMemcpyHostToDevice, ctx->stream), "upload");
+  check(hipMemcpyAsync(S.d_flags.p, h + cb + bb, fb, hipMemcpyHostToDevice, ctx->stream), "upload");
+  S.stage.queued(ctx->stream);
+}
+
 // RK4 + knot finish + spline for the resident descriptors (also used inside
 // graph capture by the batched path).
 void launch_trajectories(om_context* ctx, int np) {
   om::FieldDev none;
   std::memset(&none, 0, sizeof(none));
-  check(om_launch_rk4(ctx->d_fields.p, ctx->nfields > 0 ? &ctx->fields_host[0] : &none, ctx->nfields,
-                      ctx->d_desc.p, np, ctx->d_t.p, ctx->d_p.p, ctx->stream, ctx->nefields), "rk4");
+  const om::FieldDev* F0 = ctx->nfields > 0 ? &ctx->fields_host[0] : &none;
+  int* shot = nullptr;
+  if (ctx->shoot.nblocks > 0) {
+    auto& S = ctx->shoot;
+    om::ShootArgs A;
+    A.F = ctx->d_fields.p;
+    A.nf = ctx->nfields;
+    A.desc = ctx->d_desc.p;
+    A.chain = S.d_chain.p;
+    A.block_chain = S.d_block_chain.p;
+    A.nblocks = S.nblocks;
+    A.Mb = S.maps.p;
+    A.done = S.d_flags.p;
+    A.arrived = S.d_flags.p + S.nchains;
+    A.block_ok = S.d_flags.p + 2 * S.nchains;
+    A.t = ctx->d_t.p;
+    A.p = ctx->d_p.p;
+    check(om_launch_shoot(&A, F0, ctx->stream), "trajectory segments");
+    shot = S.d_flags.p;
+  }
+  check(om_launch_rk4(ctx->d_fields.p, F0, ctx->nfields, ctx->d_desc.p, np, ctx->d_t.p, ctx->d_p.p, ctx->stream,
+                      ctx->nefields, shot), "rk4");
   if (ctx->adj.armed) {
     // states every K steps of particle 0, taken from the raw knots before the division by c
     auto& A = ctx->adj;
@@ -1062,6 +1158,7 @@ int om_trajectories_eb(om_context* ctx, const om_field* fields, int nfields, con
     ctx->d_ppv.ensure(total);
     ctx->d_u2.ensure(9 * total);
     upload_staged(ctx, ctx->stage_desc, ctx->d_desc, ctx->desc.data(), np);
+    shoot_setup(ctx, np);
     launch_trajectories(ctx, np);
     // The integration runs on; its status is read back by the first call that
     // needs it (sync_desc), so the host can queue other work meanwhile.

@@ -103,6 +103,35 @@ struct FinArgs {
   unsigned char* out_conv;
 };
 
+// ---- trajectories in parallel segments (shoot.hip)
+constexpr int kShootWaves = 4;   // waves per workgroup, eight segments each
+constexpr int kShootWalk = 64;   // maps of other workgroups held in LDS at a time
+
+// One particle's forward or backward chain of steps.
+struct ShootChain {
+  int ip, dir;         // particle; 0 forward, 1 backward
+  int block0, nblock;  // its workgroups
+  int steps;           // per segment
+  long n;              // steps
+};
+
+struct ShootArgs {
+  const FieldDev* F;
+  int nf;
+  const TrajDesc* desc;
+  const ShootChain* chain;
+  const int* block_chain;  // chain of each workgroup
+  int nblocks;
+  double* Mb;      // 2 x 42 per workgroup: composed map of its segments, by the round's parity
+  int* block_ok;   // 2 per workgroup: its joins agree
+  // per chain (two per particle: forward, backward); all zero before the launch,
+  // and zeroed again by rk4_kernel once it has read them
+  int* done;       // accepted
+  int* arrived;    // workgroups arrived, all rounds together
+  double* t;
+  double* p;
+};
+
 // ---- level samples (traj.hip, batch.hip)
 struct LevelJob {
   const double* t;     // packed knot times

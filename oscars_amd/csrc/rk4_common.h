@@ -588,6 +588,18 @@ __device__ __forceinline__ bool rk4(RkCtx& c, const UndParams& f0, double* y, do
   return true;
 }
 
+// The knot is stored with velocity and acceleration in SI units; knot_finish_kernel
+// divides them by c afterwards (in parallel), which keeps six divisions off the
+// sequential RK4 chain and gives the same doubles.
+__device__ __forceinline__ void store_knot(double* __restrict__ t, double* __restrict__ p, long k, double tt,
+                                           const double* x, const double* d) {
+  t[k] = tt;
+  double* o = p + 9 * k;
+  o[0] = x[0]; o[1] = x[2]; o[2] = x[4];
+  o[3] = x[1]; o[4] = x[3]; o[5] = x[5];
+  o[6] = d[1]; o[7] = d[3]; o[8] = d[5];
+}
+
 // Knot interval of x: a first guess from the (nearly) uniform knot grid, then
 // moved to the reference bisection's answer (largest klo <= n-2 with
 // t[klo] <= x), which is exact for increasing knots (include/TOMATH.h:92-126).

@@ -15,26 +15,13 @@
 // doubles (t x y z bx by bz ax ay az); level L of a particle starts at row
 // 2^L - 1 of that particle's level block, so one 80-byte row is what every
 // lane of a wave reads when it walks the trajectory.
-#include <string.h>
-
 #include "om_device.h"
 #include "launch_types.h"
 #include "om_types.h"
 #include "rk4_common.h"
+#include "rk4_variant.h"
 
 namespace om {
-
-// The knot is stored with velocity and acceleration in SI units; knot_finish_kernel
-// divides them by c afterwards (in parallel), which keeps six divisions off the
-// sequential RK4 chain and gives the same doubles.
-__device__ __forceinline__ void store_knot(double* __restrict__ t, double* __restrict__ p, long k, double tt,
-                                           const double* x, const double* d) {
-  t[k] = tt;
-  double* o = p + 9 * k;
-  o[0] = x[0]; o[1] = x[2]; o[2] = x[4];
-  o[3] = x[1]; o[4] = x[3]; o[5] = x[5];
-  o[6] = d[1]; o[7] = d[3]; o[8] = d[5];
-}
 
 __global__ void __launch_bounds__(256) knot_finish_kernel(double* __restrict__ p, long total) {
   long i = (long) blockIdx.x * blockDim.x + threadIdx.x;
@@ -285,7 +272,8 @@ constexpr int rk4_lanes() {
 template <int M>
 __global__ void __launch_bounds__(64) rk4_kernel(const UndParams f_arg, const GridZ g, const FieldDev* __restrict__ F,
                                                  int nfields, TrajDesc* __restrict__ desc, int np,
-                                                 double* __restrict__ t, double* __restrict__ p, int nefields) {
+                                                 double* __restrict__ t, double* __restrict__ p, int nefields,
+                                                 int* __restrict__ shot) {
   extern __shared__ double lds_grid[];
   // Highest issue priority for these waves: the integration is one dependent
   // chain per particle, and when it runs beside other kernels (the previous
@@ -298,13 +286,28 @@ __global__ void __launch_bounds__(64) rk4_kernel(const UndParams f_arg, const Gr
   const int dir = sub / (P / 2);                   // 0 forward, 1 backward
   const int slot = M == kEpuZ ? (sub >> 1) & 1 : sub & 1;  // the stage of a field pair this lane evaluates
   RkCtx c{F, nfields, 0.0, 0, g, nefields, 0.0, 0};
+  // the knots are there already (an empty backward chain has nothing to do); the
+  // flags are cleared for the next launch, by the lanes that have all read them
+  const bool shot_f = shot && ip < np && shot[2 * ip];
+  const bool shot_b = shot && ip < np && (shot[2 * ip + 1] || desc[ip].nb == 0);
+  const bool skip = ip >= np || (shot_f && shot_b);
+  __syncthreads();
+  if (shot && ip < np && sub < 2) {
+    shot[2 * ip + sub] = 0;             // done
+    shot[2 * np + 2 * ip + sub] = 0;    // arrived
+  }
+  if (skip && ip < np && sub == 0) {
+    desc[ip].status = 0;
+    desc[ip].halved = 0;
+  }
+  if (__all(skip)) return;  // the workgroup is one wave
   if (M == kGridZ) {
     // stage the map in LDS (all lanes), then integrate
     for (long i = threadIdx.x; i < 3 * g.n; i += blockDim.x) lds_grid[i] = g.data[i];
     __syncthreads();
     c.g.data = lds_grid;
   }
-  if (ip >= np) return;  // all lanes of a particle together
+  if (skip) return;  // all lanes of a particle together
   // the single undulator's constants, in vector registers (see in_vgpr)
   UndParams f0 = (M == kOneUndulator || (M >= kAxisUndX && M <= kAxisUndZ) || M == kUndZ || M == kEpuZ)
                      ? und_in_vgpr(f_arg) : f_arg;
@@ -624,103 +627,40 @@ __global__ void __launch_bounds__(256) beta_diff_kernel(const double* __restrict
 }  // namespace om
 
 // ---------------------------------------------------------------- launchers (host)
+namespace {
+template <int M>
+hipError_t launch_rk4(const om::Rk4Variant& v, const om::FieldDev* F, int nfields, om::TrajDesc* desc, int np,
+                      double* t, double* p, hipStream_t s, int nefields, int* shot) {
+  const int threads = 64, blocks = (np * om::rk4_lanes<M>() + threads - 1) / threads;
+  if (v.grid_bytes > 0) {
+    hipError_t e = hipFuncSetAttribute((const void*) om::rk4_kernel<M>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int) v.grid_bytes);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(om::rk4_kernel<M>, dim3(blocks), dim3(threads), v.grid_bytes, s, v.und, v.grid, F, nfields, desc,
+                     np, t, p, nefields, shot);
+  return hipGetLastError();
+}
+}  // namespace
+
+// shot: null, or the flags of the segmented integration (shoot.hip), which has
+// already left the knots where they are set: done (forward, backward) of each
+// particle, then the arrival counters.  They are cleared here.
 extern "C" hipError_t om_launch_rk4(const om::FieldDev* F, const om::FieldDev* F0_host, int nfields,
                                     om::TrajDesc* desc, int np, double* t, double* p, hipStream_t s,
-                                    int nefields) {
-  if (nefields > 0) {
-    // electric fields (after the magnetic ones in F): the general equations of motion
-    om::UndParams u0;
-    memset(&u0, 0, sizeof(u0));
-    om::GridZ g0;
-    memset(&g0, 0, sizeof(g0));
-    int threads0 = 64, blocks0 = (np * om::rk4_lanes<om::kFieldsEB>() + threads0 - 1) / threads0;
-    hipLaunchKernelGGL(om::rk4_kernel<om::kFieldsEB>, dim3(blocks0), dim3(threads0), 0, s, u0, g0, F, nfields, desc,
-                       np, t, p, nefields);
-    return hipGetLastError();
+                                    int nefields, int* shot) {
+  const om::Rk4Variant v = om::rk4_variant(*F0_host, nfields, nefields);
+  switch (v.m) {
+    case om::kFieldsEB: return launch_rk4<om::kFieldsEB>(v, F, nfields, desc, np, t, p, s, nefields, shot);
+    case om::kGridZ: return launch_rk4<om::kGridZ>(v, F, nfields, desc, np, t, p, s, 0, shot);
+    case om::kAxisUndX: return launch_rk4<om::kAxisUndX>(v, F, nfields, desc, np, t, p, s, 0, shot);
+    case om::kAxisUndY: return launch_rk4<om::kAxisUndY>(v, F, nfields, desc, np, t, p, s, 0, shot);
+    case om::kAxisUndZ: return launch_rk4<om::kAxisUndZ>(v, F, nfields, desc, np, t, p, s, 0, shot);
+    case om::kUndZ: return launch_rk4<om::kUndZ>(v, F, nfields, desc, np, t, p, s, 0, shot);
+    case om::kEpuZ: return launch_rk4<om::kEpuZ>(v, F, nfields, desc, np, t, p, s, 0, shot);
+    case om::kOneUndulator: return launch_rk4<om::kOneUndulator>(v, F, nfields, desc, np, t, p, s, 0, shot);
+    default: return launch_rk4<om::kFieldsGeneric>(v, F, nfields, desc, np, t, p, s, 0, shot);
   }
-  int threads = 64;
-  // rk4_lanes lanes per particle: 4 (two per direction), 8 for kEpuZ
-  int blocks = (np * 4 + threads - 1) / threads;   // every variant but kEpuZ
-  int blocks8 = (np * 8 + threads - 1) / threads;  // kEpuZ
-  static_assert(om::rk4_lanes<om::kEpuZ>() == 8 && om::rk4_lanes<om::kAxisUndY>() == 4 &&
-                    om::rk4_lanes<om::kOneUndulator>() == 4 && om::rk4_lanes<om::kFieldsGeneric>() == 4,
-                "lanes per particle");
-  om::UndParams u;
-  memset(&u, 0, sizeof(u));
-  om::GridZ g;
-  memset(&g, 0, sizeof(g));
-  const om::FieldDev& f = *F0_host;
-  // one z grid without rotation whose samples fit in LDS: the staged-grid variant
-  const size_t grid_bytes = (size_t) 3 * f.n[2] * sizeof(double);
-  // the specialised variants hold time-independent fields only
-  if (nfields == 1 && !f.td && f.type == om::kGrid && f.axis == 2 && f.rot_sin[0] == 0 && f.rot_sin[1] == 0 &&
-      f.rot_sin[2] == 0 && f.rot_cos[0] == 1 && f.rot_cos[1] == 1 && f.rot_cos[2] == 1 &&
-      grid_bytes <= 160 * 1024) {
-    g.data = f.data;
-    g.n = f.n[2];
-    g.start = f.start[2];
-    g.stop = f.stop[2];
-    g.step = f.step[2];
-    g.inv_step = f.inv_step[2];
-    g.trans = f.trans[2];
-    hipError_t e = hipFuncSetAttribute((const void*) om::rk4_kernel<om::kGridZ>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int) grid_bytes);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(om::rk4_kernel<om::kGridZ>, dim3(blocks), dim3(threads), grid_bytes, s, u, g, F, nfields, desc,
-                       np, t, p, 0);
-    return hipGetLastError();
-  }
-  if (nfields == 1 && !f.td && (f.type == om::kUndulator || f.type == om::kEPU)) {
-    u.c0 = f.center[0]; u.c1 = f.center[1]; u.c2 = f.center[2];
-    u.u0 = f.unit[0]; u.u1 = f.unit[1]; u.u2 = f.unit[2];
-    u.taper = f.taper;
-    u.half_len = f.und_length / 2.;
-    u.PL = f.period_length;
-    u.inv_PL = f.inv_period_length;
-    u.half_PL = f.period_length / 2.;
-    u.psA = f.phase_shift_a;
-    u.psB = f.phase_shift_b;
-    u.a0 = f.field[0]; u.a1 = f.field[1]; u.a2 = f.field[2];
-    u.b0 = f.fieldB[0]; u.b1 = f.fieldB[1]; u.b2 = f.fieldB[2];
-    u.epu = f.type == om::kEPU;
-    for (int k = 0; k < 2; ++k) {
-      double ps = k == 0 ? u.psA : u.psB;
-      double* th = k == 0 ? u.thA : u.thB;
-      th[0] = -u.half_len + ps;
-      th[1] = u.half_len + ps;
-      th[2] = -u.half_len + ps + u.PL;
-      th[3] = u.half_len + ps - u.PL;
-      th[4] = -u.half_len + ps + u.half_PL;
-      th[5] = u.half_len + ps - u.half_PL;
-    }
-    // planar undulator along z, untapered, field along one axis: the reduced equations
-    int nz = (f.field[0] != 0) + (f.field[1] != 0) + (f.field[2] != 0);
-    bool axis_z = f.unit[0] == 0 && f.unit[1] == 0 && f.unit[2] == 1;
-    if (f.type == om::kUndulator && axis_z && f.taper == 0 && nz == 1) {
-      if (f.field[0] != 0)
-        hipLaunchKernelGGL(om::rk4_kernel<om::kAxisUndX>, dim3(blocks), dim3(threads), 0, s, u, g, F, nfields, desc, np,
-                           t, p, 0);
-      else if (f.field[1] != 0)
-        hipLaunchKernelGGL(om::rk4_kernel<om::kAxisUndY>, dim3(blocks), dim3(threads), 0, s, u, g, F, nfields, desc, np,
-                           t, p, 0);
-      else
-        hipLaunchKernelGGL(om::rk4_kernel<om::kAxisUndZ>, dim3(blocks), dim3(threads), 0, s, u, g, F, nfields, desc, np,
-                           t, p, 0);
-    } else if (axis_z && f.taper == 0 && f.type == om::kEPU) {
-      hipLaunchKernelGGL(om::rk4_kernel<om::kEpuZ>, dim3(blocks8), dim3(threads), 0, s, u, g, F, nfields, desc, np, t,
-                         p, 0);
-    } else if (axis_z && f.taper == 0) {
-      hipLaunchKernelGGL(om::rk4_kernel<om::kUndZ>, dim3(blocks), dim3(threads), 0, s, u, g, F, nfields, desc, np, t,
-                         p, 0);
-    } else {
-      hipLaunchKernelGGL(om::rk4_kernel<om::kOneUndulator>, dim3(blocks), dim3(threads), 0, s, u, g, F, nfields, desc,
-                         np, t, p, 0);
-    }
-  } else {
-    hipLaunchKernelGGL(om::rk4_kernel<om::kFieldsGeneric>, dim3(blocks), dim3(threads), 0, s, u, g, F, nfields, desc, np,
-                       t, p, 0);
-  }
-  return hipGetLastError();
 }
 
 extern "C" hipError_t om_launch_knot_finish(double* p, long total, hipStream_t s) {

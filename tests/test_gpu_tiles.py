@@ -46,3 +46,81 @@ def test_power_density_sizes(epu_pair, n):
     assert np.array_equal(lev[-5:], fewlev) and rel_err(v[-5:], few) < 1e-12
     assert np.array_equal(lev, levm) and np.array_equal(cv, cvm)
     assert rel_err(vm, v, 1e-6) < 1e-5
+
+
+def _field(x, name):
+    from tests.common import EPU, UNDULATOR
+    if name == "epu":
+        x.add_bfield_epu(**EPU)
+    elif name == "map":
+        from oscars_amd import adjoint as A
+        x.add_bfield_grid([0, 0, -1.0], [0, 0, 5e-4], [1, 1, 4001], A.undulator_pole_map(4001, -1.0, 5e-4))
+    else:
+        bf = dict(x=[1, 0, 0], xy=[0.5, 1, 0], tapered=[0, 1, 0], pair=[0, 1, 0]).get(name, [0, 1, 0])
+        x.add_bfield_undulator(**dict(UNDULATOR, bfield=bf), **(dict(taper=0.05) if name == "tapered" else {}))
+        if name == "pair":
+            x.add_bfield_gaussian(bfield=[0.05, 0, 0], sigma=[0, 0, 0.2], translation=[0, 0, 0.3])
+
+
+@gpu
+@pytest.mark.parametrize("field", ["y", "x", "xy", "tapered", "epu", "map", "pair"])
+def test_trajectory_in_segments(field):
+    """Chains cut into segments and joined, one to 53 workgroups long, with
+    remainders, T0 at the start, inside and at the end of the window, beside
+    chains too short to be cut.  Against the oracle's integration in order: times equal; positions
+    along the trajectory within two units in the last place of 1 m (2^-52: the
+    joins agree to a fraction of one), transverse ones and velocities to 1e-12 of
+    their largest value (the device's sine differs from the C library's in the
+    last bit; with integration in order on the device the bar is the same)."""
+    from oracle.pyoracle import Oracle
+    from oscars_amd.sr import sr
+    windows = [(0, 2, 20001), (0, 0.15, 1500), (0, 0.1500001, 1502), (0, 0.3841, 3842), (-1, 1, 20001),
+               (-0.7, 0.1, 8002), (-1, 0, 6000), (0, 1.3, 1701)]
+
+    def setup(x):
+        x.set_particle_beam(energy_GeV=3, x0=[1e-5, 0, -0.6], d0=[1e-5, 2e-5, 1], current=0.5)
+        _field(x, field)
+
+    s = sr()
+    setup(s)
+    dev = s._device()
+    dev.trajectories(s._fields, [s._om_particle(s._particle, ctstart=a, ctstop=b, npoints=n) for a, b, n in windows])
+    for i, (a, b, n) in enumerate(windows):
+        o = Oracle(nthreads=1)
+        setup(o)
+        o.set_ctstartstop(a, b)
+        o.set_npoints_trajectory(n)
+        T = o.calculate_trajectory()
+        t, p, _ = dev.trajectory(i)
+        scale = np.max(np.abs(T.p), axis=0)
+        scale[scale == 0] = 1
+        err = np.max(np.abs(p - T.p) / scale, axis=0)
+        assert np.array_equal(t, T.t), (a, b, n)
+        assert np.max(np.abs(p[:, 2] - T.p[:, 2])) <= 2.0 ** -52 and np.max(err) < 1e-12, (a, b, n, err)
+
+
+@gpu
+def test_many_trajectories_in_segments():
+    """More chains than workgroups are given out to: one workgroup a chain, no
+    waiting between them.  The same particles in one call and alone (53
+    workgroups): z within two units in the last place of 1 m, the rest to 1e-12
+    of its largest value."""
+    from oscars_amd.sr import sr
+    from tests.common import UNDULATOR
+    s = sr()
+    s.set_particle_beam(energy_GeV=3, x0=[0, 0, -1], d0=[0, 0, 1], current=0.5)
+    s.add_bfield_undulator(**UNDULATOR)
+    r = np.random.default_rng(3)
+    parts = []
+    for i in range(150):
+        s.set_particle([2e-5 * r.standard_normal(), 0, -1], [2e-5 * r.standard_normal(), 0, 0.99999998])
+        parts.append(s._om_particle(s._particle, ctstart=-0.05, ctstop=1.9, npoints=int(r.integers(1600, 20001))))
+    dev = s._device()
+    dev.trajectories(s._fields, parts)
+    many = [dev.trajectory(i) for i in (0, 74, 149)]
+    for (t, p, _), i in zip(many, (0, 74, 149)):
+        dev.trajectories(s._fields, [parts[i]])
+        t1, p1, _ = dev.trajectory(0)
+        scale = np.maximum(np.max(np.abs(p1), axis=0), 1e-300)
+        assert np.array_equal(t, t1) and np.max(np.abs(p[:, 2] - p1[:, 2])) <= 2.0 ** -52
+        assert np.max(np.abs(p - p1) / scale) < 1e-12
