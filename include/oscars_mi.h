@@ -273,9 +273,9 @@ int om_flux_dev_noalloc(om_context* ctx, int particle, const double* obs_xyz, lo
  * trajectory lengths.  Levels 0..opts->max_level of every particle are stored
  * as sample rows; deeper levels are interpolated in the kernel, so every point
  * follows the conv's level rule; points unconverged at its last level are
- * counted in stats->n_unconverged.  With opts->deep_level set, points still
- * active at that level are finished by a workgroup per point (their samples
- * split over its waves).  MIXED mode: points whose stop decision lay within
+ * counted in stats->n_unconverged.  Points still active at opts->deep_level
+ * leave their work unit and go on level by level, a level's samples split over
+ * many waves.  MIXED mode: points whose stop decision lay within
  * the reduced-accuracy sin/cos error bound are recomputed with full-accuracy
  * sin/cos in the same run (stats->n_rechecked counts them), so stopping levels
  * match the FP64 kernel. */
@@ -291,8 +291,9 @@ typedef struct {
   int max_level;    /* highest level held as stored sample rows (0: up to 18 within 40% of the
                        device memory); deeper levels, up to the conv's max_level rule, are
                        interpolated */
-  int deep_level;   /* points still active at this level are finished one workgroup per point
-                       (0: none, every point finishes in its work unit) */
+  int deep_level;   /* points still active at this level leave their work unit and go on with
+                       their samples split over the GPU (0: chosen from the number of units; a
+                       level above the conv's last: none) */
 } om_batch_opts;
 
 int om_batch_setup(om_context* ctx, const om_request* req, int n_req, const int* req_of, const double* weight,

@@ -304,9 +304,11 @@ struct om_context {
     DevBuf<unsigned long long> counters, fix;
     DevBuf<double> ws;  // per persistent wave: the state of one unit's energies
     DevBuf<int> wsi;
-    DevBuf<unsigned long long> deep_code;  // points handed to the one-wave-per-point kernel
-    DevBuf<double> deep_state;
-    DevBuf<int> deep_level, deep_flags;
+    DevBuf<int> group_list, group_n;  // groups handed to the level kernels
+    DevBuf<long> group_item;
+    DevBuf<unsigned short> group_e;
+    DevBuf<unsigned> group_arrived;
+    DevBuf<double> group_state, part;
     om::BatchArgs args;
     hipGraphExec_t exec[2] = {nullptr, nullptr};  // [without, with] trajectory recomputation
     void drop_graphs() {
@@ -321,7 +323,8 @@ struct om_context {
       rows.release(); tspan.release(); obs.release(); omega.release(); out.release(); weight.release();
       req_of.release(); prefix.release(); req.release(); counters.release(); fix.release();
       ws.release(); wsi.release();
-      deep_code.release(); deep_state.release(); deep_level.release(); deep_flags.release();
+      group_list.release(); group_n.release(); group_item.release(); group_e.release();
+      group_arrived.release(); group_state.release(); part.release();
       ready = false;
     }
   } batch;
@@ -749,8 +752,13 @@ void finish_outputs(om_context* ctx, om::FinArgs& F, long npts, double* out_valu
 // Chains of the resident descriptors for the segmented integration, and its
 // workspace.  Chains shorter than kShootMinSteps, and particles with electric
 // fields (their sqrt(1 - beta^2) leaves no room for estimates off the energy
-// shell), are stepped in order.
+// shell), are stepped in order, and so are very many particles.
 constexpr long kShootMinSteps = 1500;
+// In order, a launch takes as long as its longest chain (0.62 us a step); in
+// segments, with more chains than the chip has CUs, as long as the steps of all
+// (1 ns each): 256 particles of 8001 to 20001 points 6 against 14 ms, 2048
+// particles 28 against 19 ms.
+constexpr long kShootMaxRatio = 512;
 // Workgroups in all, shared by the chains (at least one each): one per CU, so
 // that the launches of several contexts can be resident at once.
 constexpr long kShootBlocks = 256;
@@ -763,12 +771,14 @@ void shoot_setup(om_context* ctx, int np) {
     longest = std::max(longest, std::max(ctx->desc[i].nf, ctx->desc[i].nb));
     total += ctx->desc[i].nf + ctx->desc[i].nb;
   }
-  if (ctx->nefields > 0 || longest < kShootMinSteps) return;
+  if (ctx->nefields > 0 || longest < kShootMinSteps || total > kShootMaxRatio * longest) return;
   om::FieldDev none;
   std::memset(&none, 0, sizeof(none));
   const long per_step = 8L * om::kShootWaves;  // segments of a workgroup
   long steps = om_shoot_steps(ctx->nfields > 0 ? &ctx->fields_host[0] : &none, ctx->nfields);
-  const long spare = std::max(1L, kShootBlocks - 2L * np);
+  long chains = 0;
+  for (int i = 0; i < np; ++i) chains += (ctx->desc[i].nf > 0) + (ctx->desc[i].nb > 0);
+  const long spare = std::max(1L, kShootBlocks - chains);
   steps = std::max(steps, (total + per_step * spare - 1) / (per_step * spare));
   S.chain.clear();
   S.block_chain.clear();
@@ -779,7 +789,7 @@ void shoot_setup(om_context* ctx, int np) {
       C.dir = dir;
       C.n = dir ? ctx->desc[i].nb : ctx->desc[i].nf;
       C.block0 = (int) S.block_chain.size();
-      const bool one = 2L * np >= kShootBlocks;  // a workgroup each
+      const bool one = chains >= kShootBlocks;  // a workgroup each
       C.nblock = C.n < 1 ? 0 : one ? 1 : (int) ((C.n + per_step * steps - 1) / (per_step * steps));
       C.steps = C.nblock ? (int) ((C.n + per_step * C.nblock - 1) / (per_step * C.nblock)) : 1;
       S.block_chain.insert(S.block_chain.end(), C.nblock, (int) S.chain.size());
@@ -1743,10 +1753,18 @@ int om_power_density_dev(om_context* ctx, int ip, const double* obs_xyz, long n_
 // points listed for the FP64 recheck kernel, [4] handed over, [5] amplitudes,
 // [6] evals and [8] integrand lane slots inside the persistent kernel, [7]
 // points rechecked in FP64 inside their unit
-constexpr int kBatchCounters = 9;
+constexpr int kBatchReport = 9;  // counters om_batch_profile returns
+constexpr int kBatchCounters = kBatchReport + 1 + 4 * om::kBatchLevels;
 constexpr long kBatchFixCap = 1L << 27;
-constexpr long kBatchDeepCap = 1L << 22;
-constexpr int kBatchNoHandOver = 99;         // default hand-over level: none (above every level)
+constexpr long kBatchGroupCap = 1L << 17;  // groups handed over (4.8 KB each)
+constexpr int kBatchNoHandOver = 99;  // a hand-over level above every level: none
+// Default hand-over level, by the work units: as low as the groups that leave
+// (2.2 per unit at level 12, 0.8 at 14, 0.12 at 17 with 128 to 1024 energies a
+// point) find room for, since a unit that finds none keeps its slow energies.
+// 13664 units, levels 0 (none) / 11 / 12 / 13 / 14 / 16: 183 / 43.9 / 40.8 / 40.6 /
+// 42.8 / 51.7 ms; 304032 units, 0 / 12 / 14 / 16 / 17 / 18: 993 / 1159 / 1139 / 888 /
+// 886 / 889 ms; 1755904 units, 0 / 14 / 16 / 17 / 18: 5096 / 5482 / 5709 / 4845 / 4848.
+int batch_hand_over(long units) { return units <= 40000 ? 12 : units <= 120000 ? 14 : 17; }
 constexpr int kBatchRowsCap = 17;            // highest level stored as rows by default ...
 constexpr double kBatchRowsFraction = 0.4;   // ... within this fraction of the device memory
 
@@ -1758,6 +1776,28 @@ void batch_scratch(om_context* ctx, long groups, om::BatchArgs& A) {
   B.wsi.ensure((size_t) groups * om::kBatchWsI * om::kBatchEB);
   A.ws = B.ws.p;
   A.wsi = B.wsi.p;
+}
+
+// Room for the groups of energies handed to the level kernels: three per work
+// unit (most units hand over one or none; what finds no room stays in its unit).
+void batch_groups(om_context* ctx, om::BatchArgs& A) {
+  auto& B = ctx->batch;
+  A.group_cap = std::min(kBatchGroupCap, std::max(4096L, 3 * B.total_items));
+  B.group_list.ensure(4 * A.group_cap);
+  B.group_item.ensure(A.group_cap);
+  B.group_n.ensure(A.group_cap);
+  B.group_e.ensure(64 * A.group_cap);
+  B.group_state.ensure((size_t) om::kBatchGroupD * 64 * A.group_cap);
+  B.group_arrived.ensure(A.group_cap);
+  B.part.ensure((size_t) om::kBatchParts * 8 * 64);
+  check(om_launch_adj_key_fill(reinterpret_cast<int*>(B.group_arrived.p), A.group_cap, 0, ctx->stream), "clear");
+  A.group_list = B.group_list.p;
+  A.group_item = B.group_item.p;
+  A.group_n = B.group_n.p;
+  A.group_e = B.group_e.p;
+  A.group_state = B.group_state.p;
+  A.group_arrived = B.group_arrived.p;
+  A.part = B.part.p;
 }
 }  // namespace
 
@@ -1884,17 +1924,12 @@ int om_batch_setup(om_context* ctx, const om_request* req, int n_req, const int*
     A.main_evals = B.counters.p + 6;
     A.n_recheck = B.counters.p + 7;
     A.main_slots = B.counters.p + 8;
-    A.Ldeep = (opts && opts->deep_level > 0) ? opts->deep_level : kBatchNoHandOver;
+    A.Ldeep = (opts && opts->deep_level > 0) ? opts->deep_level : batch_hand_over(B.total_items);
     if (A.Ldeep < 9) throw std::out_of_range("deep_level must be at least 9");
-    A.deep_cap = total_points < kBatchDeepCap ? total_points : kBatchDeepCap;
-    B.deep_code.ensure(A.deep_cap);
-    B.deep_state.ensure((size_t) om::kBatchWsD * A.deep_cap);
-    B.deep_level.ensure(A.deep_cap);
-    B.deep_flags.ensure(A.deep_cap);
-    A.deep_code = B.deep_code.p;
-    A.deep_state = B.deep_state.p;
-    A.deep_level = B.deep_level.p;
-    A.deep_flags = B.deep_flags.p;
+    A.n_group = B.counters.p + kBatchReport;
+    A.n_list = B.counters.p + kBatchReport + 1;
+    A.n_job = A.n_list + 2 * om::kBatchLevels;
+    batch_groups(ctx, A);
     A.total_items = B.total_items;
     B.mixed = conv->mode == OM_MODE_MIXED ? 1 : 0;
     if (B.mixed) {
@@ -2010,7 +2045,7 @@ int om_batch_profile(om_context* ctx, int recompute_trajectories, double* stage_
     }
     unsigned long long cnt[kBatchCounters];
     read_back(ctx, cnt, B.counters.p, sizeof(cnt));
-    for (int i = 0; i < kBatchCounters; ++i) counts[i] = cnt[i];
+    for (int i = 0; i < kBatchReport; ++i) counts[i] = cnt[i];
     if (stats) {
       float ms = 0;
       check(hipEventElapsedTime(&ms, ev[0], ev[5]), "elapsed");

@@ -120,10 +120,74 @@ __device__ __forceinline__ Unit unit_of(const BatchArgs& A, long item) {
   return U;
 }
 
+// End of level L for one energy: the level's sum ps added, then the convergence
+// test of src/OSCARSSR.cc:4227-4239.  SC32: anl is the level's sum of |V|_1, and
+// border is set where the decision lay within the sin/cos error bound.
+template <bool SC32>
+__device__ __forceinline__ bool batch_level_end(const BatchArgs& A, int L, double dt, const double ps[6], double maxd,
+                                                double anl, double sum[6], double& lastmag, double& prec,
+                                                double& an_run, double& dm_last, bool& border) {
+#pragma unroll
+  for (int c = 0; c < 6; ++c) sum[c] += ps[c];
+  double E[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) E[c] = sum[c] * dt;
+  if (A.use_pol) pol_project(E, A.pol);
+  const double mag = cmag2(E);
+  const double mag_prev = lastmag;
+  prec = fabs(mag - mag_prev) / mag_prev;
+  if (SC32) {
+    an_run += anl;
+    if (level_borderline(L, dt, A.precision, mag_prev, mag, prec, maxd, an_run, dm_last)) border = true;
+  }
+  lastmag = mag;
+  return (L > 8 && prec < A.precision && maxd < kPi) || (L > 8 && maxd < kPi && mag == mag_prev);
+}
+
+// Adds a finished energy of a unit to its request, and its counts.
+__device__ __forceinline__ void batch_add_point(const BatchArgs& A, const Unit& U, int e, int lev, const double sum[6],
+                                                bool converged) {
+  double f = A.C0 * (U.T / (2.0 * (double) (1L << lev) - 1));
+  double E[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) E[k] = sum[k] * f;
+  if (A.use_pol) pol_project(E, A.pol);
+  atomicAdd(&U.R.out[U.io * U.R.n_e + U.e0 + e], A.C2 * cmag2(E) * A.weight[U.ip]);
+  if (!converged) atomicAdd(A.n_unconverged, 1ULL);
+  atomicAdd(A.evals, (unsigned long long) ((2L << lev) - 1));
+}
+
+// The m replicas of W energies added into replica 0 (lanes 0..W-1): replicas
+// q..q+2s-1 into replica q, for s = 1, 2, 4, ..., in the same order for every
+// group shape.
+__device__ __forceinline__ void add_replicas(double ps[6], double& maxd, double& an, int lane, int W, int m, int q,
+                                             bool act) {
+  for (int st = 1; st < m; st <<= 1) {
+    const int src = lane + st * W < 64 ? lane + st * W : lane;
+    const bool take = act && (q % (2 * st)) == 0 && q + st < m;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      double o = __shfl(ps[c], src);
+      ps[c] = take ? ps[c] + o : ps[c];
+    }
+    double om = __shfl(maxd, src), oa = __shfl(an, src);
+    maxd = take ? fmax(maxd, om) : maxd;
+    an = take ? an + oa : an;
+  }
+}
+
+// A partial sum that another XCD's wave reads in the same launch.
+__device__ __forceinline__ void part_store(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double part_load(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Flags of an energy in the wave's scratch.
 constexpr int kFConverged = 1;
 constexpr int kFBorderline = 2;  // mixed pass: a stop decision lay within the sin/cos error bound
-constexpr int kFHanded = 4;      // handed to lw_batch_deep_kernel
+constexpr int kFHanded = 4;      // handed to lw_batch_level_kernel
 constexpr int kFRecheck = 8;     // recomputed in FP64 inside the unit
 constexpr int kFIdle = 16;       // not part of the FP64 recheck pass
 
@@ -140,9 +204,9 @@ constexpr int kFIdle = 16;       // not part of the FP64 recheck pass
 // groups.  The replicas' partial sums are added in a fixed tree order.  The
 // largest phase step takes the sample before each part from LDS (or from the
 // previous super-block), so it is the same maximum over the same consecutive
-// pairs as a sequential walk.  HANDOVER: energies still active at level Ldeep
-// are handed to lw_batch_deep_kernel.
-template <bool SC32, bool HANDOVER>
+// pairs as a sequential walk.  Energies still active at level Ldeep leave the
+// unit in groups for lw_batch_level_kernel (while there are groups to be had).
+template <bool SC32>
 __device__ __forceinline__ void unit_levels(const BatchArgs& A, const Unit& U, int lane, double* __restrict__ ws,
                                             int* __restrict__ wsi, BatchLds& S, int skip, unsigned long long& n_amp,
                                             unsigned long long& n_ev, unsigned long long& n_slot) {
@@ -156,26 +220,6 @@ __device__ __forceinline__ void unit_levels(const BatchArgs& A, const Unit& U, i
   int* w_flags = wsi + kBatchEB;
   const int n_eb = U.n_eb;
   for (int L = 0; L <= A.Lmax; ++L) {
-    if (HANDOVER && L == A.Ldeep) {
-      // hand the energies still active to the one-wave-per-point kernel
-      for (int t = 0; t < n_eb; t += 64) {
-        int e = t + lane;
-        int ec = e < n_eb ? e : 0;
-        bool a = e < n_eb && (w_flags[ec] & skip) == 0;
-        unsigned long long m = __ballot(a);
-        unsigned long long first = atomicAdd(A.n_deep, lane == 0 ? (unsigned long long) __popcll(m) : 0ULL);
-        unsigned long long j = uniform_u64(first) + (unsigned long long) __popcll(m & ((1ULL << lane) - 1ULL));
-        if (a && j < (unsigned long long) A.deep_cap) {
-          A.deep_code[j] = (unsigned long long) U.item * kBatchEB + (unsigned long long) e;
-#pragma unroll
-          for (int k = 0; k < kBatchWsD; ++k) A.deep_state[k * A.deep_cap + j] = ws[k * kBatchEB + e];
-          A.deep_level[j] = w_level[e];
-          A.deep_flags[j] = w_flags[e];
-          w_flags[e] |= kFHanded;
-        }
-      }
-      __syncthreads();
-    }
     // pack the energies still active
     int n_act = 0;
     for (int t = 0; t < n_eb; t += 64) {
@@ -187,6 +231,38 @@ __device__ __forceinline__ void unit_levels(const BatchArgs& A, const Unit& U, i
     }
     __syncthreads();
     if (n_act == 0) break;
+    if (L == A.Ldeep) {
+      const int ng = (n_act + 63) >> 6;
+      const unsigned long long g0 =
+          uniform_u64(atomicAdd(A.n_group, lane == 0 ? (unsigned long long) ng : 0ULL));
+      if (g0 + (unsigned long long) ng <= (unsigned long long) A.group_cap) {
+        constexpr int kind = SC32 ? 0 : 1;
+        for (int g = 0; g < ng; ++g) {
+          const long id = (long) g0 + g;
+          const int W = n_act - 64 * g < 64 ? n_act - 64 * g : 64;
+          if (lane < W) {
+            const int e = S.list[64 * g + lane];
+            double* st = A.group_state + id * (kBatchGroupD * 64) + lane;
+            A.group_e[64 * id + lane] = (unsigned short) e;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) st[64 * k] = w_sum[k * kBatchEB + e];
+            st[64 * 6] = w_lastmag[e];
+            st[64 * 7] = w_an[e];
+            st[64 * 8] = w_dm[e];
+            w_flags[e] |= kFHanded;
+          }
+          if (lane == 0) {
+            A.group_item[id] = U.item;
+            A.group_n[id] = W;
+            const unsigned long long j = atomicAdd(&A.n_list[kind * kBatchLevels + L], 1ULL);
+            A.group_list[(2 * kind + (L & 1)) * A.group_cap + (long) j] = (int) id;
+          }
+        }
+        atomicAdd(A.n_deep, lane == 0 ? (unsigned long long) n_act : 0ULL);
+        __syncthreads();
+        break;
+      }
+    }
     const double* __restrict__ rows = U.prow + 10 * ((1L << L) - 1);
     const long ns = 1L << L;
     // sample times of level L (the expressions of level_batch_kernel)
@@ -307,48 +383,30 @@ __device__ __forceinline__ void unit_levels(const BatchArgs& A, const Unit& U, i
         }
         // the level is complete for this group
         if (m > 1) {
-          // replicas q..q+2s-1 into replica q, for s = 1, 2, 4, ...: replica 0
-          // ends with the totals, in the same order for every group shape
-          for (int st = 1; st < m; st <<= 1) {
-            const int src = lane + st * W < 64 ? lane + st * W : lane;
-            const bool take = act && (q % (2 * st)) == 0 && q + st < m;
-#pragma unroll
-            for (int c = 0; c < 6; ++c) {
-              double o = __shfl(ps[c], src);
-              ps[c] = take ? ps[c] + o : ps[c];
-            }
-            double om = __shfl(maxd, src);
-            maxd = take ? fmax(maxd, om) : maxd;
-          }
+          double none = 0;
+          add_replicas(ps, maxd, none, lane, W, m, q, act);
         }
         if (q == 0) {
-          double sum[6];
+          double sum[6], lastmag = w_lastmag[e], prec, an_run = 0, dm_last = 0;
+          bool border = false;
 #pragma unroll
-          for (int c = 0; c < 6; ++c) sum[c] = w_sum[c * kBatchEB + e] + ps[c];
-          // convergence test, src/OSCARSSR.cc:4227-4239
-          double E[6];
-#pragma unroll
-          for (int c = 0; c < 6; ++c) E[c] = sum[c] * dt;
-          if (A.use_pol) pol_project(E, A.pol);
-          const double mag = cmag2(E);
-          const double mag_prev = w_lastmag[e];
-          const double prec = fabs(mag - mag_prev) / mag_prev;
-          const bool c = (L > 8 && prec < A.precision && maxd < kPi) || (L > 8 && maxd < kPi && mag == mag_prev);
-          int flags = w_flags[e] | (c ? kFConverged : 0);
+          for (int c = 0; c < 6; ++c) sum[c] = w_sum[c * kBatchEB + e];
           if (SC32) {
-            double an_run = w_an[e] + anl;
-            double dm_last = w_dm[e];
-            if (level_borderline(L, dt, A.precision, mag_prev, mag, prec, maxd, an_run, dm_last))
-              flags |= kFBorderline;
+            an_run = w_an[e];
+            dm_last = w_dm[e];
+          }
+          const bool c =
+              batch_level_end<SC32>(A, L, dt, ps, maxd, anl, sum, lastmag, prec, an_run, dm_last, border);
+          if (SC32) {
             w_an[e] = an_run;
             w_dm[e] = dm_last;
           }
 #pragma unroll
-          for (int c = 0; c < 6; ++c) w_sum[c * kBatchEB + e] = sum[c];
-          w_lastmag[e] = mag;
+          for (int k = 0; k < 6; ++k) w_sum[k * kBatchEB + e] = sum[k];
+          w_lastmag[e] = lastmag;
           w_prec[e] = prec;
           w_level[e] = L;
-          w_flags[e] = flags;
+          w_flags[e] = w_flags[e] | (c ? kFConverged : 0) | (border ? kFBorderline : 0);
         }
       }
       tprev = S.tau[blk(cnt - 1)];
@@ -389,9 +447,10 @@ __device__ __forceinline__ void batch_unit(const BatchArgs& A, long item, int la
   }
   __syncthreads();  // the state written above is read by other lanes
   unsigned long long n_amp = 0, n_ev = 0, n_slot = 0;  // wave-uniform work counts of this unit
-  unit_levels<MIXED, true>(A, U, lane, ws, wsi, S, kFConverged | kFHanded, n_amp, n_ev, n_slot);
+  unit_levels<MIXED>(A, U, lane, ws, wsi, S, kFConverged | kFBorderline | kFHanded, n_amp, n_ev, n_slot);
   if (MIXED) {
-    // FP64 recheck: reset the borderline energies, park the others
+    // FP64 recheck: reset the borderline energies (the first pass left them
+    // where they were met), park the others
     int n_re = 0;
     for (int t = 0; t < n_eb; t += 64) {
       const int e = t + lane;
@@ -406,13 +465,15 @@ __device__ __forceinline__ void batch_unit(const BatchArgs& A, long item, int la
         w_prec[e] = -1;
         w_level[e] = -1;
         w_flags[e] = kFRecheck;
+        w_an[e] = 0;
+        w_dm[e] = 0;
       } else if (e < n_eb) {
         w_flags[e] = flags | kFIdle;
       }
     }
     __syncthreads();
     if (n_re > 0) {
-      unit_levels<false, false>(A, U, lane, ws, wsi, S, kFConverged | kFHanded | kFIdle, n_amp, n_ev, n_slot);
+      unit_levels<false>(A, U, lane, ws, wsi, S, kFConverged | kFHanded | kFIdle, n_amp, n_ev, n_slot);
     }
     atomicAdd(A.n_recheck, lane == 0 ? (unsigned long long) n_re : 0ULL);
   }
@@ -464,140 +525,189 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) lw
     batch_unit<MIXED>(A, item, lane, ws, wsi, S);
   }
 }
-// Waves per point in the per-point kernels: each level's samples are split
-// into kPointWaves contiguous slices, one per wave, combined in LDS.
-constexpr int kPointWaves = 8;
 
-// One point (code = item * kBatchEB + energy-in-block) summed by a workgroup
-// of kPointWaves waves from level L0 with the given state; then its flux,
-// counts and (MIXED, borderline) its fix-up entry.  Levels, convergence test
-// and weighting are the batch kernel's.  Every thread returns with the same
-// decisions; thread 0 does the atomics.
-template <bool MIXED>
-__device__ __forceinline__ void batch_point(const BatchArgs& A, unsigned long long code, int L0, double sum[6],
-                                            double lastmag, double an_run, double dm_last, int flags, int lev,
-                                            double (*sh)[kPointWaves], unsigned long long* sh_slot) {
+// ---------------------------------------------------------------- deep levels
+// One level of the groups handed over.  A unit whose energies converge slowly
+// has level after level of 2^L samples: left to its one wave, a single energy
+// at level 25 takes 0.2 s, most of a batch of 64 particles (182 ms of which the
+// chip's work was 26).  Here the level's samples are cut into slices, enough to
+// occupy every wave (one each when there are many groups), a wave computes a
+// slice's amplitudes super-block by super-block as unit_levels does and walks
+// them with the group's energies, and the wave that completes a group adds the
+// slices' partial sums in order, takes the decisions and lists the group, its
+// energies packed again, for the next level.
+// Measured, 64 particles (13664 units): 182 ms and 324 ms (two seeds) with every
+// energy left to its unit, 40 ms and 38 ms handed over at level 12; 2048
+// particles (1.76 M units) 5.10 -> 4.85 s at level 17.
+constexpr int kLevelWaves = 4;  // independent waves per workgroup
+template <bool SC32>
+__global__ void __launch_bounds__(64 * kLevelWaves) __attribute__((amdgpu_waves_per_eu(4)))
+lw_batch_level_kernel(BatchArgs A, int L) {
+  __shared__ BatchLds lds[kLevelWaves];
+  constexpr int kind = SC32 ? 0 : 1;
+  BatchLds& S = lds[threadIdx.x >> 6];
   const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
-  long item = (long) (code / kBatchEB);
-  long e_in = (long) (code - (unsigned long long) item * kBatchEB);
-  int lo = 0, hi = A.np;
-  while (hi - lo > 1) {
-    int mid = (lo + hi) >> 1;
-    if (A.item_prefix[mid] <= item) lo = mid; else hi = mid;
-  }
-  const int ip = lo;
-  const long local = item - A.item_prefix[ip];
-  const ReqDev R = A.req[A.req_of[ip]];
-  const long io = local / R.n_blocks_e;
-  const long ie = (local - io * R.n_blocks_e) * kBatchEB + e_in;
-  const V3 obs = v3(R.obs[3 * io], R.obs[3 * io + 1], R.obs[3 * io + 2]);
-  const double ts = A.tspan[2 * ip], te = A.tspan[2 * ip + 1];
-  const double T = te - ts;
-  const double* prow = A.rows + 10 * (long) ip * A.stride;
-  const TrajDesc D = A.desc[ip];
-  const double negw = -R.omega[ie];
-  bool c = false;
-  for (int L = L0; L <= A.Lmax && !c; ++L) {
-    const long ns = 1L << L;
-    const double p2L = (double) (1L << L);
-    const double spacing = L > A.stop_mem ? (te - ts) / (p2L - 1) : (te - ts) / p2L;
-    const double tfirst = ts + (te - ts) / (2.0 * p2L);
-    const double* __restrict__ rows = prow + 10 * ((1L << L) - 1);
-    const long i0 = ns * w / kPointWaves, i1 = ns * (w + 1) / kPointWaves;
-    double t6[6], md, al;
-    if (L <= A.Lb) {
-      slice_level_sum_rows<MIXED>(rows, i0, i1, obs, negw, lane, t6, md, al);
-    } else {
-      slice_level_sum<MIXED>(
-          i0, i1, negw, lane, [&](long i) { return interpolated_amplitude(A, D, obs, tfirst + spacing * (double) i); },
-          t6, md, al);
-    }
-    if (lane == 0) {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) sh[k][w] = t6[k];
-      sh[6][w] = md;
-      sh[7][w] = al;
-    }
-    __syncthreads();
-    double tot[6] = {0, 0, 0, 0, 0, 0};
+  const long n = (long) A.n_list[kind * kBatchLevels + L];
+  if (n == 0) return;
+  const long ns = 1L << L;
+  // slices of at least 512 samples, at most 256 to a group, in all at most what
+  // there is room for (16 for each of the 4096 waves; their cost depends on the
+  // group's energies, so they are taken from a counter)
+  long nsl = kBatchParts / n;
+  nsl = nsl < 1 ? 1 : (nsl > 256 ? 256 : nsl);
+  nsl = nsl > ns / 512 ? ns / 512 : nsl;
+  const int* __restrict__ ids = A.group_list + (2 * kind + (L & 1)) * A.group_cap;
+  while (true) {
+    const long job = (long) uniform_u64(atomicAdd(&A.n_job[kind * kBatchLevels + L], lane == 0 ? 1ULL : 0ULL));
+    if (job >= n * nsl) break;
+    const long gi = job / nsl, sl = job - gi * nsl;
+    const long id = ids[gi];
+    const Unit U = unit_of(A, A.group_item[id]);
+    const int W = A.group_n[id];
+    const int m = 64 / W;      // replicas of each energy
+    const int q = lane / W;    // this lane's (q >= m: idle)
+    const int j = lane - q * W;
+    const bool act = q < m;
+    const int slot = act ? j : 0;
+    const int e = A.group_e[64 * id + slot];
+    const double negw = -U.R.omega[U.e0 + e];
+    const double* __restrict__ rows = U.prow + 10 * (ns - 1);
+    const double p2L = (double) ns;
+    const double spacing = L > A.stop_mem ? (U.te - U.ts) / (p2L - 1) : (U.te - U.ts) / p2L;
+    const double tfirst = U.ts + (U.te - U.ts) / (2.0 * p2L);
+    const bool stored = L <= A.Lb;
+    auto amp_at = [&](long i) {
+      return stored ? amplitude(U.obs, rows + 10 * i)
+                    : interpolated_amplitude(A, U.D, U.obs, tfirst + spacing * (double) i);
+    };
+    const long i0 = ns * sl / nsl, i1 = ns * (sl + 1) / nsl;
+    double tprev = i0 > 0 ? amp_at(i0 - 1).tau : 0.0;
+    double ps[6] = {0, 0, 0, 0, 0, 0};
     double maxd = 0, anl = 0;
-    for (int v = 0; v < kPointWaves; ++v) {  // in slice order: every thread forms the same totals
-#pragma unroll
-      for (int k = 0; k < 6; ++k) tot[k] += sh[k][v];
-      maxd = fmax(maxd, sh[6][v]);
-      anl += sh[7][v];
+    for (long base = i0; base < i1; base += kSuper) {
+      const int cnt = (int) (i1 - base < kSuper ? i1 - base : kSuper);
+#pragma unroll 1
+      for (int h = 0; h < kSuper; h += 64) {
+        if (h + lane < cnt) {
+          const Amp a = amp_at(base + h + lane);
+          S.tau[blk(h + lane)] = a.tau;
+          S.vx[blk(h + lane)] = a.V.x;
+          S.vy[blk(h + lane)] = a.V.y;
+          S.vz[blk(h + lane)] = a.V.z;
+          if (SC32) anl += fabs(a.V.x) + fabs(a.V.y) + fabs(a.V.z);
+        }
+      }
+      wave_sync();
+      const int k0 = act ? (q * cnt) / m : 0;
+      const int k1 = act ? ((q + 1) * cnt) / m : 0;
+      double lastphase = negw * (k0 > 0 ? S.tau[blk(k0 - 1)] : (base > 0 ? tprev : S.tau[0]));
+#pragma unroll 4
+      for (int k = k0; k < k1; ++k) {
+        const int b = blk(k);
+        double phi = negw * S.tau[b];
+        maxd = fmax(maxd, fabs(phi - lastphase));
+        lastphase = phi;
+        double sn, cs;
+        sincos_mode(SC32, phi, sn, cs);
+        double vx = S.vx[b], vy = S.vy[b], vz = S.vz[b];
+        ps[0] = __builtin_fma(vx, cs, ps[0]); ps[1] = __builtin_fma(vx, sn, ps[1]);
+        ps[2] = __builtin_fma(vy, cs, ps[2]); ps[3] = __builtin_fma(vy, sn, ps[3]);
+        ps[4] = __builtin_fma(vz, cs, ps[4]); ps[5] = __builtin_fma(vz, sn, ps[5]);
+      }
+      tprev = S.tau[blk(cnt - 1)];
+      wave_sync();  // the next super-block overwrites the amplitudes
     }
-    __syncthreads();  // sh is rewritten at the next level
-#pragma unroll
-    for (int k = 0; k < 6; ++k) sum[k] += tot[k];
-    lev = L;
-    // convergence test, src/OSCARSSR.cc:4227-4239
-    double E[6];
-    double dt = T / (2.0 * (double) (1L << L) - 1);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) E[k] = sum[k] * dt;
-    if (A.use_pol) pol_project(E, A.pol);
-    double mag = cmag2(E);
-    double prec = fabs(mag - lastmag) / lastmag;
-    c = (L > 8 && prec < A.precision && maxd < kPi) || (L > 8 && maxd < kPi && mag == lastmag);
-    if (MIXED) {
-      an_run += anl;
-      if (level_borderline(L, dt, A.precision, lastmag, mag, prec, maxd, an_run, dm_last)) flags |= 2;
+    double none = 0;
+    add_replicas(ps, maxd, none, lane, W, m, q, act);
+    if (SC32) {
+      for (int off = 32; off > 0; off >>= 1) anl += __shfl_xor(anl, off);
     }
-    lastmag = mag;
-  }
-  c = c || (flags & 1);
-  bool fixed = false;
-  if (MIXED && (flags & 2)) {  // the same for every thread
-    if (threadIdx.x == 0) *sh_slot = atomicAdd(A.n_fix, 1ULL);
-    __syncthreads();
-    unsigned long long j = *sh_slot;
-    __syncthreads();
-    if (j < (unsigned long long) A.fix_cap) {
-      if (threadIdx.x == 0) A.fix_list[j] = code;
-      fixed = true;
+    const bool mine = lane < W;  // replica 0
+    if (nsl > 1) {
+      // partial sums through the device's coherence point (no cache write-back):
+      // stores that bypass the caches, waited for before the arrival is counted
+      double* pp = A.part + (gi * nsl + sl) * (8 * 64) + lane;
+      if (mine) {
+#pragma unroll
+        for (int c = 0; c < 6; ++c) part_store(pp + 64 * c, ps[c]);
+        part_store(pp + 64 * 6, maxd);
+        part_store(pp + 64 * 7, anl);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const unsigned before = (unsigned) __builtin_amdgcn_readfirstlane(
+          (int) atomicAdd(&A.group_arrived[id], lane == 0 ? 1u : 0u));
+      if (before + 1 < (unsigned) nsl) continue;
+      if (lane == 0) A.group_arrived[id] = 0;
+      // replica q adds slices q, q + m, ...
+#pragma unroll
+      for (int c = 0; c < 6; ++c) ps[c] = 0;
+      maxd = anl = 0;
+      const double* pg = A.part + gi * nsl * (8 * 64) + slot;
+#pragma unroll 4
+      for (long s = act ? q : nsl; s < nsl; s += m) {
+        const double* p = pg + s * (8 * 64);
+#pragma unroll
+        for (int c = 0; c < 6; ++c) ps[c] += part_load(p + 64 * c);
+        maxd = fmax(maxd, part_load(p + 64 * 6));
+        anl += part_load(p + 64 * 7);
+      }
+      add_replicas(ps, maxd, anl, lane, W, m, q, act);
     }
-  }
-  if (threadIdx.x == 0 && !fixed) {
-    double f = A.C0 * (T / (2.0 * (double) (1L << lev) - 1));
-    double E[6];
+    // decisions, one energy per lane; the others' lanes hold none
+    double* gs = A.group_state + id * (kBatchGroupD * 64);
+    double sum[6], lastmag = 0, prec, an_run = 0, dm_last = 0;
+    bool border = false, go_on = false;
+    if (mine) {
 #pragma unroll
-    for (int k = 0; k < 6; ++k) E[k] = sum[k] * f;
-    if (A.use_pol) pol_project(E, A.pol);
-    atomicAdd(&R.out[io * R.n_e + ie], A.C2 * cmag2(E) * A.weight[ip]);
-    if (!c) atomicAdd(A.n_unconverged, 1ULL);
-    atomicAdd(A.evals, (unsigned long long) ((2L << lev) - 1));
-  }
-}
-
-// Points the batch kernel handed over at level Ldeep (slowly converging, with
-// many samples per level): one workgroup per point from its stored state.  A
-// grid-stride loop over the handed-over count (read from device memory, so the
-// launch can sit in a captured graph).
-template <bool MIXED>
-__global__ void __launch_bounds__(64 * kPointWaves) lw_batch_deep_kernel(BatchArgs A) {
-  __shared__ double sh[8][kPointWaves];
-  __shared__ unsigned long long sh_slot;
-  long n = (long) *A.n_deep;
-  if (n > A.deep_cap) n = A.deep_cap;
-  for (long k = blockIdx.x; k < n; k += gridDim.x) {
-    unsigned long long code = A.deep_code[k];
-    double st[kBatchWsD];
+      for (int k = 0; k < 6; ++k) sum[k] = gs[64 * k + lane];
+      lastmag = gs[64 * 6 + lane];
+      if (SC32) {
+        an_run = gs[64 * 7 + lane];
+        dm_last = gs[64 * 8 + lane];
+      }
+      // (a decision that lay within the error bound at an earlier level went to
+      // the recomputation list there)
+      const bool c = batch_level_end<SC32>(A, L, U.T / (2.0 * (double) ns - 1), ps, maxd, anl, sum, lastmag, prec,
+                                           an_run, dm_last, border);
+      bool listed = false;
+      if (SC32 && border) {
+        const unsigned long long k = atomicAdd(A.n_fix, 1ULL);
+        if (k < (unsigned long long) A.fix_cap) {
+          A.fix_list[k] = (unsigned long long) U.item * kBatchEB + (unsigned long long) e;
+          listed = true;
+        }
+      }
+      go_on = !listed && !c && L < A.Lmax;
+      if (!listed && !go_on) batch_add_point(A, U, e, L, sum, c);
+    }
+    const unsigned long long live = __ballot(go_on);
+    if (live) {
+      const int at = __popcll(live & ((1ULL << lane) - 1ULL));
+      if (go_on) {
+        A.group_e[64 * id + at] = (unsigned short) e;
 #pragma unroll
-    for (int q = 0; q < kBatchWsD; ++q) st[q] = A.deep_state[q * A.deep_cap + k];
-    int lev = A.deep_level[k];
-    int flags = A.deep_flags[k];
-    batch_point<MIXED>(A, code, lev + 1, st, st[6], st[8], st[9], flags, lev, sh, &sh_slot);
+        for (int k = 0; k < 6; ++k) gs[64 * k + at] = sum[k];
+        gs[64 * 6 + at] = lastmag;
+        if (SC32) {
+          gs[64 * 7 + at] = an_run;
+          gs[64 * 8 + at] = dm_last;
+        }
+      }
+      if (lane == 0) {
+        A.group_n[id] = __popcll(live);
+        const unsigned long long k = atomicAdd(&A.n_list[kind * kBatchLevels + L + 1], 1ULL);
+        A.group_list[(2 * kind + ((L + 1) & 1)) * A.group_cap + (long) k] = (int) id;
+      }
+    }
   }
 }
 
 // FP64 recomputation of the points the mixed kernels listed, from level 0, so
 // their levels and values are the FP64 path's.  One wave per point, its lanes
-// splitting each level's samples (a unit rarely holds more than a few such
-// points, so sharing the amplitude across them would leave most lanes idle):
-// no workgroup barrier, and a point's low levels occupy one wave, not eight.
-// Four waves per workgroup; the waves stride over the list independently.
+// splitting each level's samples, up to level Ldeep - 1; a point active there
+// becomes a group of its own for lw_batch_level_kernel<false> (or, with no
+// group left, goes on here).  Four waves per workgroup; the waves stride over
+// the list independently.
 __global__ void __launch_bounds__(256) lw_batch_fix_kernel(BatchArgs A) {
   const int lane = threadIdx.x & 63;
   const long wave = (long) blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -606,67 +716,52 @@ __global__ void __launch_bounds__(256) lw_batch_fix_kernel(BatchArgs A) {
   if (n > A.fix_cap) n = A.fix_cap;
   for (long k = wave; k < n; k += n_waves) {
     const unsigned long long code = A.fix_list[k];
-    const long item = (long) (code / kBatchEB);
-    const long e_in = (long) (code - (unsigned long long) item * kBatchEB);
-    int lo = 0, hi = A.np;
-    while (hi - lo > 1) {
-      int mid = (lo + hi) >> 1;
-      if (A.item_prefix[mid] <= item) lo = mid; else hi = mid;
-    }
-    const int ip = lo;
-    const long local = item - A.item_prefix[ip];
-    const ReqDev R = A.req[A.req_of[ip]];
-    const long io = local / R.n_blocks_e;
-    const long ie = (local - io * R.n_blocks_e) * kBatchEB + e_in;
-    const V3 obs = v3(R.obs[3 * io], R.obs[3 * io + 1], R.obs[3 * io + 2]);
-    const double ts = A.tspan[2 * ip], te = A.tspan[2 * ip + 1];
-    const double T = te - ts;
-    const double* prow = A.rows + 10 * (long) ip * A.stride;
-    const TrajDesc D = A.desc[ip];
-    const double negw = -R.omega[ie];
+    const Unit U = unit_of(A, (long) (code / kBatchEB));
+    const int e = (int) (code - (unsigned long long) U.item * kBatchEB);
+    const double negw = -U.R.omega[U.e0 + e];
     double sum[6] = {0, 0, 0, 0, 0, 0};
-    double lastmag = -1;
-    int lev = 0;
-    bool c = false;
+    double lastmag = -1, prec, an_run = 0, dm_last = 0;
+    int lev = -1;
+    bool c = false, border = false, handed = false;
     for (int L = 0; L <= A.Lmax && !c; ++L) {
+      if (L == A.Ldeep) {
+        const unsigned long long id =
+            uniform_u64(atomicAdd(A.n_group, lane == 0 ? 1ULL : 0ULL));
+        if (id < (unsigned long long) A.group_cap) {
+          if (lane == 0) {
+            double* st = A.group_state + (long) id * (kBatchGroupD * 64);
+#pragma unroll
+            for (int q = 0; q < 6; ++q) st[64 * q] = sum[q];
+            st[64 * 6] = lastmag;
+            A.group_e[64 * id] = (unsigned short) e;
+            A.group_item[id] = U.item;
+            A.group_n[id] = 1;
+            const unsigned long long j = atomicAdd(&A.n_list[kBatchLevels + L], 1ULL);
+            A.group_list[(2 + (L & 1)) * A.group_cap + (long) j] = (int) id;
+          }
+          handed = true;
+          break;
+        }
+      }
       const long ns = 1L << L;
+      const double p2L = (double) ns;
       double tot[6], maxd, an;
       if (L <= A.Lb) {
-        slice_level_sum_rows<false>(prow + 10 * ((1L << L) - 1), 0, ns, obs, negw, lane, tot, maxd, an);
+        slice_level_sum_rows<false>(U.prow + 10 * (ns - 1), 0, ns, U.obs, negw, lane, tot, maxd, an);
       } else {
-        const double p2L = (double) (1L << L);
-        const double spacing = L > A.stop_mem ? (te - ts) / (p2L - 1) : (te - ts) / p2L;
-        const double tfirst = ts + (te - ts) / (2.0 * p2L);
+        const double spacing = L > A.stop_mem ? (U.te - U.ts) / (p2L - 1) : (U.te - U.ts) / p2L;
+        const double tfirst = U.ts + (U.te - U.ts) / (2.0 * p2L);
         slice_level_sum<false>(
             0, ns, negw, lane,
-            [&](long i) { return interpolated_amplitude(A, D, obs, tfirst + spacing * (double) i); }, tot, maxd,
+            [&](long i) { return interpolated_amplitude(A, U.D, U.obs, tfirst + spacing * (double) i); }, tot, maxd,
             an);
       }
-#pragma unroll
-      for (int q = 0; q < 6; ++q) sum[q] += tot[q];
       lev = L;
-      // convergence test, src/OSCARSSR.cc:4227-4239 (the batch kernel's)
-      double E[6];
-      const double dt = T / (2.0 * (double) (1L << L) - 1);
-#pragma unroll
-      for (int q = 0; q < 6; ++q) E[q] = sum[q] * dt;
-      if (A.use_pol) pol_project(E, A.pol);
-      const double mag = cmag2(E);
-      const double prec = fabs(mag - lastmag) / lastmag;
-      c = (L > 8 && prec < A.precision && maxd < kPi) || (L > 8 && maxd < kPi && mag == lastmag);
-      lastmag = mag;
+      c = batch_level_end<false>(A, L, U.T / (2.0 * p2L - 1), tot, maxd, 0.0, sum, lastmag, prec, an_run, dm_last,
+                                 border);
     }
     // every lane holds the same totals (butterfly sums): lane 0 adds the point
-    const double f = A.C0 * (T / (2.0 * (double) (1L << lev) - 1));
-    double E[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) E[q] = sum[q] * f;
-    if (A.use_pol) pol_project(E, A.pol);
-    if (lane == 0) {
-      atomicAdd(&R.out[io * R.n_e + ie], A.C2 * cmag2(E) * A.weight[ip]);
-      if (!c) atomicAdd(A.n_unconverged, 1ULL);
-      atomicAdd(A.evals, (unsigned long long) ((2L << lev) - 1));
-    }
+    if (lane == 0 && !handed) batch_add_point(A, U, e, lev, sum, c);
   }
 }
 
@@ -697,23 +792,27 @@ extern "C" hipError_t om_launch_batch_clear(double* out, long n, unsigned long l
   return hipGetLastError();
 }
 
-// The batch: the persistent kernel (stage bit 0), the per-point kernel for the
-// points it handed over (bit 1) and, mixed, the FP64 recomputation of
-// borderline points (bit 2); stages = 7 launches all three in order.
+// The batch: the persistent kernel (stage bit 0), the levels of the energies it
+// handed over (bit 1) and, mixed, the FP64 recomputation of borderline points
+// (bit 2); stages = 7 launches all three in order.  A launch per level: one with
+// nothing listed returns at once (about 5 us in a graph).
 extern "C" hipError_t om_launch_lw_batch_stages(const om::BatchArgs* A, int mixed, int n_groups, int stages,
                                                 hipStream_t s) {
-  int pg = n_groups / om::kPointWaves > 0 ? n_groups / om::kPointWaves : 1;  // same wave count
-  dim3 pb(64 * om::kPointWaves);
-  if (mixed) {
-    if (stages & 1) hipLaunchKernelGGL(om::lw_batch_kernel<true>, dim3(n_groups), dim3(64), 0, s, *A);
-    if (stages & 2) hipLaunchKernelGGL(om::lw_batch_deep_kernel<true>, dim3(pg), pb, 0, s, *A);
-    if (stages & 4) {
-      int fb = n_groups / 4 > 0 ? n_groups / 4 : 1;  // four single-wave points per workgroup
-      hipLaunchKernelGGL(om::lw_batch_fix_kernel, dim3(fb), dim3(256), 0, s, *A);
+  if (stages & 1) {
+    if (mixed) hipLaunchKernelGGL(om::lw_batch_kernel<true>, dim3(n_groups), dim3(64), 0, s, *A);
+    else hipLaunchKernelGGL(om::lw_batch_kernel<false>, dim3(n_groups), dim3(64), 0, s, *A);
+  }
+  const unsigned waves = 4096;  // 16 per CU
+  const dim3 grid(waves / om::kLevelWaves), block(64 * om::kLevelWaves);
+  if (stages & 2)
+    for (int L = A->Ldeep; L <= A->Lmax; ++L) {
+      if (mixed) hipLaunchKernelGGL(om::lw_batch_level_kernel<true>, grid, block, 0, s, *A, L);
+      else hipLaunchKernelGGL(om::lw_batch_level_kernel<false>, grid, block, 0, s, *A, L);
     }
-  } else {
-    if (stages & 1) hipLaunchKernelGGL(om::lw_batch_kernel<false>, dim3(n_groups), dim3(64), 0, s, *A);
-    if (stages & 2) hipLaunchKernelGGL(om::lw_batch_deep_kernel<false>, dim3(pg), pb, 0, s, *A);
+  if (mixed && (stages & 4) && A->Ldeep <= A->Lmax) {
+    hipLaunchKernelGGL(om::lw_batch_fix_kernel, dim3(waves / 4), dim3(256), 0, s, *A);
+    for (int L = A->Ldeep; L <= A->Lmax; ++L)
+      hipLaunchKernelGGL(om::lw_batch_level_kernel<false>, grid, block, 0, s, *A, L);
   }
   return hipGetLastError();
 }

@@ -169,6 +169,11 @@ constexpr int kBatchWsD = 10;
 constexpr int kBatchWsI = 2;
 // plus, per wave, 7 partial sums x 64 lanes for each of the kBatchEB / 64
 // energy groups of a level (kept between super-blocks of samples)
+// Groups of energies handed over: sum[6], lastmag, |V|_1 sum, error bound of
+// lastmag; at most kBatchParts slices of partial sums at a time.
+constexpr int kBatchGroupD = 9;
+constexpr int kBatchLevels = kMaxLevel + 2;
+constexpr long kBatchParts = 65536;
 constexpr int kBatchWsTotal = kBatchWsD * kBatchEB + (kBatchEB / 64) * 7 * 64;
 
 struct ReqDev {
@@ -208,21 +213,28 @@ struct BatchArgs {
   // (their stop decision lay within the reduced-accuracy sin/cos error bound)
   unsigned long long* n_recheck;
   // mixed path: handed-over points whose stop decision lay within the
-  // reduced-accuracy sin/cos error bound, as item * kBatchEB + energy-in-block, recomputed in FP64 by
-  // lw_batch_fix_kernel
+  // reduced-accuracy sin/cos error bound, as item * kBatchEB + energy-in-block,
+  // recomputed in FP64 by lw_batch_fix_kernel
   unsigned long long* fix_list;
   long fix_cap;
   unsigned long long* n_fix;  // points flagged (those beyond fix_cap keep the mixed result)
-  // points still active at level Ldeep are handed to lw_batch_deep_kernel (one
-  // wave per point) with their state: code as in fix_list, kBatchWsD doubles
-  // (field-major, deep_cap per field), level and flags
+  // Energies still active at level Ldeep leave their unit in groups of up to 64
+  // and go on one level per launch, a level's samples split over many waves
+  // (lw_batch_level_kernel).  Two kinds: 0 mixed sums, 1 FP64 sums (the FP64
+  // batch, and the mixed path's recomputations).
   int Ldeep;
-  unsigned long long* deep_code;
-  double* deep_state;
-  int* deep_level;
-  int* deep_flags;
-  long deep_cap;
-  unsigned long long* n_deep;  // points handed over (those beyond deep_cap stay with their unit)
+  unsigned long long* n_deep;    // energies handed over
+  unsigned long long* n_group;   // groups taken (those beyond group_cap stay with their unit)
+  unsigned long long* n_list;    // per kind and level: groups to do (2 x kBatchLevels)
+  unsigned long long* n_job;     // per kind and level: jobs taken (2 x kBatchLevels)
+  long group_cap;
+  int* group_list;               // per kind and parity of the level: group indices (4 x group_cap)
+  long* group_item;              // work unit
+  int* group_n;                  // energies
+  unsigned short* group_e;       // 64 per group: energy in the unit's block
+  double* group_state;           // kBatchGroupD x 64 per group, field-major
+  unsigned* group_arrived;       // slices summed so far (zero between launches)
+  double* part;                  // per (group, slice) of a level: 8 x 64 partial sums
   // work done inside lw_batch_kernel itself (for its roofline): amplitude
   // evaluations, one per (unit, energy group, sample), integrand evaluations,
   // one per (active energy, sample), and lane slots of the integrand loop

@@ -124,3 +124,38 @@ def test_many_trajectories_in_segments():
         scale = np.maximum(np.max(np.abs(p1), axis=0), 1e-300)
         assert np.array_equal(t, t1) and np.max(np.abs(p[:, 2] - p1[:, 2])) <= 2.0 ** -52
         assert np.max(np.abs(p - p1) / scale) < 1e-12
+
+
+@gpu
+@pytest.mark.parametrize("mode", ["tiled", "mixed"])
+def test_batch_levels_handed_over(mode):
+    """Energies handed over at level 9 in groups of 1, 63, 64, 64 + 1 and
+    64 + 64 + 2, some to levels beyond the stored rows, against the same batch
+    with no hand-over: equal evaluation counts (identical levels), and values to
+    1e-11 (the order of up to 2^16 terms' sums: 2^16 u; 1e-6 for the mixed sums,
+    whose sines and cosines carry 4.8e-9), over several replays of the graph."""
+    from oscars_amd import multiparticle as M
+    from oscars_amd.sr import sr
+    from tests.common import UNDULATOR
+    s = sr()
+    s.add_bfield_undulator(**UNDULATOR)
+    rng = np.random.default_rng(2)
+    from oscars_amd import beam as B
+    parts = B.sample_particles(M.config_beam(), 5, rng=rng)
+    windows = M.uneven_windows(parts, rng, npts_range=(2001, 6001))
+    grid = np.array([[x, 2e-4, 30.0] for x in (-3e-3, 0.0, 1e-3)])
+    reqs = [(grid, np.linspace(150.0, 900.0, n)) for n in (1, 63, 64, 65, 130)]
+    out = {}
+    for deep in (27, 9):
+        b = M.BatchedFlux(s._device(), s._fields, parts, windows, reqs, np.arange(5), np.ones(5), mode=mode,
+                          precision=2e-3, level_cap=11, deep_level=deep)
+        runs = [b.run(recompute_trajectories=k > 0) for k in range(3)]
+        for o, st in runs[1:]:
+            assert st["evals"] == runs[0][1]["evals"] and st["n_unconverged"] == 0
+            assert all(rel_err(a, c) < 1e-12 for a, c in zip(o, runs[0][0]))
+        out[deep] = runs[0]
+        _, cnt, _ = s._device().batch_profile(False)
+        assert (cnt["handed_over"] > 0) == (deep == 9)
+    assert out[27][1]["evals"] == out[9][1]["evals"] > 323 * 3 * (2 ** 11 - 1)
+    for a, c in zip(out[9][0], out[27][0]):
+        assert rel_err(a, c, 1e-6) < (1e-11 if mode == "tiled" else 1e-6)
