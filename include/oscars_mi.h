@@ -255,7 +255,8 @@ int om_power_density_dev(om_context* ctx, int particle, const double* obs_xyz, l
  * ends), so no hipMalloc, hipFree or pinned host allocation happens.  A
  * request needing more scratch than 64 MiB (about 56 bytes per output point,
  * 76 in the mixed modes, plus 160 bytes x 2^L rows for the deepest level L
- * summed) fails with an error.  conv->accumulate must be 0.  The trajectory is
+ * summed, and 17 MB for tiled requests of at most 1024 groups of an observation
+ * point and 64 energies) fails with an error.  conv->accumulate must be 0.  The trajectory is
  * the context's current one (om_trajectories before, which allocates).  Every
  * call on a GPU shares that GPU's scratch: calls that overlap on one GPU, from
  * two contexts or threads, race. */

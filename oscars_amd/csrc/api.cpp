@@ -50,7 +50,9 @@ hipError_t om_launch_spline(const om::TrajDesc* desc, int np, const double* t, c
                             double* u, double* sig, double* sm1, double* pv, double* ppv, double* u2, long total,
                             hipStream_t s);
 hipError_t om_launch_level(const om::LevelJob* J, hipStream_t s);
-hipError_t om_launch_beta_diff(const double* rows, long npts, double* out, hipStream_t s);
+hipError_t om_launch_levels(const om::LevelsJob* J, hipStream_t s);
+hipError_t om_launch_beta_diff(const double* rows, int L0, int n, double* out, hipStream_t s);
+hipError_t om_launch_lw_slice(const om::LwArgs* A, const om::SliceArgs* X, int mixed, hipStream_t s);
 hipError_t om_launch_lw_point(const om::LwArgs* A, int mixed, int split, hipStream_t s);
 hipError_t om_launch_lw_tile(const om::LwArgs* A, long n_obs, int mixed, int split, hipStream_t s);
 hipError_t om_launch_lw_tile_list(const om::LwArgs* A, long ntiles, int mixed, int split, hipStream_t s);
@@ -228,12 +230,17 @@ struct LaunchTimer {
   }
 };
 
+// Levels 0..kBlockLevel of a trajectory are one block of rows, built in one
+// launch (1.3 MB); deeper ones have buffers of their own.
+constexpr int kBlockLevel = 13;
+
 struct LevelCache {
   double* rows[om::kMaxLevel + 1] = {};  // device buffers, kept across trajectory sets
   bool built[om::kMaxLevel + 1] = {};    // rows hold samples of the current trajectory
   int extended[om::kMaxLevel + 1] = {};
-  double beta_diff[om::kMaxLevel + 1] = {};
   bool have_bd[om::kMaxLevel + 1] = {};
+  double* bd = nullptr;  // per level: largest beta step (device, after the block's rows)
+  int block = -1;        // last level of the block at rows[0], -1: none yet
 };
 
 }  // namespace
@@ -280,7 +287,8 @@ struct om_context {
   DevBuf<int> d_level, d_conv, d_count, d_outlevel, d_list, d_border;
   DevBuf<unsigned char> d_outconv;
   DevBuf<unsigned long long> d_stats;
-  DevBuf<double> d_bd;
+  DevBuf<double> d_part;       // sliced sums: partial sums and arrivals
+  DevBuf<unsigned> d_arrived;
   DevBuf<double> d_normals, d_tp, d_tp_partial, d_et, d_stl, d_fp, d_fp_out;
   DevBuf<double> d_bvh_box;
   DevBuf<int> d_bvh_meta, d_bvh_order;
@@ -358,10 +366,7 @@ struct om_context {
   void free_levels() {
     for (auto& lc : levels)
       for (int L = 0; L <= om::kMaxLevel; ++L)
-        if (lc.rows[L]) {
-          (void) hipFree(lc.rows[L]);
-          lc.rows[L] = nullptr;
-        }
+        if (lc.rows[L] && (L == 0 || L > lc.block)) (void) hipFree(lc.rows[L]);
     levels.clear();
   }
 
@@ -377,8 +382,8 @@ struct om_context {
     d_sig.release(); d_sm1.release(); d_pv.release(); d_ppv.release(); d_u2.release();
     d_obs.release(); d_omega.release(); d_sum.release(); d_err.release(); d_lastmag.release();
     d_prec.release(); d_out.release(); d_outcomp.release(); d_oute.release(); d_level.release();
-    d_conv.release(); d_count.release(); d_outlevel.release(); d_outconv.release(); d_bd.release();
-    d_list.release(); d_border.release();
+    d_conv.release(); d_count.release(); d_outlevel.release(); d_outconv.release();
+    d_list.release(); d_border.release(); d_part.release(); d_arrived.release(); d_stats.release();
     d_normals.release(); d_tp.release(); d_tp_partial.release(); d_et.release(); d_stl.release(); d_fp.release(); d_fp_out.release(); d_fp_fields.release();
     d_bvh_box.release(); d_bvh_meta.release(); d_bvh_order.release();
     if (ev0) (void) hipEventDestroy(ev0);
@@ -552,13 +557,46 @@ void level_stops(const om_conv& c, int& stop_mem, int& stop_ext) {
 double dt_inclusive(double ts, double te, int L) { return (te - ts) / (std::pow(2., L + 1) - 1); }
 
 // Make sure levels [0, Lb] of trajectory ip exist on the device with the right
-// (memory / extended) spacing.
+// (memory / extended) spacing.  block: the last level of the block built at
+// once, where it is chosen by the caller (the allocation-free entry point).
 void ensure_levels(om_context* ctx, int ip, int Lb, int stop_mem, LevelCache* lc_own = nullptr,
-                   Arena* ar = nullptr) {
+                   Arena* ar = nullptr, int block = kBlockLevel) {
   LevelCache& lc = lc_own ? *lc_own : ctx->levels[ip];
   const om::TrajDesc& D = ctx->desc[ip];
   double ts = ctx->tstart[ip], te = ctx->tstop[ip];
-  for (int L = 0; L <= Lb; ++L) {
+  if (lc.block < 0) {
+    const size_t n = 10 * (size_t) ((2L << block) - 1);
+    double* b = ar ? ar->take<double>(n + om::kMaxLevel + 1) : nullptr;
+    if (!ar) {
+      if (g_no_alloc) throw std::logic_error("device allocation inside the allocation-free entry point");
+      check(hipMalloc((void**) &b, (n + om::kMaxLevel + 1) * sizeof(double)), "hipMalloc levels");
+    }
+    for (int L = 0; L <= block; ++L) lc.rows[L] = b + 10 * ((1L << L) - 1);
+    lc.bd = b + n;
+    lc.block = block;
+  }
+  bool stale = false;
+  for (int L = 0; L <= lc.block && L <= Lb; ++L) stale = stale || !lc.built[L] || lc.extended[L] != (L > stop_mem ? 1 : 0);
+  if (stale) {
+    for (int L = 0; L <= lc.block; ++L) {
+      lc.built[L] = true;
+      lc.extended[L] = L > stop_mem ? 1 : 0;
+      lc.have_bd[L] = false;
+    }
+    om::LevelsJob J;
+    J.t = ctx->d_t.p;
+    J.p = ctx->d_p.p;
+    J.ypp = ctx->d_ypp.p;
+    J.knot_offset = D.knot_offset;
+    J.n = D.n;
+    J.tstart = ts;
+    J.tstop = te;
+    J.out = lc.rows[0];
+    J.Lb = lc.block;
+    J.stop_mem = stop_mem;
+    check(om_launch_levels(&J, ctx->stream), "levels kernel");
+  }
+  for (int L = lc.block + 1; L <= Lb; ++L) {
     int ext = L > stop_mem ? 1 : 0;
     if (lc.rows[L] && lc.built[L] && lc.extended[L] == ext) continue;
     long np = 1L << L;
@@ -588,24 +626,19 @@ void ensure_levels(om_context* ctx, int ip, int Lb, int stop_mem, LevelCache* lc
   }
 }
 
-void ensure_beta_diff(om_context* ctx, int ip, int Lb) {
+// Largest beta steps of levels [0, Lb] (which must exist) on the device.
+const double* ensure_beta_diff(om_context* ctx, int ip, int Lb) {
   LevelCache& lc = ctx->levels[ip];
-  ctx->d_bd.ensure(om::kMaxLevel + 1);
-  bool any = false;
-  for (int L = 0; L <= Lb; ++L) {
+  if (!lc.have_bd[0]) {
+    check(om_launch_beta_diff(lc.rows[0], 0, lc.block + 1, lc.bd, ctx->stream), "beta diff");
+    for (int L = 0; L <= lc.block; ++L) lc.have_bd[L] = true;
+  }
+  for (int L = lc.block + 1; L <= Lb; ++L) {
     if (lc.have_bd[L]) continue;
-    check(om_launch_beta_diff(lc.rows[L], 1L << L, ctx->d_bd.p + L, ctx->stream), "beta diff");
-    any = true;
+    check(om_launch_beta_diff(lc.rows[L], L, 1, lc.bd, ctx->stream), "beta diff");
+    lc.have_bd[L] = true;
   }
-  if (!any) return;
-  double h[om::kMaxLevel + 1];
-  read_back(ctx, h, ctx->d_bd.p, sizeof(h));
-  for (int L = 0; L <= Lb; ++L) {
-    if (!lc.have_bd[L]) {
-      lc.beta_diff[L] = h[L];
-      lc.have_bd[L] = true;
-    }
-  }
+  return lc.bd;
 }
 
 void fill_levels(om_context* ctx, int ip, int Lb, om::Levels& lv, LevelCache* lc_own = nullptr) {
@@ -614,7 +647,6 @@ void fill_levels(om_context* ctx, int ip, int Lb, om::Levels& lv, LevelCache* lc
   for (int L = 0; L <= om::kMaxLevel; ++L) {
     lv.rows[L] = L <= Lb ? lc.rows[L] : nullptr;
     lv.dt_incl[L] = dt_inclusive(ctx->tstart[ip], ctx->tstop[ip], L);
-    lv.beta_diff[L] = lc.beta_diff[L];
   }
 }
 
@@ -627,7 +659,7 @@ T* scratch_buf(DevBuf<T>& b, size_t n, Arena* ar) {
   return b.p;
 }
 
-void state_for(om_context* ctx, long npts, bool mixed, om::State& st, Arena* ar = nullptr) {
+void state_for(om_context* ctx, long npts, bool mixed, om::State& st, Arena* ar = nullptr, bool reset = true) {
   st.sum = scratch_buf(ctx->d_sum, 6 * npts, ar);
   st.lastmag = scratch_buf(ctx->d_lastmag, npts, ar);
   st.prec = scratch_buf(ctx->d_prec, npts, ar);
@@ -635,7 +667,7 @@ void state_for(om_context* ctx, long npts, bool mixed, om::State& st, Arena* ar 
   st.conv = scratch_buf(ctx->d_conv, npts, ar);
   st.err = mixed ? scratch_buf(ctx->d_err, 2 * npts, ar) : nullptr;
   st.border = mixed ? scratch_buf(ctx->d_border, npts, ar) : nullptr;
-  check(om_launch_state_reset(&st, npts, ctx->stream), "state reset");
+  if (reset) check(om_launch_state_reset(&st, npts, ctx->stream), "state reset");
 }
 
 long count_active(om_context* ctx, const om::State& st, long npts) {
@@ -652,6 +684,14 @@ constexpr int kFirstLevels = 13;
 // Per-point modes: levels with at most this many active points run one wave per
 // point (the per-point kernel would fill only a fraction of the GPU).
 constexpr long kWaveListMax = 16384;
+// Tiled modes: requests of at most this many (observation point, 64 energies)
+// groups go through their levels in slices (lw_slice_kernel): 32 groups 1.1 ms
+// against 1.7 ms.  Beyond, a wave or more per group fills the GPU and the lists
+// pack an observation point's energies across its groups: 1444 groups 3.3 ms
+// against 3.7 ms.  The slices' 17 MB of partial sums fit into the static scratch
+// of the allocation-free entry point beside level 18 (42 MB, the deepest that
+// fits) and 65536 points.
+constexpr long kSliceGroups = 1024;
 constexpr int kListFrom = 9;  // first level that can stop a point (src/OSCARSSR.cc:2006: L > 8)
 
 // Waits for the last om_trajectories and reads back the per-trajectory status.
@@ -898,7 +938,14 @@ int lw_sums(om_context* ctx, int ip, const double* obs_xyz, long n_obs, const do
     bool mixed_any = mixed || conv->mode == OM_MODE_POINT_MIXED;
     om::LwArgs A;
     std::memset(&A, 0, sizeof(A));
-    state_for(ctx, npts, mixed_any, A.st, ar);
+    const bool tiled = !(conv->mode == OM_MODE_PLAIN || conv->mode == OM_MODE_POINT_MIXED);
+    // precision <= 0: no point stops before the cap (prec < precision never
+    // holds), so the first launch takes every level and nothing is compacted
+    const bool capped = conv->precision <= 0 && stop_ext == stop_mem;
+    const long blocks_e = (n_e + 63) / 64;
+    const bool sliced = tiled && !capped && n_obs * blocks_e <= kSliceGroups && stop_ext >= kListFrom;
+    const bool waves = !tiled && npts <= kWaveListMax;  // one wave per point from the start
+    state_for(ctx, npts, mixed_any, A.st, ar, !sliced);
     A.npts = npts;
     A.obs = ar ? d_obs : ctx->d_obs.p;
     A.omega = ar ? d_omega : ctx->d_omega.p;
@@ -925,25 +972,39 @@ int lw_sums(om_context* ctx, int ip, const double* obs_xyz, long n_obs, const do
     A.precision = conv->precision;
     float kms = 0;
     int La = 0;
-    bool tiled = !(conv->mode == OM_MODE_PLAIN || conv->mode == OM_MODE_POINT_MIXED);
     // Levels 0..8 (no point can stop before level 9) in one dense launch, then
     // one launch per level over the points still active, compacted into full
-    // waves (tiles of one observation point for the tiled kernels).
-    int Lb = stop_ext < kListFrom - 1 ? stop_ext : kListFrom - 1;
-    // precision <= 0: no point stops before the cap (prec < precision never
-    // holds), so the dense launch takes every level and nothing is compacted
-    if (conv->precision <= 0 && stop_ext == stop_mem) Lb = stop_ext;
+    // waves (tiles of one observation point for the tiled kernels).  Requests
+    // small enough to go on by themselves take levels 0..13 before the host looks.
+    int Lb = std::min(stop_ext, sliced || waves ? kBlockLevel : kListFrom - 1);
+    if (capped) Lb = stop_ext;
     long ntiles = 0;
     long n_recheck = 0;
     int Ldone = 0;  // deepest level summed so far (its samples exist)
+    const int block = ar && !(sliced || waves) ? kListFrom - 1 : kBlockLevel;
     while (true) {
-      ensure_levels(ctx, ip, Lb, stop_mem, lc, ar);
+      ensure_levels(ctx, ip, Lb, stop_mem, lc, ar, block);
       fill_levels(ctx, ip, Lb, A.lv, lc);
       A.La = La;
       A.Lb = Lb;
       if (!ar) ctx->timer.begin(ctx->stream);
-      if (!tiled && A.list && A.n_list <= kWaveListMax) {
-        // few points left: one wave per point
+      if (sliced && La == 0) {
+        om::SliceArgs X;
+        X.n_groups = n_obs * blocks_e;
+        X.blocks_e = blocks_e;
+        X.part = scratch_buf(ctx->d_part, (size_t) om::kSliceJobs * 8 * 64, ar);
+        const bool fresh = ar || !ctx->d_arrived.p;  // zero between launches
+        X.arrived = scratch_buf(ctx->d_arrived, kSliceGroups, ar);
+        if (fresh)
+          check(om_launch_adj_key_fill(reinterpret_cast<int*>(X.arrived), kSliceGroups, 0, ctx->stream), "clear");
+        for (int L = kListFrom - 1; L <= Lb; ++L) {
+          const long most = L < kListFrom ? 8 : (1L << L) / om::kSliceMin;
+          X.L = L;
+          X.nsl = (int) std::max(1L, std::min(most, om::kSliceJobs / X.n_groups));
+          check(om_launch_lw_slice(&A, &X, mixed ? 1 : 0, ctx->stream), "lw_slice");
+        }
+      } else if (!tiled && (A.list ? A.n_list : npts) <= kWaveListMax) {
+        // few points: one wave per point
         check(om_launch_lw_wave(&A, conv->mode == OM_MODE_POINT_MIXED ? 1 : 0, ctx->stream), "lw_wave");
       } else if (!tiled) {
         check(om_launch_lw_point(&A, conv->mode == OM_MODE_POINT_MIXED ? 1 : 0, ctx->split, ctx->stream),
@@ -996,7 +1057,7 @@ int lw_sums(om_context* ctx, int ip, const double* obs_xyz, long n_obs, const do
         La = 0;
         Lb = Ldone;
         while (true) {
-          ensure_levels(ctx, ip, Lb, stop_mem, lc, ar);
+          ensure_levels(ctx, ip, Lb, stop_mem, lc, ar, block);
           fill_levels(ctx, ip, Lb, A.lv, lc);
           A.La = La;
           A.Lb = Lb;
@@ -1414,7 +1475,7 @@ int power_density(om_context* ctx, int ip, const double* obs_xyz, long n_obs, co
       int Ldone = La;
       while (true) {
         ensure_levels(ctx, ip, Lb, stop_mem);
-        ensure_beta_diff(ctx, ip, Lb);
+        A.beta_diff = ensure_beta_diff(ctx, ip, Lb);
         fill_levels(ctx, ip, Lb, A.lv);
         A.La = La;
         A.Lb = Lb;
@@ -1696,7 +1757,7 @@ int om_total_power(om_context* ctx, int ip, const om_conv* conv, double* out_pow
     while (La <= stop_ext && Result_Level == -1) {
       int Lb = La == 0 ? (stop_ext < kFirstLevels ? stop_ext : kFirstLevels) : La;
       ensure_levels(ctx, ip, Lb, stop_mem);
-      ensure_beta_diff(ctx, ip, Lb);
+      const double* d_bd = ensure_beta_diff(ctx, ip, Lb);
       ctx->d_tp_partial.ensure(om_tp_blocks(1L << Lb));
       for (int L = La; L <= Lb; ++L) {
         om::TpArgs T;
@@ -1709,13 +1770,15 @@ int om_total_power(om_context* ctx, int ip, const om_conv* conv, double* out_pow
         ctx->timer.end(ctx->stream);
       }
       double h[om::kMaxLevel + 1];
+      double bd[om::kMaxLevel + 1];
       read_back(ctx, h + La, ctx->d_tp.p + La, (Lb - La + 1) * sizeof(double));
+      read_back(ctx, bd + La, d_bd + La, (Lb - La + 1) * sizeof(double));
       for (int L = La; L <= Lb; ++L) {
         Sum += h[L];
         evals += (double) (1L << L);
         double ThisSum = Sum * dt_inclusive(ctx->tstart[ip], ctx->tstop[ip], L);
         Result_Precision = std::fabs(ThisSum - LastSum) / LastSum;
-        if (L > 8 && Result_Precision < conv->precision && ctx->levels[ip].beta_diff[L] < 2. / P.gamma) {
+        if (L > 8 && Result_Precision < conv->precision && bd[L] < 2. / P.gamma) {
           Result_Level = L;
           LastSum = ThisSum;
           break;

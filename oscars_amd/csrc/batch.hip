@@ -68,20 +68,20 @@ __device__ __forceinline__ unsigned long long uniform_u64(unsigned long long v) 
   return ((unsigned long long) hi << 32) | lo;
 }
 
-// LDS of one persistent wave: the amplitudes of the current super-block of
-// kSuper samples (one double of padding after every 16 samples, so replicas
-// that walk different parts of it read different banks) and the active list.
-constexpr int kSuper = 256;
-constexpr int kBlkPad = kSuper + kSuper / 16;
-__device__ __forceinline__ int blk(int k) { return k + (k >> 4); }
-
-struct BatchLds {
-  double tau[kBlkPad];
-  double vx[kBlkPad];
-  double vy[kBlkPad];
-  double vz[kBlkPad];
+// LDS of one persistent wave: the amplitudes of the current super-block and the
+// active list.
+struct BatchLds : AmpLds {
   unsigned short list[kBatchEB];
 };
+
+// One atomic for the wave, by lane 0, its old value in every lane.  (An atomic
+// executed by all lanes with zeros but in lane 0 is 64 operations on one
+// address, one after the other.)
+__device__ __forceinline__ unsigned long long wave_add(unsigned long long* p, int lane, unsigned long long v) {
+  unsigned long long old = 0;
+  if (lane == 0) old = atomicAdd(p, v);
+  return uniform_u64(old);
+}
 
 // One work unit (particle ip, observation point io, energies e0 .. e0+n_eb-1).
 struct Unit {
@@ -157,33 +157,6 @@ __device__ __forceinline__ void batch_add_point(const BatchArgs& A, const Unit& 
   atomicAdd(A.evals, (unsigned long long) ((2L << lev) - 1));
 }
 
-// The m replicas of W energies added into replica 0 (lanes 0..W-1): replicas
-// q..q+2s-1 into replica q, for s = 1, 2, 4, ..., in the same order for every
-// group shape.
-__device__ __forceinline__ void add_replicas(double ps[6], double& maxd, double& an, int lane, int W, int m, int q,
-                                             bool act) {
-  for (int st = 1; st < m; st <<= 1) {
-    const int src = lane + st * W < 64 ? lane + st * W : lane;
-    const bool take = act && (q % (2 * st)) == 0 && q + st < m;
-#pragma unroll
-    for (int c = 0; c < 6; ++c) {
-      double o = __shfl(ps[c], src);
-      ps[c] = take ? ps[c] + o : ps[c];
-    }
-    double om = __shfl(maxd, src), oa = __shfl(an, src);
-    maxd = take ? fmax(maxd, om) : maxd;
-    an = take ? an + oa : an;
-  }
-}
-
-// A partial sum that another XCD's wave reads in the same launch.
-__device__ __forceinline__ void part_store(double* p, double v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ double part_load(const double* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Flags of an energy in the wave's scratch.
 constexpr int kFConverged = 1;
 constexpr int kFBorderline = 2;  // mixed pass: a stop decision lay within the sin/cos error bound
@@ -234,7 +207,7 @@ __device__ __forceinline__ void unit_levels(const BatchArgs& A, const Unit& U, i
     if (L == A.Ldeep) {
       const int ng = (n_act + 63) >> 6;
       const unsigned long long g0 =
-          uniform_u64(atomicAdd(A.n_group, lane == 0 ? (unsigned long long) ng : 0ULL));
+          wave_add(A.n_group, lane, (unsigned long long) ng);
       if (g0 + (unsigned long long) ng <= (unsigned long long) A.group_cap) {
         constexpr int kind = SC32 ? 0 : 1;
         for (int g = 0; g < ng; ++g) {
@@ -258,7 +231,7 @@ __device__ __forceinline__ void unit_levels(const BatchArgs& A, const Unit& U, i
             A.group_list[(2 * kind + (L & 1)) * A.group_cap + (long) j] = (int) id;
           }
         }
-        atomicAdd(A.n_deep, lane == 0 ? (unsigned long long) n_act : 0ULL);
+        if (lane == 0) atomicAdd(A.n_deep, (unsigned long long) n_act);
         __syncthreads();
         break;
       }
@@ -475,10 +448,10 @@ __device__ __forceinline__ void batch_unit(const BatchArgs& A, long item, int la
     if (n_re > 0) {
       unit_levels<false>(A, U, lane, ws, wsi, S, kFConverged | kFHanded | kFIdle, n_amp, n_ev, n_slot);
     }
-    atomicAdd(A.n_recheck, lane == 0 ? (unsigned long long) n_re : 0ULL);
+    if (lane == 0 && n_re > 0) atomicAdd(A.n_recheck, (unsigned long long) n_re);
   }
-  // outputs and bookkeeping for the block's energies (all lanes take part in
-  // the atomics; only lane 0 adds nonzero counts)
+  // outputs and bookkeeping for the block's energies
+  unsigned long long n_unc = 0, n_evals = 0;  // lane 0's
   for (int t = 0; t < n_eb; t += 64) {
     const int e = t + lane;
     const int ec = e < n_eb ? e : 0;
@@ -496,12 +469,16 @@ __device__ __forceinline__ void batch_unit(const BatchArgs& A, long item, int la
     unsigned long long nc = __ballot(v && !(flags & kFConverged));
     unsigned long long ev = v ? (unsigned long long) ((2L << lev) - 1) : 0ULL;
     for (int off = 32; off > 0; off >>= 1) ev += __shfl_down(ev, off);
-    atomicAdd(A.n_unconverged, lane == 0 ? (unsigned long long) __popcll(nc) : 0ULL);
-    atomicAdd(A.evals, lane == 0 ? ev : 0ULL);
+    n_unc += (unsigned long long) __popcll(nc);
+    n_evals += ev;
   }
-  atomicAdd(A.main_amps, lane == 0 ? n_amp : 0ULL);
-  atomicAdd(A.main_evals, lane == 0 ? n_ev : 0ULL);
-  atomicAdd(A.main_slots, lane == 0 ? n_slot : 0ULL);
+  if (lane == 0) {
+    if (n_unc) atomicAdd(A.n_unconverged, n_unc);
+    atomicAdd(A.evals, n_evals);
+    atomicAdd(A.main_amps, n_amp);
+    atomicAdd(A.main_evals, n_ev);
+    atomicAdd(A.main_slots, n_slot);
+  }
   __syncthreads();  // the next unit overwrites the scratch
 }
 
@@ -514,13 +491,9 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) lw
   double* ws = A.ws + (long) blockIdx.x * kBatchWsTotal;
   int* wsi = A.wsi + (long) blockIdx.x * kBatchWsI * kBatchEB;
   while (true) {
-    // Next work unit.  Every lane executes the atomic (lane 0 adds 1, the others
-    // 0) and the index is taken from lane 0 with readfirstlane, so it is a
-    // scalar and the loop exit is a uniform branch.  No lane-conditional block
-    // surrounds a cross-lane operation, which keeps the compiler from splitting
-    // the wave between two copies of the loop.
-    unsigned long long mine = atomicAdd(A.counter, lane == 0 ? 1ULL : 0ULL);
-    long item = (long) uniform_u64(mine);
+    // Next work unit: the index is taken from lane 0 with readfirstlane, so it is
+    // a scalar and the loop exit a uniform branch.
+    const long item = (long) wave_add(A.counter, lane, 1ULL);
     if (item >= A.total_items) break;
     batch_unit<MIXED>(A, item, lane, ws, wsi, S);
   }
@@ -558,7 +531,7 @@ lw_batch_level_kernel(BatchArgs A, int L) {
   nsl = nsl > ns / 512 ? ns / 512 : nsl;
   const int* __restrict__ ids = A.group_list + (2 * kind + (L & 1)) * A.group_cap;
   while (true) {
-    const long job = (long) uniform_u64(atomicAdd(&A.n_job[kind * kBatchLevels + L], lane == 0 ? 1ULL : 0ULL));
+    const long job = (long) wave_add(&A.n_job[kind * kBatchLevels + L], lane, 1ULL);
     if (job >= n * nsl) break;
     const long gi = job / nsl, sl = job - gi * nsl;
     const long id = ids[gi];
@@ -581,77 +554,16 @@ lw_batch_level_kernel(BatchArgs A, int L) {
                     : interpolated_amplitude(A, U.D, U.obs, tfirst + spacing * (double) i);
     };
     const long i0 = ns * sl / nsl, i1 = ns * (sl + 1) / nsl;
-    double tprev = i0 > 0 ? amp_at(i0 - 1).tau : 0.0;
-    double ps[6] = {0, 0, 0, 0, 0, 0};
-    double maxd = 0, anl = 0;
-    for (long base = i0; base < i1; base += kSuper) {
-      const int cnt = (int) (i1 - base < kSuper ? i1 - base : kSuper);
-#pragma unroll 1
-      for (int h = 0; h < kSuper; h += 64) {
-        if (h + lane < cnt) {
-          const Amp a = amp_at(base + h + lane);
-          S.tau[blk(h + lane)] = a.tau;
-          S.vx[blk(h + lane)] = a.V.x;
-          S.vy[blk(h + lane)] = a.V.y;
-          S.vz[blk(h + lane)] = a.V.z;
-          if (SC32) anl += fabs(a.V.x) + fabs(a.V.y) + fabs(a.V.z);
-        }
-      }
-      wave_sync();
-      const int k0 = act ? (q * cnt) / m : 0;
-      const int k1 = act ? ((q + 1) * cnt) / m : 0;
-      double lastphase = negw * (k0 > 0 ? S.tau[blk(k0 - 1)] : (base > 0 ? tprev : S.tau[0]));
-#pragma unroll 4
-      for (int k = k0; k < k1; ++k) {
-        const int b = blk(k);
-        double phi = negw * S.tau[b];
-        maxd = fmax(maxd, fabs(phi - lastphase));
-        lastphase = phi;
-        double sn, cs;
-        sincos_mode(SC32, phi, sn, cs);
-        double vx = S.vx[b], vy = S.vy[b], vz = S.vz[b];
-        ps[0] = __builtin_fma(vx, cs, ps[0]); ps[1] = __builtin_fma(vx, sn, ps[1]);
-        ps[2] = __builtin_fma(vy, cs, ps[2]); ps[3] = __builtin_fma(vy, sn, ps[3]);
-        ps[4] = __builtin_fma(vz, cs, ps[4]); ps[5] = __builtin_fma(vz, sn, ps[5]);
-      }
-      tprev = S.tau[blk(cnt - 1)];
-      wave_sync();  // the next super-block overwrites the amplitudes
-    }
+    double ps[6], maxd, anl;
+    walk_slice<SC32>(amp_at, i0, i1, negw, lane, m, q, act, S, ps, maxd, anl);
     double none = 0;
     add_replicas(ps, maxd, none, lane, W, m, q, act);
-    if (SC32) {
-      for (int off = 32; off > 0; off >>= 1) anl += __shfl_xor(anl, off);
-    }
     const bool mine = lane < W;  // replica 0
     if (nsl > 1) {
-      // partial sums through the device's coherence point (no cache write-back):
-      // stores that bypass the caches, waited for before the arrival is counted
-      double* pp = A.part + (gi * nsl + sl) * (8 * 64) + lane;
-      if (mine) {
-#pragma unroll
-        for (int c = 0; c < 6; ++c) part_store(pp + 64 * c, ps[c]);
-        part_store(pp + 64 * 6, maxd);
-        part_store(pp + 64 * 7, anl);
-      }
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      const unsigned before = (unsigned) __builtin_amdgcn_readfirstlane(
-          (int) atomicAdd(&A.group_arrived[id], lane == 0 ? 1u : 0u));
-      if (before + 1 < (unsigned) nsl) continue;
+      part_publish(A.part + (gi * nsl + sl) * (8 * 64), lane, mine, ps, maxd, anl);
+      if (part_arrive(&A.group_arrived[id], lane) + 1 < (unsigned) nsl) continue;
       if (lane == 0) A.group_arrived[id] = 0;
-      // replica q adds slices q, q + m, ...
-#pragma unroll
-      for (int c = 0; c < 6; ++c) ps[c] = 0;
-      maxd = anl = 0;
-      const double* pg = A.part + gi * nsl * (8 * 64) + slot;
-#pragma unroll 4
-      for (long s = act ? q : nsl; s < nsl; s += m) {
-        const double* p = pg + s * (8 * 64);
-#pragma unroll
-        for (int c = 0; c < 6; ++c) ps[c] += part_load(p + 64 * c);
-        maxd = fmax(maxd, part_load(p + 64 * 6));
-        anl += part_load(p + 64 * 7);
-      }
-      add_replicas(ps, maxd, anl, lane, W, m, q, act);
+      part_gather(A.part + gi * nsl * (8 * 64), nsl, lane, W, m, q, act, ps, maxd, anl);
     }
     // decisions, one energy per lane; the others' lanes hold none
     double* gs = A.group_state + id * (kBatchGroupD * 64);
@@ -725,8 +637,7 @@ __global__ void __launch_bounds__(256) lw_batch_fix_kernel(BatchArgs A) {
     bool c = false, border = false, handed = false;
     for (int L = 0; L <= A.Lmax && !c; ++L) {
       if (L == A.Ldeep) {
-        const unsigned long long id =
-            uniform_u64(atomicAdd(A.n_group, lane == 0 ? 1ULL : 0ULL));
+        const unsigned long long id = wave_add(A.n_group, lane, 1ULL);
         if (id < (unsigned long long) A.group_cap) {
           if (lane == 0) {
             double* st = A.group_state + (long) id * (kBatchGroupD * 64);

@@ -10,7 +10,6 @@ namespace om {
 struct Levels {
   const double* rows[kMaxLevel + 1];  // 2^L rows of 10 doubles per level (device)
   double dt_incl[kMaxLevel + 1];      // (tstop - tstart) / (2^(L+1) - 1)
-  double beta_diff[kMaxLevel + 1];    // per level max |beta_i - beta_{i-1}| (power density)
 };
 
 struct State {
@@ -42,6 +41,7 @@ struct LwArgs {
 
 struct PdArgs {
   Levels lv;
+  const double* beta_diff;  // per level max |beta_i - beta_{i-1}| (device)
   State st;
   int La, Lb;
   long npts;
@@ -103,6 +103,18 @@ struct FinArgs {
   unsigned char* out_conv;
 };
 
+// One step of the sliced sums of a small tiled request (lw_slice_kernel).
+constexpr int kSliceJobs = 4096;  // waves a step is cut into, and partial sums held
+constexpr int kSliceMin = 256;    // samples a slice has at least, above level 8
+struct SliceArgs {
+  int L;           // the level summed; 8: levels 0..8 together (no point stops before level 9)
+  long n_groups;   // (observation point, 64 energies) groups
+  long blocks_e;   // groups per observation point
+  int nsl;         // slices per group
+  double* part;    // 8 x 64 per (group, slice)
+  unsigned* arrived;  // per group, zero between launches
+};
+
 // ---- trajectories in parallel segments (shoot.hip)
 constexpr int kShootWaves = 4;   // waves per workgroup, eight segments each
 constexpr int kShootWalk = 64;   // maps of other workgroups held in LDS at a time
@@ -143,6 +155,19 @@ struct LevelJob {
   double* out;          // destination rows (10 doubles) for this level
   long npts;            // 2^L
   double t_first, spacing;
+};
+
+// Levels 0..Lb of one trajectory as one block: level L at row 2^L - 1.
+struct LevelsJob {
+  const double* t;
+  const double* p;
+  const double* ypp;
+  long knot_offset;
+  long n;
+  double tstart, tstop;
+  double* out;
+  int Lb;
+  int stop_mem;  // levels above it use the extended spacing
 };
 
 struct LevelJobBatch {

@@ -358,6 +358,91 @@ __global__ void __launch_bounds__(64 * S) lw_tile_kernel(LwArgs A, long n_tiles_
   }
 }
 
+// ---------------------------------------------------------------- sliced tiles
+// A spectrum or a small sweep has few (observation point, 64 energies) groups:
+// 32 for 2000 energies on axis, 256 waves with a level shared by 8, a quarter of
+// the SIMDs, waiting for the host's look at the active list before every level
+// (0.43 ms of kernels and 0.4 ms of lists and waits for 6 levels).  Here a level
+// of every group is cut into slices, about kSliceJobs in all (4096: four waves a
+// SIMD); a group's active energies are packed from their flags by each of its
+// slices, in replicas when few are left; and the slice that completes a group
+// adds the partial sums and takes the decisions.  The levels follow each other
+// on the stream with no look from the host.  Bound by the chain of one slice:
+// 37 us a level, of which 256 samples in FP64 take 25.  2000 energies on axis:
+// 1.73 -> 1.13 ms a call, 0.18 ms of it in these launches.
+template <bool MIXED>
+__global__ void __launch_bounds__(256) lw_slice_kernel(LwArgs A, SliceArgs X) {
+  __shared__ AmpLds lds[4];
+  __shared__ unsigned char lists[4][64];
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const long job = (long) blockIdx.x * 4 + wv;
+  if (job >= X.n_groups * X.nsl) return;  // whole waves leave; no workgroup barrier below
+  const long g = job / X.nsl, sl = job - g * X.nsl;
+  const long io = g / X.blocks_e, e0 = (g - io * X.blocks_e) * 64;
+  const bool first = X.L == 8;
+  const long p0 = io * A.n_omega + e0;
+  const bool in = e0 + lane < A.n_omega;
+  const bool live = in && (first || (!A.st.conv[p0 + lane] && A.st.level[p0 + lane] == X.L - 1));
+  const unsigned long long mask = __ballot(live);
+  const int W = __popcll(mask);
+  if (W == 0) return;  // the same for every slice of the group: its state changes after all have arrived
+  unsigned char* list = lists[wv];
+  if (live) list[__popcll(mask & ((1ULL << lane) - 1ULL))] = (unsigned char) lane;
+  wave_sync();
+  const int m = 64 / W, q = lane / W;
+  const bool act = q < m;
+  const int e = list[act ? lane - q * W : 0];
+  const double negw = -A.omega[e0 + e];
+  const V3 obs = v3(A.obs[3 * io], A.obs[3 * io + 1], A.obs[3 * io + 2]);
+  // levels 0..8 lie one after the other: their sums are one sum of 511 samples
+  const double* __restrict__ rows = A.lv.rows[first ? 0 : X.L];
+  const long ns = first ? 511 : 1L << X.L;
+  double ps[6], maxd, an;
+  walk_slice<MIXED>([&](long i) { return amplitude(obs, rows + 10 * i); }, ns * sl / X.nsl, ns * (sl + 1) / X.nsl, negw,
+                    lane, m, q, act, lds[wv], ps, maxd, an);
+  double none = 0;
+  add_replicas(ps, maxd, none, lane, W, m, q, act);
+  const bool mine = lane < W;
+  if (X.nsl > 1) {
+    part_publish(X.part + job * (8 * 64), lane, mine, ps, maxd, an);
+    if (part_arrive(&X.arrived[g], lane) + 1 < (unsigned) X.nsl) return;
+    if (lane == 0) X.arrived[g] = 0;
+    part_gather(X.part + g * X.nsl * (8 * 64), X.nsl, lane, W, m, q, act, ps, maxd, an);
+  }
+  if (!mine) return;
+  const long p = p0 + e;
+  double sum[6], lastmag = -1, prec = -1, an_run = an, dm_last = 0;
+  if (first) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) sum[k] = ps[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) sum[k] = A.st.sum[6 * p + k] + ps[k];
+    lastmag = A.st.lastmag[p];
+    if (MIXED) {
+      an_run += A.st.err[2 * p];
+      dm_last = A.st.err[2 * p + 1];
+    }
+  }
+  const double mag_prev = lastmag;
+  bool c = level_converged(A, X.L, sum, maxd, lastmag, prec);
+  if (MIXED) {
+    // a borderline decision sends the point to the FP64 recomputation: it stops here
+    const bool border = level_borderline(X.L, A.lv.dt_incl[X.L], A.precision, mag_prev, lastmag, prec, maxd, an_run,
+                                         dm_last);
+    c = c || border;
+    A.st.err[2 * p] = an_run;
+    A.st.err[2 * p + 1] = dm_last;
+    if (first || border) A.st.border[p] = border ? 1 : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) A.st.sum[6 * p + k] = sum[k];
+  A.st.lastmag[p] = lastmag;
+  A.st.prec[p] = prec;
+  A.st.level[p] = X.L;
+  if (first || c) A.st.conv[p] = c ? 1 : 0;
+}
+
 // ---------------------------------------------------------------- power density
 // Bound by the issue of the terms' instructions (FP64: ~112 per term, a square
 // root, a reciprocal and two quotients the most of them; mixed ~65).  The lanes
@@ -501,7 +586,7 @@ __device__ __forceinline__ bool pd_level_end(const PdArgs& A, int L, double ps, 
   double thisSum = q.sum * dt;
   double prev = q.lastsum;
   q.prec = fabs(thisSum - q.lastsum) / q.lastsum;
-  double bd = A.lv.beta_diff[L];
+  double bd = A.beta_diff[L];
   bool c = (L > 8 && q.prec < A.precision && bd < A.two_over_gamma) ||
            (L > 8 && bd < A.two_over_gamma && thisSum == q.lastsum);
   bool c2 = !c && L > 8 && thisSum == q.lastsum;
@@ -855,18 +940,19 @@ __global__ void __launch_bounds__(256) lw_finalize_kernel(FinArgs F) {
   if (F.out_conv) F.out_conv[p] = (unsigned char) conv;
 }
 
-// Listed points, one wave per point, the lanes splitting each level's
+// One wave per point (all, or the listed ones), the lanes splitting each level's
 // samples, levels La..Lb from the point's state.  Used where few points are
-// active (the last levels of a map, and the FP64 recomputation of the mixed
-// path's borderline points): a wave per point keeps their latency low.
+// active (maps of at most 16384 points, the last levels of larger ones, and the
+// FP64 recomputation of the mixed path's borderline points): a wave per point
+// keeps their latency low and goes from level to level by itself.
 // MIXED: reduced-accuracy sin/cos with the error-bound bookkeeping of the per-point kernel.
 // Four waves (points) per workgroup.
 template <bool MIXED>
 __global__ void __launch_bounds__(256) lw_wave_kernel(LwArgs A) {
   int lane = threadIdx.x & 63;
   long g = (long) blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (g >= A.n_list) return;  // whole waves leave; no workgroup barrier below
-  long p = A.list[g];
+  if (g >= (A.list ? A.n_list : A.npts)) return;  // whole waves leave; no workgroup barrier below
+  long p = A.list ? (long) A.list[g] : g;
   if (A.st.conv[p] || A.st.level[p] != A.La - 1) return;
   long io = p / A.n_omega;
   long iw = p - io * A.n_omega;
@@ -1172,8 +1258,15 @@ extern "C" hipError_t om_launch_lw_tile_list(const om::LwArgs* A, long ntiles, i
   return hipGetLastError();
 }
 
+extern "C" hipError_t om_launch_lw_slice(const om::LwArgs* A, const om::SliceArgs* X, int mixed, hipStream_t s) {
+  const dim3 g((unsigned) ((X->n_groups * X->nsl + 3) / 4));
+  if (mixed) hipLaunchKernelGGL(om::lw_slice_kernel<true>, g, dim3(256), 0, s, *A, *X);
+  else hipLaunchKernelGGL(om::lw_slice_kernel<false>, g, dim3(256), 0, s, *A, *X);
+  return hipGetLastError();
+}
+
 extern "C" hipError_t om_launch_lw_wave(const om::LwArgs* A, int mixed, hipStream_t s) {
-  long blocks = (A->n_list + 3) / 4;
+  long blocks = ((A->list ? A->n_list : A->npts) + 3) / 4;
   if (blocks > 0) {
     if (mixed)
       hipLaunchKernelGGL(om::lw_wave_kernel<true>, dim3((unsigned) blocks), dim3(256), 0, s, *A);

@@ -206,6 +206,168 @@ __device__ __forceinline__ void slice_level_sum_rows(const double* __restrict__ 
   an = al;
 }
 
+// ---------------------------------------------------------------- slices of a level
+// A wave's share of a level for a group of W <= 64 energies of one observation
+// point (lw_slice_kernel, lw_batch_level_kernel).  LDS: the amplitudes of a
+// super-block of kSuper samples, one double of padding after every 16, so
+// replicas that walk different parts of it read different banks.
+constexpr int kSuper = 256;
+constexpr int kBlkPad = kSuper + kSuper / 16;
+__device__ __forceinline__ int blk(int k) { return k + (k >> 4); }
+
+// Samples whose sines and cosines are formed side by side: one after the other
+// they are one chain of dependent instructions, 500 cycles a sample where a SIMD
+// has a wave or two.
+constexpr int kAtOnce = 4;
+
+struct AmpLds {
+  double tau[kBlkPad];
+  double vx[kBlkPad];
+  double vy[kBlkPad];
+  double vz[kBlkPad];
+};
+
+// Samples [i0, i1) of a level, super-block by super-block: the lanes compute its
+// amplitudes (amp_at(i)), then each walks it at its energy -- W energies in m =
+// 64 / W replicas, replica q taking the q-th contiguous part.  ps and maxd are
+// the lane's partial sums and largest phase step (the sample before the slice
+// and before each part included), an the wave's sum of |V|_1 (mixed).
+template <bool MIXED, class AmpAt>
+__device__ __forceinline__ void walk_slice(AmpAt amp_at, long i0, long i1, double negw, int lane, int m, int q,
+                                           bool act, AmpLds& S, double ps[6], double& maxd, double& an) {
+#pragma unroll
+  for (int c = 0; c < 6; ++c) ps[c] = 0;
+  maxd = an = 0;
+  double tprev = i0 > 0 ? amp_at(i0 - 1).tau : 0.0;
+  for (long base = i0; base < i1; base += kSuper) {
+    const int cnt = (int) (i1 - base < kSuper ? i1 - base : kSuper);
+#pragma unroll 1
+    for (int h = 0; h < kSuper; h += 64) {
+      if (h + lane < cnt) {
+        const Amp a = amp_at(base + h + lane);
+        S.tau[blk(h + lane)] = a.tau;
+        S.vx[blk(h + lane)] = a.V.x;
+        S.vy[blk(h + lane)] = a.V.y;
+        S.vz[blk(h + lane)] = a.V.z;
+        if (MIXED) an += fabs(a.V.x) + fabs(a.V.y) + fabs(a.V.z);
+      }
+    }
+    wave_sync();
+    const int k0 = act ? (q * cnt) / m : 0;
+    const int k1 = act ? ((q + 1) * cnt) / m : 0;
+    double lastphase = negw * (k0 > 0 ? S.tau[blk(k0 - 1)] : (base > 0 ? tprev : S.tau[0]));
+    int k = k0;
+    for (; k + kAtOnce <= k1; k += kAtOnce) {
+      double phi[kAtOnce], sn[kAtOnce], cs[kAtOnce], vx[kAtOnce], vy[kAtOnce], vz[kAtOnce];
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) {
+        const int b = blk(k + u);
+        phi[u] = negw * S.tau[b];
+        vx[u] = S.vx[b];
+        vy[u] = S.vy[b];
+        vz[u] = S.vz[b];
+      }
+      sincos_n<MIXED, kAtOnce>(phi, sn, cs);
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) {
+        maxd = fmax(maxd, fabs(phi[u] - (u > 0 ? phi[u - 1] : lastphase)));
+        ps[0] = __builtin_fma(vx[u], cs[u], ps[0]); ps[1] = __builtin_fma(vx[u], sn[u], ps[1]);
+        ps[2] = __builtin_fma(vy[u], cs[u], ps[2]); ps[3] = __builtin_fma(vy[u], sn[u], ps[3]);
+        ps[4] = __builtin_fma(vz[u], cs[u], ps[4]); ps[5] = __builtin_fma(vz[u], sn[u], ps[5]);
+      }
+      lastphase = phi[kAtOnce - 1];
+    }
+    for (; k < k1; ++k) {
+      const int b = blk(k);
+      double phi = negw * S.tau[b];
+      maxd = fmax(maxd, fabs(phi - lastphase));
+      lastphase = phi;
+      double sn, cs;
+      sincos_mode(MIXED, phi, sn, cs);
+      double vx = S.vx[b], vy = S.vy[b], vz = S.vz[b];
+      ps[0] = __builtin_fma(vx, cs, ps[0]); ps[1] = __builtin_fma(vx, sn, ps[1]);
+      ps[2] = __builtin_fma(vy, cs, ps[2]); ps[3] = __builtin_fma(vy, sn, ps[3]);
+      ps[4] = __builtin_fma(vz, cs, ps[4]); ps[5] = __builtin_fma(vz, sn, ps[5]);
+    }
+    tprev = S.tau[blk(cnt - 1)];
+    wave_sync();  // the next super-block overwrites the amplitudes
+  }
+  if (MIXED) {
+    for (int off = 32; off > 0; off >>= 1) an += __shfl_xor(an, off);
+  }
+}
+
+// The m replicas of W energies added into replica 0 (lanes 0..W-1): replicas
+// q..q+2s-1 into replica q, for s = 1, 2, 4, ..., in the same order for every
+// group shape.
+__device__ __forceinline__ void add_replicas(double ps[6], double& maxd, double& an, int lane, int W, int m, int q,
+                                             bool act) {
+  for (int st = 1; st < m; st <<= 1) {
+    const int src = lane + st * W < 64 ? lane + st * W : lane;
+    const bool take = act && (q % (2 * st)) == 0 && q + st < m;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      double o = __shfl(ps[c], src);
+      ps[c] = take ? ps[c] + o : ps[c];
+    }
+    double om = __shfl(maxd, src), oa = __shfl(an, src);
+    maxd = take ? fmax(maxd, om) : maxd;
+    an = take ? an + oa : an;
+  }
+}
+
+// Partial sums that another XCD's wave reads in the same launch (8 x 64 doubles
+// per slice): stores that bypass the caches, with no write-back, waited for, so
+// the caller's arrival count follows them; the reader drops its caches' copies
+// once and loads them plainly, many at a time.
+__device__ __forceinline__ void part_publish(double* p, int lane, bool mine, const double ps[6], double maxd,
+                                             double an) {
+  if (mine) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      __hip_atomic_store(p + 64 * c + lane, c < 6 ? ps[c < 6 ? c : 0] : (c == 6 ? maxd : an), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// Arrivals before this wave's (one atomic, by lane 0).
+__device__ __forceinline__ unsigned part_arrive(unsigned* p, int lane) {
+  unsigned before = 0;
+  if (lane == 0) before = atomicAdd(p, 1u);
+  return (unsigned) __builtin_amdgcn_readfirstlane((int) before);
+}
+
+// The nsl slices' partial sums at p added in replica 0: replica q takes slices
+// q, q + m, ...
+__device__ __forceinline__ void part_gather(const double* p, long nsl, int lane, int W, int m, int q, bool act,
+                                            double ps[6], double& maxd, double& an) {
+#pragma unroll
+  for (int c = 0; c < 6; ++c) ps[c] = 0;
+  maxd = an = 0;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  const double* pg = p + (act ? lane - q * W : 0);
+  for (long s = act ? q : nsl; s < nsl; s += 4L * m) {
+    double v[4][8];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const long t = s + (long) u * m;
+      const double* ps_t = pg + 8 * 64 * (t < nsl ? t : s);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) v[u][c] = ps_t[64 * c];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (s + (long) u * m >= nsl) continue;
+#pragma unroll
+      for (int c = 0; c < 6; ++c) ps[c] += v[u][c];
+      maxd = fmax(maxd, v[u][6]);
+      an += v[u][7];
+    }
+  }
+  add_replicas(ps, maxd, an, lane, W, m, q, act);
+}
+
 // Mixed path: bound of the error the reduced-accuracy sin/cos (sincos_fast64)
 // puts into a level's stop decision.  Its cos/sin of the exactly reduced phase
 // are within OM_SINCOS_FAST_ERR of the exact values (the polynomials' largest

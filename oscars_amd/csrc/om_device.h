@@ -163,4 +163,90 @@ __device__ __forceinline__ void sincos_fast64(double phi, double* s, double* c) 
   *c = __longlong_as_double(__double_as_longlong(cr) ^ (long long) sg);
 }
 
+// sin/cos of N phases side by side, step by step: the operations of
+// sincos_fast64 (FAST) or sincos_huge64 on each.
+template <bool FAST, int N>
+__device__ __forceinline__ void sincos_n(const double* phi, double* s, double* c) {
+  double r[N], u[N], ps[N], pc[N];
+  unsigned q[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const double kk = __builtin_fma(phi[i], FAST ? kOneOverPi : kTwoOverPi, kRoundMagic);
+    q[i] = (unsigned) (uint32_t) __double_as_longlong(kk);
+    r[i] = kk - kRoundMagic;
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const double k = r[i];
+    r[i] = __builtin_fma(-k, FAST ? kPiHi : kPio2Hi, phi[i]);
+    r[i] = __builtin_fma(-k, FAST ? kPiLo : kPio2Lo, r[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) u[i] = r[i] * r[i];
+  if (FAST) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      ps[i] = __builtin_fma(u[i], OM_SF_3, OM_SF_2);
+      pc[i] = __builtin_fma(u[i], OM_QF_4, OM_QF_3);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      ps[i] = __builtin_fma(u[i], ps[i], OM_SF_1);
+      pc[i] = __builtin_fma(u[i], pc[i], OM_QF_2);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      ps[i] = __builtin_fma(u[i], ps[i], OM_SF_0);
+      pc[i] = __builtin_fma(u[i], pc[i], OM_QF_1);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      ps[i] = __builtin_fma(r[i] * u[i], ps[i], r[i]);
+      pc[i] = __builtin_fma(u[i], pc[i], OM_QF_0);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      pc[i] = __builtin_fma(u[i], pc[i], 1.0);
+      const unsigned long long sg = (unsigned long long) (q[i] << 31) << 32;
+      s[i] = __longlong_as_double(__double_as_longlong(ps[i]) ^ (long long) sg);
+      c[i] = __longlong_as_double(__double_as_longlong(pc[i]) ^ (long long) sg);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      ps[i] = __builtin_fma(u[i], OM_S64_5, OM_S64_4);
+      pc[i] = __builtin_fma(u[i], OM_C64_5, OM_C64_4);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      ps[i] = __builtin_fma(u[i], ps[i], OM_S64_3);
+      pc[i] = __builtin_fma(u[i], pc[i], OM_C64_3);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      ps[i] = __builtin_fma(u[i], ps[i], OM_S64_2);
+      pc[i] = __builtin_fma(u[i], pc[i], OM_C64_2);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      ps[i] = __builtin_fma(u[i], ps[i], OM_S64_1);
+      pc[i] = __builtin_fma(u[i], pc[i], OM_C64_1);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      ps[i] = __builtin_fma(u[i], ps[i], OM_S64_0);
+      pc[i] = __builtin_fma(u[i], pc[i], OM_C64_0);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const double sr = __builtin_fma(r[i] * u[i], ps[i], r[i]);
+      const double cr = __builtin_fma(u[i] * u[i], pc[i], __builtin_fma(-0.5, u[i], 1.0));
+      const double ss = (q[i] & 1) ? cr : sr;
+      const double cc = (q[i] & 1) ? sr : cr;
+      s[i] = (q[i] & 2) ? -ss : ss;
+      c[i] = ((q[i] + 1) & 2) ? -cc : cc;
+    }
+  }
+}
+
 }  // namespace om

@@ -602,11 +602,35 @@ __global__ void __launch_bounds__(256) level_kernel(LevelJob J) {
   for (int c = 0; c < 9; ++c) o[1 + c] = v[c];
 }
 
-// Largest |beta_i - beta_{i-1}| over one level (src/OSCARSSR.cc:2884-2890);
-// it does not depend on the observation point, so it is computed once per level.
-__global__ void __launch_bounds__(256) beta_diff_kernel(const double* __restrict__ rows, long npts,
+// Levels 0..Lb in one launch (2^(Lb+1) - 1 samples; one launch a level left
+// most of a call's launches to levels of a few samples).
+__global__ void __launch_bounds__(256) levels_kernel(LevelsJob J) {
+  const long g = (long) blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= (2L << J.Lb) - 1) return;
+  const int L = 63 - __clzll((unsigned long long) (g + 1));
+  const double p2L = (double) (1L << L);
+  const double span = J.tstop - J.tstart;
+  // src/TParticleTrajectoryInterpolated.cc:138-147, 264-270 and
+  // src/TParticleTrajectoryInterpolatedPoints.cc:33-37
+  const double spacing = L > J.stop_mem ? span / (p2L - 1) : span / p2L;
+  const double tt = J.tstart + span / (2.0 * p2L) + spacing * (double) (g - ((1L << L) - 1));
+  double v[9];
+  spline_value(J.t + J.knot_offset, J.p + 9 * J.knot_offset, J.ypp + 9 * J.knot_offset, J.n, tt, v);
+  double* o = J.out + 10 * g;
+  o[0] = tt;
+#pragma unroll
+  for (int c = 0; c < 9; ++c) o[1 + c] = v[c];
+}
+
+// Largest |beta_i - beta_{i-1}| over a level (src/OSCARSSR.cc:2884-2890); it
+// does not depend on the observation point, so it is computed once per level:
+// workgroup b takes level L0 + b, at rows + 10 (2^(L0+b) - 2^L0).
+__global__ void __launch_bounds__(256) beta_diff_kernel(const double* __restrict__ rows0, int L0,
                                                         double* __restrict__ out) {
   __shared__ double red[256];
+  const int L = L0 + blockIdx.x;
+  const long npts = 1L << L;
+  const double* rows = rows0 + 10 * (npts - (1L << L0));
   double m = -1;
   for (long i = 1 + threadIdx.x; i < npts; i += blockDim.x) {
     const double* a = rows + 10 * i + 4;
@@ -621,7 +645,7 @@ __global__ void __launch_bounds__(256) beta_diff_kernel(const double* __restrict
     if ((int) threadIdx.x < s) red[threadIdx.x] = red[threadIdx.x + s] > red[threadIdx.x] ? red[threadIdx.x + s] : red[threadIdx.x];
     __syncthreads();
   }
-  if (threadIdx.x == 0) *out = red[0];
+  if (threadIdx.x == 0) out[L] = red[0];
 }
 
 }  // namespace om
@@ -719,7 +743,14 @@ extern "C" hipError_t om_launch_level(const om::LevelJob* J, hipStream_t s) {
   return hipGetLastError();
 }
 
-extern "C" hipError_t om_launch_beta_diff(const double* rows, long npts, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(om::beta_diff_kernel, dim3(1), dim3(256), 0, s, rows, npts, out);
+extern "C" hipError_t om_launch_levels(const om::LevelsJob* J, hipStream_t s) {
+  long blocks = ((2L << J->Lb) - 1 + 255) / 256;
+  hipLaunchKernelGGL(om::levels_kernel, dim3((unsigned) blocks), dim3(256), 0, s, *J);
+  return hipGetLastError();
+}
+
+// Levels L0 .. L0 + n - 1, consecutive in memory from rows; out[L] per level.
+extern "C" hipError_t om_launch_beta_diff(const double* rows, int L0, int n, double* out, hipStream_t s) {
+  hipLaunchKernelGGL(om::beta_diff_kernel, dim3((unsigned) n), dim3(256), 0, s, rows, L0, out);
   return hipGetLastError();
 }

@@ -159,3 +159,30 @@ def test_batch_levels_handed_over(mode):
     assert out[27][1]["evals"] == out[9][1]["evals"] > 323 * 3 * (2 ** 11 - 1)
     for a, c in zip(out[9][0], out[27][0]):
         assert rel_err(a, c, 1e-6) < (1e-11 if mode == "tiled" else 1e-6)
+
+
+@gpu
+@pytest.mark.parametrize("mode,tol", [("tiled", 1e-9), ("mixed", 1e-5), ("plain", 1e-9), ("point_mixed", 1e-5)])
+@pytest.mark.parametrize("shape", [(1, 1), (1, 63), (1, 64), (1, 65), (3, 130), (41, 3), (512, 65), (1025, 64),
+                                   (16384, 1), (16385, 1)])
+def test_flux_request_shapes(epu_pair, mode, tol, shape):
+    """Requests on both sides of the rules that choose the kernels (1024 groups of
+    one observation point and 64 energies; 16384 points), with groups of 1, 63,
+    64, 64 + 1 energies.  Three observation points against the plain path's values
+    in a call of their own, levels identical, and against the oracle (1e-9 in FP64; 1e-5 mixed, whose sines and cosines carry
+    4.8e-9)."""
+    o, dev = epu_pair
+    n_obs, n_e = shape
+    obs = _scatter(n_obs, 0.002, 20.0, seed=n_obs)
+    e = np.linspace(120.0, 700.0, n_e)
+    conv = dev.conv(precision=5e-3, mode=mode)
+    v, lev, cv, _, st = dev.flux(0, obs, e, [0.0] * 6, conv)
+    assert cv.all() and st["n_unconverged"] == 0
+    k = np.unique(np.array([0, n_obs // 2, n_obs - 1]))
+    pv, plev, _, _, _ = dev.flux(0, obs[k], e, [0.0] * 6, dev.conv(precision=5e-3, mode="plain"))
+    v, lev = v.reshape(n_obs, n_e)[k], lev.reshape(n_obs, n_e)[k]
+    assert np.array_equal(lev.ravel(), plev) and rel_err(v.ravel(), pv, 1e-6) < tol
+    je = np.unique(np.array([0, n_e // 2, n_e - 1]))
+    for j in je:
+        ov, olev, _, _ = o.flux_points(obs[k], float(e[j]), precision=5e-3, carry_quirk=False)
+        assert np.array_equal(lev[:, j], olev) and rel_err(v[:, j], ov, 1e-6) < tol
