@@ -735,6 +735,9 @@ struct Timer {
   }
 };
 
+// Results of at most this many bytes come back through pinned memory.
+constexpr size_t kPinnedBack = (size_t) 4 << 20;
+
 // Finalize kernel into the caller's buffers: host pointers (copied back) or,
 // with dev_io, device pointers written in place.  Statistics are reduced on
 // the device.
@@ -769,19 +772,41 @@ void finish_outputs(om_context* ctx, om::FinArgs& F, long npts, double* out_valu
   unsigned long long st3[3] = {0, 0, 0};
   unsigned long long* d_stats = stats ? scratch_buf(ctx->d_stats, 3, ar) : nullptr;
   if (stats) check(om_launch_level_stats(F.out_level, F.out_conv, npts, d_stats, ctx->stream), "level stats");
+  // host outputs: what goes back, through pinned memory where it is small (a
+  // copy into pageable memory is 40 us and a wait of its own: three of them
+  // were a sixth of a call of a few hundred points)
+  struct Back {
+    void* dst;
+    const void* src;
+    size_t bytes;
+  } back[5];
+  int n_back = 0;
+  size_t total = 0;
+  auto add = [&](void* dst, const void* src, size_t bytes) {
+    if (!dst) return;
+    back[n_back++] = {dst, src, bytes};
+    total += (bytes + 15) & ~(size_t) 15;
+  };
   if (!dev_io) {
-    check(hipMemcpyAsync(out_value, ctx->d_out.p, npts * sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
-          "out");
-    if (out_level)
-      check(hipMemcpyAsync(out_level, ctx->d_outlevel.p, npts * sizeof(int), hipMemcpyDeviceToHost, ctx->stream),
-            "lev");
-    if (out_conv) check(hipMemcpyAsync(out_conv, ctx->d_outconv.p, npts, hipMemcpyDeviceToHost, ctx->stream), "conv");
-    if (out_e)
-      check(hipMemcpyAsync(out_e, ctx->d_oute.p, 6 * npts * sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
-            "efield");
+    add(out_value, ctx->d_out.p, npts * sizeof(double));
+    add(out_level, ctx->d_outlevel.p, npts * sizeof(int));
+    add(out_conv, ctx->d_outconv.p, npts);
+    add(out_e, ctx->d_oute.p, 6 * npts * sizeof(double));
   }
-  if (stats) read_back(ctx, st3, d_stats, sizeof(st3));  // also waits for the copies above
-  else check(hipStreamSynchronize(ctx->stream), "sync");
+  if (stats) add(st3, d_stats, sizeof(st3));
+  char* pin = !g_no_alloc && total <= kPinnedBack ? static_cast<char*>(ctx->stage_rb.get(total)) : nullptr;
+  size_t at = 0;
+  for (int i = 0; i < n_back; ++i) {
+    check(hipMemcpyAsync(pin ? pin + at : back[i].dst, back[i].src, back[i].bytes, hipMemcpyDeviceToHost, ctx->stream),
+          "results");
+    at += (back[i].bytes + 15) & ~(size_t) 15;
+  }
+  check(hipStreamSynchronize(ctx->stream), "sync");
+  at = 0;
+  for (int i = 0; pin && i < n_back; ++i) {
+    std::memcpy(back[i].dst, pin + at, back[i].bytes);
+    at += (back[i].bytes + 15) & ~(size_t) 15;
+  }
   if (stats) {
     stats->evals = (double) st3[0];
     stats->max_level = (int) st3[1] - 1;

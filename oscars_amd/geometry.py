@@ -1,7 +1,8 @@
 """Host-side geometry and particle set-up for the drop-in ``sr`` class.
 
-Everything here is scalar IEEE-754 double arithmetic written in the
-reference's operation order, with ``math`` (the C library's sin/cos/sqrt), so
+Everything here is IEEE-754 double arithmetic written in the reference's
+operation order (scalar, but for the points of a surface, whose coordinates are
+formed an operation at a time for all points), with ``math`` (the C library's sin/cos/sqrt), so
 observation points, energies, polarization vectors and initial particle
 conditions are bit-identical to what the reference computes before it calls
 its integrand.  Reference files restated (paths relative to the reference root):
@@ -17,6 +18,8 @@ its integrand.  Reference files restated (paths relative to the reference root):
 import ctypes
 import ctypes.util
 import math
+
+import numpy as np
 
 PI = 3.14159265358979323846
 C = 2.99792458e8
@@ -159,7 +162,27 @@ def ideal_particle(ptype, energy_GeV, x0, d0, t0=0.0, current=0.0, charge=0.0, m
     return p
 
 
-def rectangle(plane, n1, n2, w1, w2, rotations=(0, 0, 0), translation=(0, 0, 0), normal=0, dim=2):
+def _lattice(x0, a1, a2, n1, n2, s1, s2, dim):
+    """Points x0 + a1 i + a2 j, j fastest, and the coordinates stored with them:
+    the points (dim 3), or s1 i and s2 j from the middle (dim 2)."""
+    i, j = np.repeat(np.arange(n1, dtype=np.float64), n2), np.tile(np.arange(n2, dtype=np.float64), n1)
+    obs = np.stack([x0[k] + a1[k] * i + a2[k] * j for k in range(3)], axis=1)
+    if dim != 2:
+        return obs, obs.copy()
+    m1, m2 = math.sqrt(mag2(a1)), math.sqrt(mag2(a2))
+    cont = np.zeros((n1 * n2, 3))
+    cont[:, 0] = s1 * i - m1 * (n1 - 1) / 2.
+    cont[:, 1] = s2 * j - m2 * (n2 - 1) / 2.
+    return obs, cont
+
+
+def rectangle(*args, **kw):
+    """``rectangle_arrays`` with the points and coordinates as lists."""
+    obs, nv, cont = rectangle_arrays(*args, **kw)
+    return obs.tolist(), nv, cont.tolist()
+
+
+def rectangle_arrays(plane, n1, n2, w1, w2, rotations=(0, 0, 0), translation=(0, 0, 0), normal=0, dim=2):
     """Observation points, the normal and the coordinates the reference stores
     (TSurfacePoints_Rectangle::Init / GetXYZ / GetX1 / GetX2)."""
     P = plane.upper()
@@ -199,23 +222,17 @@ def rectangle(plane, n1, n2, w1, w2, rotations=(0, 0, 0), translation=(0, 0, 0),
         nv = [nv[0] * -1, nv[1] * -1, nv[2] * -1]
     elif normal not in (0, 1):
         raise ValueError("normal must be -1, 0, or 1")
-    m1 = math.sqrt(mag2(a1))
-    m2 = math.sqrt(mag2(a2))
-    obs = []
-    cont = []
-    for i in range(n1 * n2):
-        ix1 = i // n2
-        ix2 = i % n2
-        o = [st[k] + a1[k] * float(ix1) + a2[k] * float(ix2) for k in range(3)]
-        obs.append(o)
-        if dim == 2:
-            cont.append([s1 * ix1 - m1 * (n1 - 1) / 2., s2 * ix2 - m2 * (n2 - 1) / 2., 0.0])
-        else:
-            cont.append(o)
+    obs, cont = _lattice(st, a1, a2, n1, n2, s1, s2, dim)
     return obs, nv, cont
 
 
-def parallelogram(n1, n2, x0, x1, x2, rotations=(0, 0, 0), translation=(0, 0, 0), normal=0, dim=2):
+def parallelogram(*args, **kw):
+    """``parallelogram_arrays`` with the points and coordinates as lists."""
+    obs, nv, cont = parallelogram_arrays(*args, **kw)
+    return obs.tolist(), nv, cont.tolist()
+
+
+def parallelogram_arrays(n1, n2, x0, x1, x2, rotations=(0, 0, 0), translation=(0, 0, 0), normal=0, dim=2):
     """Observation points, normal and stored coordinates of a surface given by
     three corners (TSurfacePoints_Rectangle::Init from X0, X1, X2,
     src/TSurfacePoints_Rectangle.cc:76-123; the binding rotates, then
@@ -237,16 +254,7 @@ def parallelogram(n1, n2, x0, x1, x2, rotations=(0, 0, 0), translation=(0, 0, 0)
     elif normal not in (0, 1):
         raise ValueError("fNormal is of the incorrect form.  Must be -1, 0, 1")
     nv = unit(nv)  # each surface point normalises its normal again (src/TSurfacePoint.cc:16)
-    m1, m2 = math.sqrt(mag2(a1)), math.sqrt(mag2(a2))
-    obs, cont = [], []
-    for i in range(n1 * n2):
-        ix1, ix2 = i // n2, i % n2
-        o = [X0[k] + a1[k] * float(ix1) + a2[k] * float(ix2) for k in range(3)]
-        obs.append(o)
-        if dim == 2:
-            cont.append([s1 * ix1 - m1 * (n1 - 1) / 2., s2 * ix2 - m2 * (n2 - 1) / 2., 0.0])
-        else:
-            cont.append(o)
+    obs, cont = _lattice(X0, a1, a2, n1, n2, s1, s2, dim)
     return obs, nv, cont
 
 

@@ -908,7 +908,7 @@ class sr:
             IO.write_spectrum_text(ofile, e, v)
         if bofile != "":
             IO.write_spectrum_binary(bofile, e, v)
-        return [[e[i], float(v[i])] for i in range(len(e))]
+        return [[c, x] for c, x in zip(e, v.tolist())]
 
     # ------------------------------------------------------------ flux
     def _rect(self, npoints, plane, width, rotations, translation, normal, dim, x0x1x2):
@@ -930,10 +930,10 @@ class sr:
             X = [_v3(x, "x0x1x2") for x in x0x1x2]
             if n1 < 2 or n2 < 2:
                 raise ValueError("'npoints' must be >= 2 in each direction for 'x0x1x2'")
-            return G.parallelogram(n1, n2, X[0], X[1], X[2], rot, tr, normal, dim)
+            return G.parallelogram_arrays(n1, n2, X[0], X[1], X[2], rot, tr, normal, dim)
         if width is None or len(width) != 2 or not (width[0] > 0 and width[1] > 0):
             raise ValueError("must specify 'width' (positive only)")
-        return G.rectangle(plane, n1, n2, float(width[0]), float(width[1]), rot, tr, normal, dim)
+        return G.rectangle_arrays(plane, n1, n2, float(width[0]), float(width[1]), rot, tr, normal, dim)
 
     def calculate_flux_rectangle(self, energy_eV, npoints=None, plane="XY", normal=0, dim=2, width=None,
                                  rotations=None, translation=None, x0x1x2=None, polarization="", angle=_NOANGLE,
@@ -943,12 +943,11 @@ class sr:
         if self._beam is None:
             raise ValueError("No particle beam defined")
         self._check_common(nparticles, nthreads, 0 if gpu == 0 else gpu)
-        obs, nv, cont = self._rect(npoints, plane, width, rotations, translation, normal, dim, x0x1x2)
+        obs_a, nv, cont = self._rect(npoints, plane, width, rotations, translation, normal, dim, x0x1x2)
         hdir = _v3(horizontal_direction, "translation") if horizontal_direction else [1.0, 0.0, 0.0]
         pdir = _v3(propogation_direction, "translation") if propogation_direction else [0.0, 0.0, 1.0]
         q = self._quantity(quantity)
         pol = self._polarization(polarization, angle, hdir, pdir)
-        obs_a = np.array(obs)
 
         def run(dev, ip, w, acc, out=None):
             conv = dev.conv(precision, max_level, max_level_extended, q, mode, w, acc)
@@ -962,11 +961,12 @@ class sr:
         if not self._last_conv.all():
             _warn("Not all points converged to desired precision.  Can try increasing 'max_level_extended'\n")
         # src/OSCARSSR_Python.cc:8310-8318: the container's points (local x1, x2 for dim 2)
+        cont = cont.tolist()
         if ofile != "":
             IO.write_points_text(ofile, cont, v, dim)
         if bofile != "":
             IO.write_points_binary(bofile, cont, v, dim)
-        return [[list(cont[i]), float(v[i])] for i in range(len(cont))]
+        return [[c, x] for c, x in zip(cont, v.tolist())]
 
     def calculate_flux_rectangle_energies(self, energies_eV, npoints=None, plane="XY", normal=0, dim=2, width=None,
                                           rotations=None, translation=None, polarization="", angle=_NOANGLE,
@@ -977,12 +977,11 @@ class sr:
         Returns (coords[n_obs, 3], flux[n_obs, n_energies])."""
         if self._beam is None:
             raise ValueError("No particle beam defined")
-        obs, nv, cont = self._rect(npoints, plane, width, rotations, translation, normal, dim, None)
+        obs_a, nv, cont = self._rect(npoints, plane, width, rotations, translation, normal, dim, None)
         hdir = _v3(horizontal_direction, "translation") if horizontal_direction else [1.0, 0.0, 0.0]
         pdir = _v3(propogation_direction, "translation") if propogation_direction else [0.0, 0.0, 1.0]
         q = self._quantity(quantity)
         pol = self._polarization(polarization, angle, hdir, pdir)
-        obs_a = np.array(obs)
         e = np.ascontiguousarray(energies_eV, dtype=np.float64)
 
         def run(dev, ip, w, acc, out=None):
@@ -997,7 +996,7 @@ class sr:
             v = self._batched(nparticles, obs_a, e, pol, precision, max_level, max_level_extended, mode)
         else:
             v = self._run_particles(nparticles, run)
-        return np.array(cont), v.reshape(len(obs), len(e))
+        return cont, v.reshape(len(obs_a), len(e))
 
     # ------------------------------------------------------------ power density
     def calculate_power_density_rectangle(self, npoints=None, plane="XY", normal=0, width=None, rotations=None,
@@ -1017,10 +1016,9 @@ class sr:
         if width is None:
             width = [0.010, 0.010]
         self._check_common(nparticles, nthreads, 0 if gpu == 0 else gpu)
-        obs, nv, cont = self._rect(npoints, plane, width, rotations, translation, normal, dim, x0x1x2)
+        obs_a, nv, cont = self._rect(npoints, plane, width, rotations, translation, normal, dim, x0x1x2)
         q = self._quantity(quantity, pd=True)
         directional = normal != 0
-        obs_a = np.array(obs)
 
         def run(dev, ip, w, acc, out=None):
             conv = dev.conv(precision, max_level, max_level_extended, q, mode, w, acc)
@@ -1034,11 +1032,12 @@ class sr:
         if not self._last_conv.all():
             _warn("Not all points converged to desired precision.  Can try increasing 'max_level_extended'\n")
         # src/OSCARSSR_Python.cc:6755-6763
+        cont = cont.tolist()
         if ofile != "":
             IO.write_points_text(ofile, cont, v, dim)
         if bofile != "":
             IO.write_points_binary(bofile, cont, v, dim)
-        return [[list(cont[i]), float(v[i])] for i in range(len(cont))]
+        return [[c, x] for c, x in zip(cont, v.tolist())]
 
     def _pd_points(self, obs, normals, directional, nparticles, precision, max_level, max_level_extended, q,
                    mode="plain"):
@@ -1163,8 +1162,7 @@ class sr:
         v = self._run_particles(nparticles, run)
         if stlofile != "":
             IO.write_stl(stlofile, tri, np.concatenate([[s] * len(t) for _, t, s in self._stl]))
-        return [[[tri[i, 0:3].tolist(), tri[i, 3:6].tolist(), tri[i, 6:9].tolist()], float(v[i])]
-                for i in range(len(tri))]
+        return [[c, x] for c, x in zip(tri[:, :9].reshape(-1, 3, 3).tolist(), v.tolist())]
 
     def calculate_efield_vs_time(self, obs, ofile=""):
         """Electric field in the time domain at obs: [[t, [Ex, Ey, Ez]], ...],
