@@ -1007,22 +1007,25 @@ int lw_sums(om_context* ctx, int ip, const double* obs_xyz, long n_obs, const do
     long n_recheck = 0;
     int Ldone = 0;  // deepest level summed so far (its samples exist)
     const int block = ar && !(sliced || waves) ? kListFrom - 1 : kBlockLevel;
+    om::SliceArgs X;
+    std::memset(&X, 0, sizeof(X));
+    if (sliced) {
+      X.n_groups = n_obs * blocks_e;
+      X.blocks_e = blocks_e;
+      X.part = scratch_buf(ctx->d_part, (size_t) om::kSliceJobs * 8 * 64, ar);
+      const bool fresh = ar || !ctx->d_arrived.p;  // zero between launches
+      X.arrived = scratch_buf(ctx->d_arrived, kSliceGroups, ar);
+      if (fresh)
+        check(om_launch_adj_key_fill(reinterpret_cast<int*>(X.arrived), kSliceGroups, 0, ctx->stream), "clear");
+    }
     while (true) {
       ensure_levels(ctx, ip, Lb, stop_mem, lc, ar, block);
       fill_levels(ctx, ip, Lb, A.lv, lc);
       A.La = La;
       A.Lb = Lb;
       if (!ar) ctx->timer.begin(ctx->stream);
-      if (sliced && La == 0) {
-        om::SliceArgs X;
-        X.n_groups = n_obs * blocks_e;
-        X.blocks_e = blocks_e;
-        X.part = scratch_buf(ctx->d_part, (size_t) om::kSliceJobs * 8 * 64, ar);
-        const bool fresh = ar || !ctx->d_arrived.p;  // zero between launches
-        X.arrived = scratch_buf(ctx->d_arrived, kSliceGroups, ar);
-        if (fresh)
-          check(om_launch_adj_key_fill(reinterpret_cast<int*>(X.arrived), kSliceGroups, 0, ctx->stream), "clear");
-        for (int L = kListFrom - 1; L <= Lb; ++L) {
+      if (sliced) {
+        for (int L = std::max(La, kListFrom - 1); L <= Lb; ++L) {
           const long most = L < kListFrom ? 8 : (1L << L) / om::kSliceMin;
           X.L = L;
           X.nsl = (int) std::max(1L, std::min(most, om::kSliceJobs / X.n_groups));

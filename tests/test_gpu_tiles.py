@@ -186,3 +186,21 @@ def test_flux_request_shapes(epu_pair, mode, tol, shape):
     for j in je:
         ov, olev, _, _ = o.flux_points(obs[k], float(e[j]), precision=5e-3, carry_quirk=False)
         assert np.array_equal(lev[:, j], olev) and rel_err(v[:, j], ov, 1e-6) < tol
+
+
+@gpu
+@pytest.mark.parametrize("mode,tol", [("tiled", 1e-9), ("mixed", 1e-5)])
+@pytest.mark.parametrize("shape", [(1, 65), (5, 3)])
+def test_flux_deep_levels(epu_pair, mode, tol, shape):
+    """Small requests whose energies stop at levels 9 to 15, through the levels
+    the host looks between: against the plain path's values (tolerances as
+    above), levels identical."""
+    o, dev = epu_pair
+    n_obs, n_e = shape
+    obs = _scatter(n_obs, 0.002, 20.0, seed=n_obs)
+    e = np.linspace(400.0, 6000.0, n_e)
+    kw = dict(precision=1e-6, max_level=15, max_level_extended=15)
+    v, lev, cv, _, _ = dev.flux(0, obs, e, [0.0] * 6, dev.conv(mode=mode, **kw))
+    pv, plev, pcv, _, _ = dev.flux(0, obs, e, [0.0] * 6, dev.conv(mode="plain", **kw))
+    assert np.array_equal(lev, plev) and np.array_equal(cv, pcv) and lev.max() >= 14
+    assert rel_err(v, pv, 1e-6) < tol
