@@ -234,6 +234,12 @@ struct LaunchTimer {
 // launch (1.3 MB); deeper ones have buffers of their own.
 constexpr int kBlockLevel = 13;
 
+// The reverse pass goes through the RK4 steps in at most this many segments
+// (eight lanes each in the map kernel: one workgroup per CU), of at least 4
+// steps.  20000 steps: maps, chain and reverse sweep 172 us; in ceil(sqrt(n)) =
+// 142 segments, which also bounded the storage, 1477 us.
+constexpr long kAdjSegments = 2048;
+
 struct LevelCache {
   double* rows[om::kMaxLevel + 1] = {};  // device buffers, kept across trajectory sets
   bool built[om::kMaxLevel + 1] = {};    // rows hold samples of the current trajectory
@@ -911,7 +917,7 @@ void launch_trajectories(om_context* ctx, int np) {
     // states every K steps of particle 0, taken from the raw knots before the division by c
     auto& A = ctx->adj;
     A.nf = ctx->desc[0].nf;
-    A.K = (long) std::ceil(std::sqrt((double) A.nf));
+    A.K = std::max(4L, (A.nf + kAdjSegments - 1) / kAdjSegments);
     A.nseg = (A.nf + A.K - 1) / A.K;
     A.ckpt.ensure(6 * A.nseg);
     check(om_launch_adj_ckpt(ctx->d_p.p + 9 * ctx->desc[0].knot_offset, A.K, A.nseg, A.ckpt.p, ctx->stream),
@@ -2366,17 +2372,27 @@ int adjoint_backward(om_context* ctx, const double* dloss_dflux, double* grad_fi
     int stop_mem = A.L;
     ensure_levels(ctx, 0, A.L, stop_mem);
     long ns = (2L << A.L) - 1;
-    A.rows.ensure(10 * ns);
-    for (int L = 0; L <= A.L; ++L)
-      check(hipMemcpyAsync(A.rows.p + 10 * ((1L << L) - 1), ctx->levels[0].rows[L], (1L << L) * 10 * sizeof(double),
-                           hipMemcpyDeviceToDevice, ctx->stream), "rows");
+    // the block of levels is one after the other already
+    const double* rows = ctx->levels[0].rows[0];
+    if (A.L > ctx->levels[0].block) {
+      A.rows.ensure(10 * ns);
+      const int block = ctx->levels[0].block;
+      for (int L = block; L <= A.L; ++L) {
+        const long n = L == block ? (2L << L) - 1 : 1L << L;
+        check(hipMemcpyAsync(A.rows.p + (L == block ? 0 : 10 * ((1L << L) - 1)),
+                             ctx->levels[0].rows[L == block ? 0 : L], n * 10 * sizeof(double),
+                             hipMemcpyDeviceToDevice, ctx->stream), "rows");
+      }
+      rows = A.rows.p;
+    }
     hipEvent_t e0 = ctx->ev0, e1 = ctx->ev1;
     check(hipEventRecord(e0, ctx->stream), "event");
     // 1. LW sum: dLoss/d(sample x, beta, a/c)
     int cus = 0;
     check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device), "attribute");
-    long target = (long) cus * 8 * 64;  // about 8 waves per CU
-    long nchunks = (target + ns - 1) / ns;
+    // workgroups of 256 samples by chunks of points: as many as are resident at
+    // once, three per CU (165 registers)
+    long nchunks = 3L * cus / ((ns + 255) / 256);
     if (nchunks > A.n_obs) nchunks = A.n_obs;
     if (nchunks < 1) nchunks = 1;
     long per = (A.n_obs + nchunks - 1) / nchunks;
@@ -2384,7 +2400,7 @@ int adjoint_backward(om_context* ctx, const double* dloss_dflux, double* grad_fi
     A.partial.ensure(9 * ns * nchunks);
     A.sb.ensure(9 * ns);
     om::AdjLwArgs L;
-    L.rows = A.rows.p;
+    L.rows = rows;
     L.ns = ns;
     L.obs = A.obs.p;
     L.n_obs = A.n_obs;
@@ -2406,7 +2422,7 @@ int adjoint_backward(om_context* ctx, const double* dloss_dflux, double* grad_fi
     A.ub.ensure(9 * n);
     A.cc.ensure(9 * n);
     const double* X = ctx->d_t.p + D.knot_offset;
-    check(om_launch_adj_spline(A.rows.p, ns, A.sb.p, A.L, X, n, A.klo.p, A.yb.p, A.yppb.p, A.Pw.p, A.ppw.p, A.sgw.p,
+    check(om_launch_adj_spline(rows, ns, A.sb.p, A.L, X, n, A.klo.p, A.yb.p, A.yppb.p, A.Pw.p, A.ppw.p, A.sgw.p,
                                A.ub.p, A.cc.p, ctx->stream), "adjoint spline");
     // 3. RK4 with checkpoints: dLoss/d(initial state), dLoss/d(grid samples)
     A.segmap.ensure(42 * A.nseg);
