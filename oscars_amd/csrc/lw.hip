@@ -697,22 +697,26 @@ __global__ void __launch_bounds__(64) pd_wave_kernel(PdArgs A) {
 }
 
 // ---------------------------------------------------------------- power density on STL triangles
-// src/OSCARSSR.cc:3318-3527.  One wave per triangle centre; its lanes take 64
-// consecutive samples of a level at a time.  Each lane asks whether any other
+// src/OSCARSSR.cc:3318-3527.  One workgroup per triangle centre, a quarter of a
+// level's samples per wave, 64 at a time.  Each lane asks whether any other
 // triangle lies between its sample and the centre (src/TTriangle3D.cc:159-215,
 // Moller and Trumbore, same operations), walking a bounding-volume hierarchy
 // whose boxes are inflated by more than the test's rounding can move an
 // accepted intersection, so it finds a hit exactly when the test of every
 // triangle would.  Unblocked samples add the power density integrand with
 // |N1 . normal| and move the beta-step maximum, the step taken from the last
-// unblocked sample before (the lane's ballot gives it), as in the reference;
-// the 64 terms are added by a butterfly in a fixed order.
+// unblocked sample before (the lane's ballot gives it; across the waves' parts
+// from what each part's first and last unblocked samples were), as in the
+// reference; the terms are added in a fixed order.
+// Bound by the latency of the walk: the rays of 64 neighbouring samples meet
+// much the same boxes, so the lanes walk together (a node is a scalar load, and
+// is entered when any lane's ray meets it), and four waves per triangle keep a
+// SIMD busy where meshes have a few thousand triangles.  1280 triangles of a
+// sphere: one wave per triangle, each lane at a node of its own, 1075 us; 274 us.
 constexpr int kStlWaves = 4;
 
-__device__ __forceinline__ bool stl_blocks(const double* __restrict__ T, V3 O, V3 D, double dist) {
-  // T: A, edge1, edge2 of one triangle; D: the unit ray direction, normalised again
-  double m = sqrt(mag2(D));
-  V3 R = v3(D.x / m, D.y / m, D.z / m);
+__device__ __forceinline__ bool stl_blocks(const double* __restrict__ T, V3 O, V3 R, double dist) {
+  // T: A, edge1, edge2 of one triangle; R: the ray direction
   V3 A = v3(T[0], T[1], T[2]), e1 = v3(T[3], T[4], T[5]), e2 = v3(T[6], T[7], T[8]);
   V3 p = cross(R, e2);
   double det = dot(e1, p);
@@ -747,29 +751,37 @@ __device__ __forceinline__ bool stl_box_hit(const double* __restrict__ b, V3 X, 
 }
 
 // Any triangle other than `self` between X and the point at distance dist
-// along the unit direction N1.
-__device__ __forceinline__ bool stl_any_hit(const StlArgs& A, V3 X, V3 N1, double dist, long self) {
+// along the unit direction N1.  All lanes of the wave walk together, `want`
+// those with a ray.
+__device__ __forceinline__ bool stl_any_hit(const StlArgs& A, V3 X, V3 N1, double dist, int self, bool want) {
   V3 inv = v3(1.0 / N1.x, 1.0 / N1.y, 1.0 / N1.z);
+  double m = sqrt(mag2(N1));
+  V3 R = v3(N1.x / m, N1.y / m, N1.z / m);  // normalised again, as the reference does
+  bool hit = false;
   int i = 0;
   while (i < A.bvh_nodes) {
-    const int* m = A.bvh_meta + 3 * i;
-    int next = m[0];
-    if (!stl_box_hit(A.bvh_box + 6 * i, X, N1, inv, -A.pad_t, dist + A.pad_t)) {
+    const int* n = A.bvh_meta + 3 * i;
+    const int next = __builtin_amdgcn_readfirstlane(n[0]);
+    const bool in = want && stl_box_hit(A.bvh_box + 6 * i, X, N1, inv, -A.pad_t, dist + A.pad_t);
+    if (!__any(in)) {
       i = next;
       continue;
     }
-    int cnt = m[2];
+    const int cnt = __builtin_amdgcn_readfirstlane(n[2]);
     if (cnt == 0) {  // inner node: its first child follows it
       ++i;
       continue;
     }
+    const int first = __builtin_amdgcn_readfirstlane(n[1]);
     for (int k = 0; k < cnt; ++k) {
-      int j = A.bvh_order[m[1] + k];
-      if (j != self && stl_blocks(A.tri + 12 * j, X, N1, dist)) return true;
+      const int j = __builtin_amdgcn_readfirstlane(A.bvh_order[first + k]);
+      if (j != self && in && !hit) hit = stl_blocks(A.tri + 12 * j, X, R, dist);
     }
+    want = want && !hit;
+    if (!__any(want)) break;
     i = next;
   }
-  return false;
+  return hit;
 }
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -783,58 +795,88 @@ __device__ __forceinline__ double wave_max(double v) {
 }
 
 __global__ void __launch_bounds__(64 * kStlWaves) pd_stl_kernel(StlArgs A) {
-  const int lane = threadIdx.x & 63;
-  const long p = (long) blockIdx.x * kStlWaves + (threadIdx.x >> 6);
-  if (p >= A.ntri) return;
+  // per wave, of the level it shares: sum, largest beta step, its first and last
+  // unblocked samples' beta, and what of these there is (double-buffered)
+  __shared__ double part[2][kStlWaves][8];
+  __shared__ int have[2][kStlWaves];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+  const int p = blockIdx.x;
   int lev = A.st.level[p];
-  if (A.st.conv[p] || lev != A.La - 1) return;
-  const V3 obs = v3(A.centre[3 * p], A.centre[3 * p + 1], A.centre[3 * p + 2]);
-  const V3 nrm = v3(A.tri[12 * p + 9], A.tri[12 * p + 10], A.tri[12 * p + 11]);
-  double sum = A.st.sum[6 * p];
+  if (A.st.conv[p] || lev != A.La - 1) return;  // the same for the whole workgroup
+  const V3 obs = v3(A.centre[3L * p], A.centre[3L * p + 1], A.centre[3L * p + 2]);
+  const V3 nrm = v3(A.tri[12L * p + 9], A.tri[12L * p + 10], A.tri[12L * p + 11]);
+  double sum = A.st.sum[6L * p];
   double lastsum = A.st.lastmag[p];
   double prec = A.st.prec[p];
   bool done = false;
-  for (int L = A.La; L <= A.Lb && !done; ++L) {
+  int buf = 0;
+  for (int L = A.La; L <= A.Lb && !done; ++L, buf ^= 1) {
+    // levels 0..8, where nothing is decided, lie one after the other: one sum of
+    // 511 samples
+    const bool first = L == 0 && A.Lb > 8;
     const double* __restrict__ rows = A.lv.rows[L];
-    const long ns = 1L << L;
-    V3 lastB = v3(0, 0, 0);  // the last unblocked sample's beta (none yet: zero)
-    double bdmax = -1;
-    for (long base = 0; base < ns; base += 64) {
+    const long ns = first ? 511 : 1L << L;
+    if (first) L = 8;
+    const long i0 = ns * wv / kStlWaves, i1 = ns * (wv + 1) / kStlWaves;
+    V3 firstB = v3(0, 0, 0), lastB = v3(0, 0, 0);
+    int any = 0;  // bit 0: an unblocked sample, bit 1: its first one is not sample 0
+    double acc = 0, bdmax = -1;
+    for (long base = i0; base < i1; base += 64) {
       const long i = base + lane;
-      const bool valid = i < ns;
-      const double* s = rows + 10 * (valid ? i : 0);
+      const bool valid = i < i1;
+      const double* s = rows + 10 * (valid ? i : i0);
       V3 X = v3(s[1], s[2], s[3]);
       V3 R = sub(obs, X);
       double r2 = mag2(R);
       double dist = sqrt(r2);
       V3 N1 = v3(R.x / dist, R.y / dist, R.z / dist);
-      const bool blocked = !valid || stl_any_hit(A, X, N1, dist, p);
+      const bool blocked = stl_any_hit(A, X, N1, dist, p, valid) || !valid;
       const unsigned long long open = __ballot(!blocked);
+      if (open == 0) continue;
       V3 B = v3(s[4], s[5], s[6]);
       V3 Ac = v3(s[7], s[8], s[9]);
       // the last unblocked sample before this one: in this group, else carried
       const unsigned long long below = lane ? open & ((1ull << lane) - 1) : 0ull;
       const int src = below ? 63 - __clzll(below) : lane;
       V3 pB = v3(__shfl(B.x, src), __shfl(B.y, src), __shfl(B.z, src));
-      V3 prevB = below ? pB : lastB;
-      double term = 0, bd = -1;
+      const int f = __ffsll(open) - 1, l = 63 - __clzll(open);
+      const bool carried = any != 0;  // else this part's first has no step here
+      if (!below) pB = lastB;
+      if (!carried) {
+        firstB = v3(__shfl(B.x, f), __shfl(B.y, f), __shfl(B.z, f));
+        any = base + f > 0 ? 3 : 1;
+      }
       if (!blocked) {
-        V3 dB = sub(B, prevB);
-        bd = i > 0 ? sqrt(mag2(dB)) : -1.0;
+        if (below || carried) bdmax = fmax(bdmax, sqrt(mag2(sub(B, pB))));
         double ndn = fabs(dot(N1, nrm));
         V3 Num = cross(N1, cross(sub(N1, B), Ac));
         double x = 1 - dot(B, N1);
         double x2 = x * x;
         double den = x2 * x2 * x;
         // (Num.N2)^2 + (Num.N3)^2 = |Num|^2 because Num is perpendicular to N1
-        term = mag2(Num) / den / r2 * ndn;
+        acc += mag2(Num) / den / r2 * ndn;
       }
-      sum += wave_sum(term);
-      bdmax = fmax(bdmax, wave_max(bd));
-      if (open) {
-        const int last = 63 - __clzll(open);
-        lastB = v3(__shfl(B.x, last), __shfl(B.y, last), __shfl(B.z, last));
-      }
+      lastB = v3(__shfl(B.x, l), __shfl(B.y, l), __shfl(B.z, l));
+    }
+    acc = wave_sum(acc);
+    bdmax = wave_max(bdmax);
+    if (lane == 0) {
+      double* w = part[buf][wv];
+      w[0] = acc; w[1] = bdmax;
+      w[2] = firstB.x; w[3] = firstB.y; w[4] = firstB.z;
+      w[5] = lastB.x; w[6] = lastB.y; w[7] = lastB.z;
+      have[buf][wv] = any;
+    }
+    __syncthreads();
+    V3 prevB = v3(0, 0, 0);  // none yet: zero
+    bdmax = -1;
+    for (int k = 0; k < kStlWaves; ++k) {
+      const double* w = part[buf][k];
+      sum += w[0];
+      if (!have[buf][k]) continue;
+      bdmax = fmax(bdmax, w[1]);
+      if (have[buf][k] & 2) bdmax = fmax(bdmax, sqrt(mag2(sub(v3(w[2], w[3], w[4]), prevB))));
+      prevB = v3(w[5], w[6], w[7]);
     }
     lev = L;
     double thisSum = sum * A.lv.dt_incl[L];
@@ -846,8 +888,8 @@ __global__ void __launch_bounds__(64 * kStlWaves) pd_stl_kernel(StlArgs A) {
     if (c || c2) done = true;
     else lastsum = thisSum;
   }
-  if (lane == 0) {
-    A.st.sum[6 * p] = sum;
+  if (threadIdx.x == 0) {
+    A.st.sum[6L * p] = sum;
     A.st.lastmag[p] = lastsum;
     A.st.prec[p] = prec;
     A.st.level[p] = lev;
@@ -1373,7 +1415,7 @@ extern "C" hipError_t om_launch_pd_point(const om::PdArgs* A, int mixed, hipStre
 }
 
 extern "C" hipError_t om_launch_pd_stl(const om::StlArgs* A, hipStream_t s) {
-  long blocks = (A->ntri + om::kStlWaves - 1) / om::kStlWaves;
+  long blocks = A->ntri;
   hipLaunchKernelGGL(om::pd_stl_kernel, dim3((unsigned) blocks), dim3(64 * om::kStlWaves), 0, s, *A);
   return hipGetLastError();
 }

@@ -204,3 +204,64 @@ def test_flux_deep_levels(epu_pair, mode, tol, shape):
     pv, plev, pcv, _, _ = dev.flux(0, obs, e, [0.0] * 6, dev.conv(mode="plain", **kw))
     assert np.array_equal(lev, plev) and np.array_equal(cv, pcv) and lev.max() >= 14
     assert rel_err(v, pv, 1e-6) < tol
+
+
+@gpu
+@pytest.mark.parametrize("level", [0, 1, 2, 7, 8, 9, 10])
+def test_power_density_stl_caps(tmp_path, level):
+    """Levels on both sides of the first ones summed as one (0..8), down to
+    levels of fewer samples than the waves that share them: the oracle on the
+    device's own trajectory takes the same occlusion decisions, values to 1e-12
+    (sums of at most 2047 positive terms in another order), and levels where they
+    stopped before the cap."""
+    from oracle.pyoracle import Trajectory
+    from oscars_amd import io as IO
+    from tests.common import stl_scene
+    from tests.test_gpu_power import _pair
+    scene = stl_scene(str(tmp_path))
+    o, s = _pair(planar, 2001)
+    for k, (path, scale, tr) in enumerate(scene):
+        s.add_stl(path, scale=scale, translation=tr, name="s%d" % k)
+    v = np.array([r[1] for r in s.calculate_power_density_stl(max_level=level)])
+    tri = np.concatenate([IO.read_stl(p, sc, t) for p, sc, t in scene])
+    o.traj = Trajectory(*s._device().trajectory(0))
+    ov, olev, oconv = o.power_density_stl(tri, max_level=level, carry_quirk=False)
+    done = np.asarray(oconv, dtype=bool)
+    assert np.array_equal(np.asarray(s._last_conv, dtype=bool), done)
+    assert np.array_equal(s._last_levels[done], olev[done]) and rel_err(v, ov, 1e-6) < 1e-12
+
+
+@gpu
+@pytest.mark.parametrize("npts", [66, 127, 2049, 8194])
+def test_adjoint_segments(npts):
+    """Reverse passes of fewer segments than the chain has groups, of about one
+    a group, and of the most there are (2048) with a short last one: the angle
+    gradients against 4th-order differences of the long-double forward (1e-4, as
+    at 4001 points)."""
+    from oracle.pyoracle import fdref_flux
+    from oscars_amd import _lib
+    from oscars_amd import adjoint as A
+    from oscars_amd import geometry as G
+    n, z0, dz = 1001, -0.4, 8e-4
+    samples = np.zeros((n, 3))
+    z = z0 + dz * np.arange(n)
+    samples[:, 1] = 0.05 * np.sin(2 * np.pi * z / 0.2) * np.exp(-(z / 0.2) ** 2)
+    obs = np.array([[0.001, 0.0005, 30.0], [-0.0007, 0.001, 30.0]])
+    e = np.array([20.0, 31.0])
+    prob = A.FieldMapProblem(_lib.Device(0), [0, 0, z0], [0, 0, dz], [1, 1, n], 3.0, [0, 0, -0.5], 0.0, 1.0, npts, obs,
+                             e, 10)
+    prob.forward(samples, (0.0, 0.0))
+    w = np.array([[1.0, -0.4], [0.7, 0.2]])
+    _, ga, _ = prob.backward(w)
+    p0 = G.ideal_particle("electron", 3.0, [0, 0, -0.5], [0, 0, 1], 0.0, 0.5)
+
+    def loss(ang):
+        b0, _, _ = A.beta0_from_angles(p0.b0, ang[0], ang[1])
+        return float(np.sum(w * fdref_flux(samples, z0, dz, [0, 0, -0.5], b0, 0.5, 0.0, 1.0, npts, obs, e, 10,
+                                           long_double=True)))
+    for k in range(2):
+        def at(d):
+            return loss([d if j == k else 0.0 for j in range(2)])
+        fd = (-at(2e-7) + 8 * at(1e-7) - 8 * at(-1e-7) + at(-2e-7)) / 1.2e-6
+        print("npts %d angle %d: adjoint %.10e differences %.10e" % (npts, k, ga[k], fd))
+        assert abs(ga[k] - fd) < 1e-4 * abs(fd)
