@@ -248,10 +248,13 @@ __global__ void __launch_bounds__(64 * kShootWaves) shoot_kernel(const ShootArgs
         if (lane < 7) {
           shoot_compose(&sWave[0][0], kShootWaves, 42, lane, v);
 #pragma unroll
-          for (int k = 0; k < 6; ++k) Mb[42L * ib + 7 * k + lane] = v[k];
+          for (int k = 0; k < 6; ++k)
+            __hip_atomic_store(Mb + 42L * ib + 7 * k + lane, v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        if (lane == 0) okb[ib] = done ? 1 : 0;
-        __threadfence();
+        if (lane == 0) __hip_atomic_store(okb + ib, done ? 1 : 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // the map and the flag are past the caches before the arrival is; a fence
+        // here would write the knots back from L2 in every round
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (lane == 0) {
           int* cnt = A.arrived + A.block_chain[ib];
           const int target = C.nblock * (round + 1);
@@ -266,7 +269,7 @@ __global__ void __launch_bounds__(64 * kShootWaves) shoot_kernel(const ShootArgs
       }
       __syncthreads();
       if (!sWait) return;  // given up: the chain is not marked done
-      __threadfence();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       bool ok = true;
       for (int b = lane; b < C.nblock; b += 64) ok = ok && okb[C.block0 + b] != 0;
       done = __all(ok);
