@@ -439,60 +439,82 @@ __global__ void __launch_bounds__(256) spline_p_kernel(const TrajDesc* __restric
   ppv[g] = pp;
 }
 
+// The run-up of kSplineWin knots is shared by `run` knots, which a lane does one
+// after the other: bound by the issue of the run-up's divisions where there are
+// many knots (64 particles, 0.9 M knots, a knot a lane: 682 and 446 us; in runs 77
+// and 71), by their chain where there are few (40001 knots: 44 and 25 us; 24 and
+// 19).  The run is about what leaves every SIMD one wave.
+constexpr long kSplineRunMax = 32;
+
+static long spline_run(long total) {
+  const long run = (9 * total + 64 * 1024 - 1) / (64 * 1024);
+  return run < 1 ? 1 : (run > kSplineRunMax ? kSplineRunMax : run);
+}
+
 // U_i per (knot, channel); w_i is in u (from spline_pre_kernel), U_i goes to u2
 __global__ void __launch_bounds__(256) spline_u_kernel(const TrajDesc* __restrict__ desc, int np,
                                                        const double* __restrict__ t, const double* __restrict__ p,
                                                        const double* __restrict__ sig, const double* __restrict__ ppv,
                                                        const double* __restrict__ u, double* __restrict__ u2,
-                                                       long total) {
-  long gg = (long) blockIdx.x * blockDim.x + threadIdx.x;
-  if (gg >= 9 * total) return;
-  long g = gg / 9;
-  int c = (int) (gg - 9 * g);
-  int ip = particle_of_knot(desc, np, g);
-  long o = desc[ip].knot_offset, N = desc[ip].n, i = g - o;
-  if (N < 3 || i > N - 2) return;
-  const double* X = t + o;
-  const double* Y = p + 9 * o + c;
-  double dydx0 = (Y[9] - Y[0]) / (X[1] - X[0]);
-  double u0 = ((Y[9] - Y[0]) / (X[1] - X[0]) - dydx0) * (3. / (X[1] - X[0]));
-  if (i == 0) {
-    u2[9 * g + c] = u0;
-    return;
+                                                       long total, long run) {
+  const long gg = (long) blockIdx.x * blockDim.x + threadIdx.x;
+  const long r = gg / 9;
+  const int c = (int) (gg - 9 * r);
+  const long g1 = (r + 1) * run < total ? (r + 1) * run : total;
+  for (long g = r * run; g < g1;) {  // once, or once per particle the run's knots belong to
+    const int ip = particle_of_knot(desc, np, g);
+    const long o = desc[ip].knot_offset, N = desc[ip].n, i = g - o;
+    const long end = g1 - o < N ? g1 - o : N;  // the knots i .. end - 1 of this particle
+    g = o + end > g ? o + end : g + 1;
+    if (N < 3 || i > N - 2) continue;
+    const double* X = t + o;
+    const double* Y = p + 9 * o + c;
+    double dydx0 = (Y[9] - Y[0]) / (X[1] - X[0]);
+    double u0 = ((Y[9] - Y[0]) / (X[1] - X[0]) - dydx0) * (3. / (X[1] - X[0]));
+    if (i == 0) u2[9 * o + c] = u0;
+    const long j0 = i - kSplineWin > 1 ? i - kSplineWin : 1;
+    double U = j0 == 1 ? u0 : 0.0;
+    const long i1 = i > 1 ? i : 1, top = end < N - 1 ? end : N - 1;
+    for (long j = j0; j < i1; ++j) U = (u[9 * (o + j) + c] - sig[o + j] * U) / ppv[o + j];
+    for (long j = i1; j < top; ++j) {
+      U = (u[9 * (o + j) + c] - sig[o + j] * U) / ppv[o + j];
+      u2[9 * (o + j) + c] = U;
+    }
   }
-  long j0 = i - kSplineWin > 1 ? i - kSplineWin : 1;
-  double U = j0 == 1 ? u0 : 0.0;
-  for (long j = j0; j <= i; ++j) U = (u[9 * (o + j) + c] - sig[o + j] * U) / ppv[o + j];
-  u2[9 * g + c] = U;
 }
 
 // Y''_k per (knot, channel), back substitution from the end (or from k + kWin)
 __global__ void __launch_bounds__(256) spline_b_kernel(const TrajDesc* __restrict__ desc, int np,
                                                        const double* __restrict__ t, const double* __restrict__ p,
                                                        const double* __restrict__ pv, const double* __restrict__ u2,
-                                                       double* __restrict__ ypp, long total) {
-  long gg = (long) blockIdx.x * blockDim.x + threadIdx.x;
-  if (gg >= 9 * total) return;
-  long g = gg / 9;
-  int c = (int) (gg - 9 * g);
-  int ip = particle_of_knot(desc, np, g);
-  long o = desc[ip].knot_offset, N = desc[ip].n, k = g - o;
-  if (N < 3) return;
-  const double* X = t + o;
-  const double* Y = p + 9 * o + c;
-  double qn = 0.5;
-  double xa = X[N - 2], xb = X[N - 1], ya = Y[9 * (N - 2)], yb = Y[9 * (N - 1)];
-  double dydxN = (yb - ya) / (xb - xa);
-  double un = (dydxN - (yb - ya) / (xb - xa)) * (3. / (xb - xa));
-  double last = (un - u2[9 * (o + N - 2) + c] * qn) / (pv[o + N - 2] * qn + 1.);
-  if (k == N - 1) {
-    ypp[9 * g + c] = last;
-    return;
+                                                       double* __restrict__ ypp, long total, long run) {
+  const long gg = (long) blockIdx.x * blockDim.x + threadIdx.x;
+  const long r = gg / 9;
+  const int c = (int) (gg - 9 * r);
+  const long g1 = (r + 1) * run < total ? (r + 1) * run : total;
+  for (long g = r * run; g < g1;) {
+    const int ip = particle_of_knot(desc, np, g);
+    const long o = desc[ip].knot_offset, N = desc[ip].n, k = g - o;
+    const long end = g1 - o < N ? g1 - o : N;
+    g = o + end > g ? o + end : g + 1;
+    if (N < 3 || k >= end) continue;
+    const double* X = t + o;
+    const double* Y = p + 9 * o + c;
+    double qn = 0.5;
+    double xa = X[N - 2], xb = X[N - 1], ya = Y[9 * (N - 2)], yb = Y[9 * (N - 1)];
+    double dydxN = (yb - ya) / (xb - xa);
+    double un = (dydxN - (yb - ya) / (xb - xa)) * (3. / (xb - xa));
+    double last = (un - u2[9 * (o + N - 2) + c] * qn) / (pv[o + N - 2] * qn + 1.);
+    if (end == N) ypp[9 * (o + N - 1) + c] = last;
+    const long j1 = end - 1 + kSplineWin < N - 1 ? end - 1 + kSplineWin : N - 1;
+    double v = j1 == N - 1 ? last : 0.0;
+    long j = j1 - 1;
+    for (; j >= end; --j) v = pv[o + j] * v + u2[9 * (o + j) + c];
+    for (; j >= k; --j) {
+      v = pv[o + j] * v + u2[9 * (o + j) + c];
+      ypp[9 * (o + j) + c] = v;
+    }
   }
-  long j1 = k + kSplineWin < N - 1 ? k + kSplineWin : N - 1;
-  double v = j1 == N - 1 ? last : 0.0;
-  for (long j = j1 - 1; j >= k; --j) v = pv[o + j] * v + u2[9 * (o + j) + c];
-  ypp[9 * g + c] = v;
 }
 
 // Trajectories given by the user (any increasing knot times): the sequential
@@ -697,11 +719,13 @@ extern "C" hipError_t om_launch_knot_finish(double* p, long total, hipStream_t s
 extern "C" hipError_t om_launch_spline(const om::TrajDesc* desc, int np, const double* t, const double* p,
                                        double* ypp, double* u, double* sig, double* sm1, double* pv, double* ppv,
                                        double* u2, long total, hipStream_t s) {
-  unsigned b1 = (unsigned) ((total + 255) / 256), b9 = (unsigned) ((9 * total + 255) / 256);
+  const long run = om::spline_run(total);
+  const unsigned b1 = (unsigned) ((total + 255) / 256);
+  const unsigned b9 = (unsigned) ((9 * ((total + run - 1) / run) + 255) / 256);
   hipLaunchKernelGGL(om::spline_pre_kernel, dim3(b1), dim3(256), 0, s, desc, np, t, p, sig, sm1, u, total);
   hipLaunchKernelGGL(om::spline_p_kernel, dim3(b1), dim3(256), 0, s, desc, np, sig, sm1, pv, ppv, total);
-  hipLaunchKernelGGL(om::spline_u_kernel, dim3(b9), dim3(256), 0, s, desc, np, t, p, sig, ppv, u, u2, total);
-  hipLaunchKernelGGL(om::spline_b_kernel, dim3(b9), dim3(256), 0, s, desc, np, t, p, pv, u2, ypp, total);
+  hipLaunchKernelGGL(om::spline_u_kernel, dim3(b9), dim3(256), 0, s, desc, np, t, p, sig, ppv, u, u2, total, run);
+  hipLaunchKernelGGL(om::spline_b_kernel, dim3(b9), dim3(256), 0, s, desc, np, t, p, pv, u2, ypp, total, run);
   return hipGetLastError();
 }
 
