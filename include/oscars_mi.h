@@ -179,6 +179,9 @@ int om_field_points(om_context* ctx, const om_field* fields, int nfields, const 
  * reference halves them, src/OSCARSSR.cc:1362-1378), 1 a step still met
  * |beta| >= 1 after 40 halvings (the reference recurses without limit). */
 int om_trajectory_status(om_context* ctx, int i);
+/* How trajectory i was last integrated: rounds[2], the rounds of the segmented
+ * integration forward and backward from T0; 0: in order (or no steps). */
+int om_trajectory_rounds(om_context* ctx, int i, int* rounds);
 
 /* Flux on n_obs observation points x n_e photon energies (point index
  * obs*n_e + e); n_e = 1 is the reference's flux map at one energy.

@@ -1383,6 +1383,17 @@ int om_trajectory_status(om_context* ctx, int i) {
   return ctx->desc[i].status;
 }
 
+int om_trajectory_rounds(om_context* ctx, int i, int* rounds) {
+  return guarded(ctx, [&] {
+    if (i < 0 || i >= ctx->np) throw std::out_of_range("trajectory index out of range");
+    if (!rounds) throw std::invalid_argument("rounds is NULL");
+    om::TrajDesc D;
+    read_back(ctx, &D, ctx->d_desc.p + i, sizeof(D));  // the last launch's, a batch's replay included
+    rounds[0] = D.rounds[0];
+    rounds[1] = D.rounds[1];
+  });
+}
+
 int om_trajectory_get(om_context* ctx, int i, long* n, double* t, double* p9, double* ypp9) {
   return guarded(ctx, [&] {
     if (i < 0 || i >= ctx->np) throw std::out_of_range("trajectory index out of range");

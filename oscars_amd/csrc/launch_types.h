@@ -138,7 +138,7 @@ struct ShootArgs {
   int* block_ok;   // 2 per workgroup: its joins agree
   // per chain (two per particle: forward, backward); all zero before the launch,
   // and zeroed again by rk4_kernel once it has read them
-  int* done;       // accepted
+  int* done;       // rounds taken by a chain accepted
   int* arrived;    // workgroups arrived, all rounds together
   double* t;
   double* p;

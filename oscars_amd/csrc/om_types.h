@@ -53,6 +53,8 @@ struct TrajDesc {
   long n;            // nf + nb
   int status;        // written by the kernel: 0 ok, 1 the step halving met its depth limit
   int halved;        // written by the kernel: number of steps that were halved (|beta| >= 1 met)
+  int rounds[2];     // written by the kernel: rounds of the segmented integration, forward and
+                     // backward; 0: in order (or no steps)
 };
 
 }  // namespace om

@@ -15,11 +15,11 @@
 // last bits.  The corrections are exact there (r is the exact difference of
 // two close doubles, so a segment whose start stops changing repeats its bits),
 // and a chain is accepted when no join differs by more than a small fraction of
-// the last bit of the position and velocity along the trajectory (kShootAlong):
-// the knots are then those of the integration in order, apart from the last
-// bits of the small transverse components.  On the undulators, EPUs, maps and
-// field pairs tried: 5 to 16 rounds, z and beta_z equal in every bit, x within
-// 4e-18 m.
+// the last bit of the position and velocity along the trajectory (kShootPos,
+// kShootVelAlong): the knots are then those of the integration in order, apart
+// from the last bits of the small transverse components.  On the undulators,
+// EPUs, maps and field pairs tried: 12 rounds, 25 at most, z and beta_z equal in every
+// bit, x and y within 2.1e-16 m (8e-18 m in all but four settings).
 //
 // Every step is the reference's, in the operation order of rk4_kernel (derivs
 // and rk4_try of rk4_common.h).  A segment in which |beta| >= 1 is met is never
@@ -57,15 +57,14 @@ namespace om {
 // rad, is sensitive to the last bit of z, and a join off by less than a bit
 // there is off by one further on.  Across, two units of the coordinate's own last
 // place: the joins' mismatches add up along the chain.  The random walk of the
-// last bits can keep a chain from settling (of 30 tried on the CPU the slowest
-// took 17 rounds, the mean 10.5): after kShootStrict rounds what the rounding of
-// one step in order amounts to is accepted.
+// last bits can keep a chain from settling for long: 1920 electrons through five
+// settings of fields with 3001 to 40001 points took 12 rounds at the median, 25
+// at most, and z and beta_z were those of the integration in order in every bit.
 constexpr double kShootPos = 1.3552527156068805e-20;      // 2^-66
 constexpr double kShootVelAlong = 5.551115123125783e-17;  // 2^-54
 constexpr double kShootVel = 2.168404344971009e-19;       // 2^-62
 constexpr double kShootUlps = 4.440892098500626e-16;      // 2^-51 of the component itself
-constexpr double kShootLoosePos = 1.1102230246251565e-16, kShootLooseVel = 8.881784197001252e-16;  // 2^-53, 2^-50
-constexpr int kShootRounds = 24, kShootStrict = 18;
+constexpr int kShootRounds = 32;
 constexpr int kShootSpins = 20000;  // polls of about 1 us
 
 // d <- J d + r, d in every lane; lane r < 6 holds row r of J and r_r (lanes
@@ -218,11 +217,9 @@ __global__ void __launch_bounds__(64 * kShootWaves) shoot_kernel(const ShootArgs
       if (q < 7) sSeg[wv][grp][7 * k + (q == 0 ? 6 : q - 1)] = v;
     }
     {
-      const bool strict = round < kShootStrict;
-      const double tol_x = (strict ? kShootPos : kShootLoosePos) * length;
-      const double tol_v = (strict ? kShootVel : kShootLooseVel) * speed;
+      const double tol_x = kShootPos * length, tol_v = kShootVel * speed;
       bool ok = !bad && fabs(U[1] * r[0] + U[3] * r[2] + U[5] * r[4]) <= tol_x * speed &&
-                fabs(U[1] * r[1] + U[3] * r[3] + U[5] * r[5]) <= fmax(tol_v, kShootVelAlong * speed) * speed;
+                fabs(U[1] * r[1] + U[3] * r[3] + U[5] * r[5]) <= kShootVelAlong * speed * speed;
 #pragma unroll
       for (int k = 0; k < 6; ++k)  // (a NaN is not accepted)
         ok = ok && fabs(r[k]) <= fmax((k & 1) ? tol_v : tol_x, kShootUlps * fabs(U[k]));
@@ -275,7 +272,7 @@ __global__ void __launch_bounds__(64 * kShootWaves) shoot_kernel(const ShootArgs
       done = __all(ok);
     }
     if (done) {
-      if (me == 0 && threadIdx.x == 0) A.done[A.block_chain[ib]] = 1;
+      if (me == 0 && threadIdx.x == 0) A.done[A.block_chain[ib]] = round + 1;
       return;
     }
     // The corrections.  Un must stay the very double the next segment's lanes

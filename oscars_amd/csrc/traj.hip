@@ -288,17 +288,21 @@ __global__ void __launch_bounds__(64) rk4_kernel(const UndParams f_arg, const Gr
   RkCtx c{F, nfields, 0.0, 0, g, nefields, 0.0, 0};
   // the knots are there already (an empty backward chain has nothing to do); the
   // flags are cleared for the next launch, by the lanes that have all read them
-  const bool shot_f = shot && ip < np && shot[2 * ip];
-  const bool shot_b = shot && ip < np && (shot[2 * ip + 1] || desc[ip].nb == 0);
-  const bool skip = ip >= np || (shot_f && shot_b);
+  const int shot_f = shot && ip < np ? shot[2 * ip] : 0;  // rounds taken
+  const int shot_b = shot && ip < np ? shot[2 * ip + 1] : 0;
+  const bool skip = ip >= np || (shot_f && (shot_b || desc[ip].nb == 0));
   __syncthreads();
   if (shot && ip < np && sub < 2) {
     shot[2 * ip + sub] = 0;             // done
     shot[2 * np + 2 * ip + sub] = 0;    // arrived
   }
-  if (skip && ip < np && sub == 0) {
-    desc[ip].status = 0;
-    desc[ip].halved = 0;
+  if (ip < np && sub == 0) {
+    desc[ip].rounds[0] = skip ? shot_f : 0;
+    desc[ip].rounds[1] = skip ? shot_b : 0;
+    if (skip) {
+      desc[ip].status = 0;
+      desc[ip].halved = 0;
+    }
   }
   if (__all(skip)) return;  // the workgroup is one wave
   if (M == kGridZ) {
