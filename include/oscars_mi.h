@@ -182,6 +182,13 @@ int om_trajectory_status(om_context* ctx, int i);
 /* How trajectory i was last integrated: rounds[2], the rounds of the segmented
  * integration forward and backward from T0; 0: in order (or no steps). */
 int om_trajectory_rounds(om_context* ctx, int i, int* rounds);
+/* Limits of the segmented integration in this context, from the next
+ * integration on: rounds before a trajectory is integrated in order instead
+ * (0: always in order; at most 32), and polls of 0.4 us that one of its
+ * workgroups waits for the others (0: no wait).  -1: the default (32 rounds, a
+ * poll per step).  The trajectory is the same within the last bits
+ * whichever way it is integrated. */
+int om_trajectory_limits(om_context* ctx, int rounds, int polls);
 
 /* Flux on n_obs observation points x n_e photon energies (point index
  * obs*n_e + e); n_e = 1 is the reference's flux map at one energy.

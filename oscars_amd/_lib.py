@@ -62,7 +62,7 @@ class om_stats(C.Structure):
 EXPORTS = ["om_device_count", "om_device_info", "om_context_create", "om_context_destroy", "om_last_error",
            "om_trajectories", "om_trajectories_eb", "om_trajectory_set", "om_trajectory_get", "om_power_density_surface",
            "om_total_power", "om_efield_time", "om_field_points", "om_power_density_stl", "om_level_get",
-           "om_trajectory_status", "om_trajectory_rounds", "om_flux",
+           "om_trajectory_status", "om_trajectory_rounds", "om_trajectory_limits", "om_flux",
            "om_spectrum", "om_power_density", "om_batch_setup", "om_batch_run", "om_batch_tune",
            "om_batch_profile",
            "om_adjoint_forward", "om_adjoint_backward", "om_flux_dev", "om_spectrum_dev", "om_power_density_dev",
@@ -102,6 +102,7 @@ def lib():
     L.om_trajectory_set.argtypes = [C.c_void_p, C.POINTER(om_particle), C.c_long, _dp, _dp, C.c_int]
     L.om_level_get.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, _dp]
     L.om_trajectory_status.argtypes = [C.c_void_p, C.c_int]
+    L.om_trajectory_limits.argtypes = [C.c_void_p, C.c_int, C.c_int]
     L.om_trajectory_rounds.argtypes = [C.c_void_p, C.c_int, _ip]
     L.om_flux.argtypes = [C.c_void_p, C.c_int, _dp, C.c_long, _dp, C.c_long, _dp, C.POINTER(om_conv), _dp, _ip,
                           _up, _dp, C.POINTER(om_stats)]
@@ -227,6 +228,10 @@ class Device:
         r = np.zeros(2, dtype=np.int32)
         self._chk(self.L.om_trajectory_rounds(self.h, i, _ptr(r, _ip)))
         return int(r[0]), int(r[1])
+
+    def trajectory_limits(self, rounds=-1, polls=-1):
+        """Limits of the segmented integration from the next integration on (om_trajectory_limits)."""
+        self._chk(self.L.om_trajectory_limits(self.h, int(rounds), int(polls)))
 
     def level(self, i, L, extended=False):
         out = np.zeros((2 ** L, 10))

@@ -277,6 +277,7 @@ struct om_context {
   // (nblocks 0) where the steps are taken in order
   struct Shoot {
     int nchains = 0, nblocks = 0;
+    int rounds = om::kShootRounds, polls = -1;  // om_trajectory_limits
     std::vector<om::ShootChain> chain;
     std::vector<int> block_chain, flags;
     DevBuf<om::ShootChain> d_chain;
@@ -842,7 +843,7 @@ void shoot_setup(om_context* ctx, int np) {
     longest = std::max(longest, std::max(ctx->desc[i].nf, ctx->desc[i].nb));
     total += ctx->desc[i].nf + ctx->desc[i].nb;
   }
-  if (ctx->nefields > 0 || longest < kShootMinSteps || total > kShootMaxRatio * longest) return;
+  if (ctx->nefields > 0 || longest < kShootMinSteps || total > kShootMaxRatio * longest || S.rounds < 1) return;
   om::FieldDev none;
   std::memset(&none, 0, sizeof(none));
   const long per_step = 8L * om::kShootWaves;  // segments of a workgroup
@@ -903,6 +904,8 @@ void launch_trajectories(om_context* ctx, int np) {
     A.block_chain = S.d_block_chain.p;
     A.nblocks = S.nblocks;
     A.Mb = S.maps.p;
+    A.rounds = S.rounds;
+    A.polls = S.polls;
     A.done = S.d_flags.p;
     A.arrived = S.d_flags.p + S.nchains;
     A.block_ok = S.d_flags.p + 2 * S.nchains;
@@ -1381,6 +1384,16 @@ int om_trajectory_status(om_context* ctx, int i) {
   if (!ctx || i < 0 || i >= ctx->np) return -1;
   if (guarded(ctx, [&] { sync_desc(ctx); })) return -1;
   return ctx->desc[i].status;
+}
+
+int om_trajectory_limits(om_context* ctx, int rounds, int polls) {
+  return guarded(ctx, [&] {
+    if (rounds < -1 || rounds > om::kShootRounds) throw std::out_of_range("rounds must be -1 .. 32");
+    if (polls < -1) throw std::out_of_range("polls must be -1 or more");
+    ctx->shoot.rounds = rounds < 0 ? om::kShootRounds : rounds;
+    ctx->shoot.polls = polls;
+    ctx->batch.drop_graphs();
+  });
 }
 
 int om_trajectory_rounds(om_context* ctx, int i, int* rounds) {

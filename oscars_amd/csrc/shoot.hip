@@ -24,7 +24,7 @@
 // Every step is the reference's, in the operation order of rk4_kernel (derivs
 // and rk4_try of rk4_common.h).  A segment in which |beta| >= 1 is met is never
 // accepted (its steps would have to be halved), nor is a chain whose joins
-// still differ after kShootRounds rounds: rk4_kernel then integrates that
+// still differ after A.rounds rounds: rk4_kernel then integrates that
 // particle in order, as it does for short chains.
 //
 // Layout: one wave holds eight segments of eight lanes.  Lane 0 of a segment
@@ -40,9 +40,16 @@
 // points 37.5 -> 0.44 ms, 1-D map 20001 points 18.1 -> 0.3 ms, undulator and
 // Gaussian 8001 points 23.7 -> 0.5 ms.
 //
-// The wait is bounded (kShootSpins): if the workgroups of a chain cannot all be
-// resident, because other work fills the GPU, the chain is given up after some
-// tens of milliseconds and integrated in order.
+// The wait is bounded: if the workgroups of a chain cannot all be resident,
+// because other work fills the GPU, the first whose wait runs out gives the chain
+// up for all (the count of arrivals turns negative), and it is integrated in
+// order.  It runs out after a poll (0.4 us) per step, about half the time in
+// order takes with one magnet and far more than a round's.  300 calls beside a
+// batch of 8 / 12 waves per CU: 20001 planar points 4 / 15 given up (16 to 21 ms
+// each), mean 1.9 / 4.9 ms; 40001 EPU points 9 / 29 (42 to 55 ms, 107 for a few
+// that found no place to run), mean 4.6 / 9.3 ms; every call in order takes 13 and
+// 36 ms.  A quarter of the wait: 5 / 46 and 8 / 33 given up; three times: 4 / 8 and
+// 10 / 8, of 25 to 32 and 52 to 64 ms.
 #include "om_device.h"
 #include "launch_types.h"
 #include "om_types.h"
@@ -64,8 +71,7 @@ constexpr double kShootPos = 1.3552527156068805e-20;      // 2^-66
 constexpr double kShootVelAlong = 5.551115123125783e-17;  // 2^-54
 constexpr double kShootVel = 2.168404344971009e-19;       // 2^-62
 constexpr double kShootUlps = 4.440892098500626e-16;      // 2^-51 of the component itself
-constexpr int kShootRounds = 32;
-constexpr int kShootSpins = 20000;  // polls of about 1 us
+constexpr int kShootGivenUp = -(1 << 30);  // arrivals of a chain given up, plus those since
 
 // d <- J d + r, d in every lane; lane r < 6 holds row r of J and r_r (lanes
 // beyond compute copies of row 5).
@@ -173,7 +179,7 @@ __global__ void __launch_bounds__(64 * kShootWaves) shoot_kernel(const ShootArgs
   double* tk = A.t + D->knot_offset;
   double* pk = A.p + 9 * D->knot_offset;
   const long nb = D->nb;
-  for (int round = 0; round < kShootRounds; ++round) {
+  for (int round = 0; round < A.rounds; ++round) {
     // lanes 1..6: the start moved along coordinate q - 1, by 2^-26 m or 2^-24 c
     // (any step between the roundings and the fields' scale serves: the
     // differences only steer the corrections)
@@ -255,13 +261,13 @@ __global__ void __launch_bounds__(64 * kShootWaves) shoot_kernel(const ShootArgs
         if (lane == 0) {
           int* cnt = A.arrived + A.block_chain[ib];
           const int target = C.nblock * (round + 1);
-          atomicAdd(cnt, 1);
-          int spins = 0;
-          while (__hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target && spins < kShootSpins) {
+          int now = atomicAdd(cnt, 1) + 1;
+          for (long polls = A.polls >= 0 ? A.polls : n; now >= 0 && now < target && polls > 0; --polls) {
             __builtin_amdgcn_s_sleep(1);
-            ++spins;
+            now = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           }
-          sWait = spins < kShootSpins ? 1 : 0;
+          if (now < target) atomicMin(cnt, kShootGivenUp);
+          sWait = now < target ? 0 : 1;
         }
       }
       __syncthreads();
