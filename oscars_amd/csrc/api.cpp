@@ -697,7 +697,10 @@ constexpr long kWaveListMax = 16384;
 // pack an observation point's energies across its groups: 1444 groups 3.3 ms
 // against 3.7 ms.  The slices' 17 MB of partial sums fit into the static scratch
 // of the allocation-free entry point beside level 18 (42 MB, the deepest that
-// fits) and 65536 points.
+// fits) and 65536 points.  From the host's first look on the list's tiles are cut
+// in place of the groups, so that the slices follow the energies still active:
+// 1024 groups of which one goes on to level 20, 49 ms with a tile's level shared
+// by 8 waves, 63 ms with slices by the request's groups, 2.5 ms by the tiles.
 constexpr long kSliceGroups = 1024;
 constexpr int kListFrom = 9;  // first level that can stop a point (src/OSCARSSR.cc:2006: L > 8)
 
@@ -1037,7 +1040,8 @@ int lw_sums(om_context* ctx, int ip, const double* obs_xyz, long n_obs, const do
         for (int L = std::max(La, kListFrom - 1); L <= Lb; ++L) {
           const long most = L < kListFrom ? 8 : (1L << L) / om::kSliceMin;
           X.L = L;
-          X.nsl = (int) std::max(1L, std::min(most, om::kSliceJobs / X.n_groups));
+          if (A.list) X.n_groups = ntiles;  // never more tiles than groups
+          X.nsl = (int) std::max(1L, std::min({most, om::kSliceMost, om::kSliceJobs / X.n_groups}));
           check(om_launch_lw_slice(&A, &X, mixed ? 1 : 0, ctx->stream), "lw_slice");
         }
       } else if (!tiled && (A.list ? A.n_list : npts) <= kWaveListMax) {

@@ -363,36 +363,48 @@ __global__ void __launch_bounds__(64 * S) lw_tile_kernel(LwArgs A, long n_tiles_
 // 32 for 2000 energies on axis, 256 waves with a level shared by 8, a quarter of
 // the SIMDs, waiting for the host's look at the active list before every level
 // (0.43 ms of kernels and 0.4 ms of lists and waits for 6 levels).  Here a level
-// of every group is cut into slices, about kSliceJobs in all (4096: four waves a
-// SIMD); a group's active energies are packed from their flags by each of its
-// slices, in replicas when few are left; and the slice that completes a group
-// adds the partial sums and takes the decisions.  The levels follow each other
-// on the stream with no look from the host.  Bound by the chain of one slice:
-// 37 us a level, of which 256 samples in FP64 take 25.  2000 energies on axis:
-// 1.73 -> 1.13 ms a call, 0.18 ms of it in these launches.
+// of every group is cut into slices of at least 256 samples, at most 4096 in all
+// (four waves a SIMD) and 512 to a group: 2000 energies take 64 waves at level 9
+// and 1024 at level 13, 128 groups and more 4096 from level 13 on.  A group's
+// active energies are packed from their flags by each of its slices, in replicas
+// when few are left; and the slice that completes a group adds the partial sums
+// and takes the decisions.  Up to level 13 the levels follow each other on the
+// stream with no look from the host; beyond, the host has listed the active
+// energies in tiles, and the tiles take the groups' place.  Bound by the chain of
+// one slice: 37 us a level, of which 256 samples in FP64 take 25.  2000 energies
+// on axis: 1.73 -> 1.13 ms a call, 0.18 ms of it in these launches.
 template <bool MIXED>
 __global__ void __launch_bounds__(256) lw_slice_kernel(LwArgs A, SliceArgs X) {
   __shared__ AmpLds lds[4];
-  __shared__ unsigned char lists[4][64];
+  __shared__ int lists[4][64];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const long job = (long) blockIdx.x * 4 + wv;
   if (job >= X.n_groups * X.nsl) return;  // whole waves leave; no workgroup barrier below
   const long g = job / X.nsl, sl = job - g * X.nsl;
-  const long io = g / X.blocks_e, e0 = (g - io * X.blocks_e) * 64;
   const bool first = X.L == 8;
-  const long p0 = io * A.n_omega + e0;
-  const bool in = e0 + lane < A.n_omega;
-  const bool live = in && (first || (!A.st.conv[p0 + lane] && A.st.level[p0 + lane] == X.L - 1));
+  long io;
+  int pl;     // this lane's point of the group
+  bool live;  // still to be summed
+  if (A.list) {  // tile g of the list: energies of one observation point, pads (-1) last
+    pl = A.list[64 * g + lane];
+    io = A.list[64 * g] / A.n_omega;
+    live = pl >= 0;
+  } else {
+    io = g / X.blocks_e;
+    const long e = (g - io * X.blocks_e) * 64 + lane;
+    pl = (int) (io * A.n_omega + e);
+    live = e < A.n_omega && (first || (!A.st.conv[pl] && A.st.level[pl] == X.L - 1));
+  }
   const unsigned long long mask = __ballot(live);
   const int W = __popcll(mask);
   if (W == 0) return;  // the same for every slice of the group: its state changes after all have arrived
-  unsigned char* list = lists[wv];
-  if (live) list[__popcll(mask & ((1ULL << lane) - 1ULL))] = (unsigned char) lane;
+  int* list = lists[wv];
+  if (live) list[__popcll(mask & ((1ULL << lane) - 1ULL))] = pl;
   wave_sync();
   const int m = 64 / W, q = lane / W;
   const bool act = q < m;
-  const int e = list[act ? lane - q * W : 0];
-  const double negw = -A.omega[e0 + e];
+  const long p = list[act ? lane - q * W : 0];
+  const double negw = -A.omega[p - io * A.n_omega];
   const V3 obs = v3(A.obs[3 * io], A.obs[3 * io + 1], A.obs[3 * io + 2]);
   // levels 0..8 lie one after the other: their sums are one sum of 511 samples
   const double* __restrict__ rows = A.lv.rows[first ? 0 : X.L];
@@ -410,7 +422,6 @@ __global__ void __launch_bounds__(256) lw_slice_kernel(LwArgs A, SliceArgs X) {
     part_gather(X.part + g * X.nsl * (8 * 64), X.nsl, lane, W, m, q, act, ps, maxd, an);
   }
   if (!mine) return;
-  const long p = p0 + e;
   double sum[6], lastmag = -1, prec = -1, an_run = an, dm_last = 0;
   if (first) {
 #pragma unroll

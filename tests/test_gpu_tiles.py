@@ -207,6 +207,31 @@ def test_flux_deep_levels(epu_pair, mode, tol, shape):
 
 
 @gpu
+@pytest.mark.parametrize("mode,tol", [("tiled", 1e-9), ("mixed", 1e-5)])
+@pytest.mark.parametrize("n_obs,n_e,far", [(1024, 64, [0.02]), (1000, 3, [0.015, 0.03]), (97, 650, [0.02, 0.02]),
+                                           (1, 65, [0.02])])
+def test_flux_stragglers(epu_pair, mode, tol, n_obs, n_e, far):
+    """Requests of up to 1024 groups of which one or two observation points go on
+    beyond level 13, through the tiles listed for them: whole ones, remainders,
+    and energies packed across a point's groups.  Against the plain path's values
+    in a call of their own (tolerances as above), levels identical."""
+    o, dev = epu_pair
+    obs = _scatter(n_obs, 0.0005, 20.0, seed=n_obs)
+    at = np.linspace(0, n_obs - 1, len(far) + 2).astype(int)[1:-1]
+    obs[at, 0] = far
+    e = np.linspace(600.0, 3000.0, n_e)
+    kw = dict(precision=3e-3, max_level=16, max_level_extended=16)
+    v, lev, cv, _, _ = dev.flux(0, obs, e, [0.0] * 6, dev.conv(mode=mode, **kw))
+    v, lev, cv = (x.reshape(n_obs, n_e) for x in (v, lev, cv))
+    assert np.all(lev[at].max(axis=1) > 13)
+    k = np.unique(np.concatenate([at, [0, n_obs - 1]]))
+    pv, plev, pcv, _, _ = dev.flux(0, obs[k], e, [0.0] * 6, dev.conv(mode="plain", **kw))
+    pv, plev, pcv = (x.reshape(len(k), n_e) for x in (pv, plev, pcv))
+    assert np.array_equal(lev[k], plev) and np.array_equal(cv[k], pcv)
+    assert all(rel_err(v[i], pv[j], 1e-6) < tol for j, i in enumerate(k))
+
+
+@gpu
 @pytest.mark.parametrize("level", [0, 1, 2, 7, 8, 9, 10])
 def test_power_density_stl_caps(tmp_path, level):
     """Levels on both sides of the first ones summed as one (0..8), down to
