@@ -150,8 +150,8 @@ def batched_headline(args, cfg):
     # units is not representative of the mix of request sizes
     best, tt = bf.tune(candidates=(8, 16), sample_items=1 << 40)
     # then the level from which the points still running are handed over to
-    # the level kernels (0: none), on the whole launch
-    deep, td = bf.tune_deep((0, 13, 17))
+    # the level kernels (-1: none, 0: by the number of units), on the whole launch
+    deep, td = bf.tune_deep((-1, 13, 0))
     log("setup + tuner %.1f s: %d waves/CU %s, hand-over level %d %s" % (time.perf_counter() - t0, best, tt, deep, td))
     for k in range(args.warmup):
         _, st = bf.run(recompute_trajectories=True)

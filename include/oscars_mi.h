@@ -302,9 +302,9 @@ typedef struct {
   int max_level;    /* highest level held as stored sample rows (0: up to 18 within 40% of the
                        device memory); deeper levels, up to the conv's max_level rule, are
                        interpolated */
-  int deep_level;   /* points still active at this level leave their work unit and go on with
-                       their samples split over the GPU (0: chosen from the number of units; a
-                       level above the conv's last: none) */
+  int deep_level;   /* points still active at this level (at least 9) leave their work unit and
+                       go on with their samples split over the GPU (0: chosen from the number of
+                       units; negative, or above the conv's last level: none) */
 } om_batch_opts;
 
 int om_batch_setup(om_context* ctx, const om_request* req, int n_req, const int* req_of, const double* weight,
@@ -330,9 +330,8 @@ int om_batch_profile(om_context* ctx, int recompute_trajectories, double* stage_
  * keeps the fastest (returned in *best). */
 int om_batch_tune(om_context* ctx, const int* candidates, int n, long sample_items, int* best, double* ms_out);
 /* Times the whole batch launch (persistent kernel, deep-level and recheck
- * kernels) on the full workload for each candidate hand-over level (0: none;
- * else at least 9, as om_batch_opts.deep_level) and keeps the fastest
- * (returned in *best; the times in ms_out[n] when not NULL).  No counterpart
+ * kernels) on the full workload for each candidate hand-over level (as
+ * om_batch_opts.deep_level) and keeps the fastest (that candidate in *best; the times in ms_out[n] when not NULL).  No counterpart
  * in the reference. */
 int om_batch_tune_deep(om_context* ctx, const int* deep_levels, int n, int* best, double* ms_out);
 

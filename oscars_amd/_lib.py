@@ -510,8 +510,8 @@ class Device:
             C.byref(st)))
         return st.as_dict()
 
-    def batch_tune_deep(self, deep_levels=(0, 13, 15)):
-        """om_batch_tune_deep: (best hand-over level, {level: ms})."""
+    def batch_tune_deep(self, deep_levels=(0, -1, 13, 15)):
+        """om_batch_tune_deep: (best hand-over level, {level: ms}); 0: the rule's, negative: none."""
         c = np.ascontiguousarray(deep_levels, dtype=np.int32)
         ms = np.zeros(len(c))
         best = C.c_int(0)

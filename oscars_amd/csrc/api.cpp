@@ -1890,6 +1890,12 @@ constexpr int kBatchNoHandOver = 99;  // a hand-over level above every level: no
 // 42.8 / 51.7 ms; 304032 units, 0 / 12 / 14 / 16 / 17 / 18: 993 / 1159 / 1139 / 888 /
 // 886 / 889 ms; 1755904 units, 0 / 14 / 16 / 17 / 18: 5096 / 5482 / 5709 / 4845 / 4848.
 int batch_hand_over(long units) { return units <= 40000 ? 12 : units <= 120000 ? 14 : 17; }
+
+// deep_level as the entry points take it: 0 by the rule, negative none.
+int batch_deep(int deep_level, long units) {
+  if (deep_level > 0 && deep_level < 9) throw std::out_of_range("deep_level must be at least 9, 0 or negative");
+  return deep_level > 0 ? deep_level : deep_level < 0 ? kBatchNoHandOver : batch_hand_over(units);
+}
 constexpr int kBatchRowsCap = 17;            // highest level stored as rows by default ...
 constexpr double kBatchRowsFraction = 0.4;   // ... within this fraction of the device memory
 
@@ -2049,8 +2055,7 @@ int om_batch_setup(om_context* ctx, const om_request* req, int n_req, const int*
     A.main_evals = B.counters.p + 6;
     A.n_recheck = B.counters.p + 7;
     A.main_slots = B.counters.p + 8;
-    A.Ldeep = (opts && opts->deep_level > 0) ? opts->deep_level : batch_hand_over(B.total_items);
-    if (A.Ldeep < 9) throw std::out_of_range("deep_level must be at least 9");
+    A.Ldeep = batch_deep(opts ? opts->deep_level : 0, B.total_items);
     A.n_group = B.counters.p + kBatchReport;
     A.n_list = B.counters.p + kBatchReport + 1;
     A.n_job = A.n_list + 2 * om::kBatchLevels;
@@ -2232,13 +2237,12 @@ int om_batch_tune_deep(om_context* ctx, const int* deep_levels, int n, int* best
     auto& B = ctx->batch;
     if (!B.ready) throw std::logic_error("om_batch_setup has not been called");
     if (n < 1 || !deep_levels) throw std::invalid_argument("no candidates");
-    for (int i = 0; i < n; ++i)
-      if (deep_levels[i] != 0 && deep_levels[i] < 9) throw std::out_of_range("deep_level must be 0 or at least 9");
+    for (int i = 0; i < n; ++i) (void) batch_deep(deep_levels[i], B.total_items);
     batch_levels(ctx);
     double best_ms = 1e300;
     int best_d = deep_levels[0];
     for (int i = 0; i < n; ++i) {
-      B.args.Ldeep = deep_levels[i] > 0 ? deep_levels[i] : kBatchNoHandOver;
+      B.args.Ldeep = batch_deep(deep_levels[i], B.total_items);
       check(om_launch_batch_clear(B.out.p, B.total_out, B.counters.p, kBatchCounters, ctx->stream), "clear");
       check(hipEventRecord(ctx->ev0, ctx->stream), "event");
       check(om_launch_lw_batch(&B.args, B.mixed, B.groups, ctx->stream), "lw batch");
@@ -2252,7 +2256,7 @@ int om_batch_tune_deep(om_context* ctx, const int* deep_levels, int n, int* best
         best_d = deep_levels[i];
       }
     }
-    B.args.Ldeep = best_d > 0 ? best_d : kBatchNoHandOver;
+    B.args.Ldeep = batch_deep(best_d, B.total_items);
     B.drop_graphs();
     if (best) *best = best_d;
   });

@@ -197,3 +197,38 @@ def test_batched_mixed_levels_match_fp64(deep_level):
           % (deep_level, s32["evals"], s64["evals"], s32["n_rechecked"], max(errs)))
     assert s32["evals"] == s64["evals"]
     assert max(errs) < 1e-5
+
+
+@gpu
+def test_hand_over_level_has_one_meaning(batch_case):
+    """deep_level 0 is the rule's level and a negative one none, in the set-up and
+    in the tuner, whose choice can be given back to the set-up."""
+    from oscars_amd import multiparticle as M
+    from oscars_amd.sr import sr
+    parts, windows, reqs, req_of, weights, ref = batch_case
+    s = sr()
+    s.add_bfield_undulator(**UNDULATOR)
+    dev = s._device()
+
+    def handed(deep):
+        bf = M.BatchedFlux(dev, s._fields, parts, windows, reqs, req_of, weights, mode="tiled", precision=1e-3,
+                           deep_level=deep)
+        return bf, dev.batch_profile(False)[1]["handed_over"]
+    n = {deep: handed(deep)[1] for deep in (0, 12, -1, 27)}
+    assert n[0] == n[12] > 0 and n[-1] == n[27] == 0
+    bf, _ = handed(9)
+    for deep in (0, 12, -1):
+        best, times = bf.tune_deep((deep,))
+        assert best == deep and list(times) == [deep]
+        assert dev.batch_profile(False)[1]["handed_over"] == n[deep]
+    for bad in (1, 8):
+        with pytest.raises(Exception):
+            bf.tune_deep((bad,))
+        with pytest.raises(Exception):
+            handed(bad)
+
+
+@gpu
+def test_batched_mixed_levels_in_their_unit():
+    """As above with every point finished in its unit, its FP64 recheck included."""
+    test_batched_mixed_levels_match_fp64(-1)
