@@ -310,7 +310,7 @@ struct om_context {
   struct Batch {
     bool ready = false;
     int np = 0, n_req = 0, Lb = 0, Lmax = 0, stop_mem = 0, mixed = 0, groups = 0;
-    long stride = 0, total_items = 0, total_out = 0;
+    long stride = 0, total_items = 0, total_out = 0, total_points = 0, total_groups = 0;
     std::vector<long> out_off, out_n;
     DevBuf<double> rows, tspan, obs, omega, out, weight;
     DevBuf<int> req_of;
@@ -1909,18 +1909,24 @@ void batch_scratch(om_context* ctx, long groups, om::BatchArgs& A) {
   A.wsi = B.wsi.p;
 }
 
-// Room for the groups of energies handed to the level kernels: three per work
-// unit (most units hand over one or none; what finds no room stays in its unit).
+// Room for the groups of energies handed to the level kernels (what finds no room
+// stays in its unit): three per work unit, as most units hand over one or none,
+// and no more than there can be; none where no level is handed over.
 void batch_groups(om_context* ctx, om::BatchArgs& A) {
   auto& B = ctx->batch;
-  A.group_cap = std::min(kBatchGroupCap, std::max(4096L, 3 * B.total_items));
+  if (A.Ldeep > A.Lmax) return;  // group_cap 0
+  // a unit hands each of its passes' energies over once, the recomputation list
+  // its points one by one
+  const long most = B.mixed ? 2 * B.total_groups + B.total_points : B.total_groups;
+  A.group_cap = std::min({kBatchGroupCap, std::max(4096L, 3 * B.total_items), most});
   B.group_list.ensure(4 * A.group_cap);
   B.group_item.ensure(A.group_cap);
   B.group_n.ensure(A.group_cap);
   B.group_e.ensure(64 * A.group_cap);
   B.group_state.ensure((size_t) om::kBatchGroupD * 64 * A.group_cap);
   B.group_arrived.ensure(A.group_cap);
-  B.part.ensure((size_t) om::kBatchParts * 8 * 64);
+  // a level is cut into at most 256 slices a group and kBatchParts in all
+  B.part.ensure((size_t) std::min(om::kBatchParts, om::kBatchGroupSlices * A.group_cap) * 8 * 64);
   check(om_launch_adj_key_fill(reinterpret_cast<int*>(B.group_arrived.p), A.group_cap, 0, ctx->stream), "clear");
   A.group_list = B.group_list.p;
   A.group_item = B.group_item.p;
@@ -1998,13 +2004,16 @@ int om_batch_setup(om_context* ctx, const om_request* req, int n_req, const int*
     }
     upload(ctx, B.req, rd.data(), n_req);
     std::vector<long> prefix(np + 1, 0);
-    long total_points = 0;
+    long total_points = 0, total_groups = 0;
     for (int i = 0; i < np; ++i) {
       const om::ReqDev& R = rd[req_of[i]];
       prefix[i + 1] = prefix[i] + R.n_obs * R.n_blocks_e;
       total_points += R.n_obs * R.n_e;
+      total_groups += R.n_obs * ((R.n_e + 63) / 64);
     }
     B.total_items = prefix[np];
+    B.total_points = total_points;
+    B.total_groups = total_groups;
     upload(ctx, B.prefix, prefix.data(), prefix.size());
     upload(ctx, B.req_of, req_of, np);
     upload(ctx, B.weight, weight, np);
@@ -2059,9 +2068,9 @@ int om_batch_setup(om_context* ctx, const om_request* req, int n_req, const int*
     A.n_group = B.counters.p + kBatchReport;
     A.n_list = B.counters.p + kBatchReport + 1;
     A.n_job = A.n_list + 2 * om::kBatchLevels;
-    batch_groups(ctx, A);
     A.total_items = B.total_items;
     B.mixed = conv->mode == OM_MODE_MIXED ? 1 : 0;
+    batch_groups(ctx, A);
     if (B.mixed) {
       // room for every point up to kBatchFixCap; points flagged beyond it keep the mixed result
       A.fix_cap = total_points < kBatchFixCap ? total_points : kBatchFixCap;
@@ -2243,6 +2252,7 @@ int om_batch_tune_deep(om_context* ctx, const int* deep_levels, int n, int* best
     int best_d = deep_levels[0];
     for (int i = 0; i < n; ++i) {
       B.args.Ldeep = batch_deep(deep_levels[i], B.total_items);
+      if (B.args.group_cap == 0) batch_groups(ctx, B.args);
       check(om_launch_batch_clear(B.out.p, B.total_out, B.counters.p, kBatchCounters, ctx->stream), "clear");
       check(hipEventRecord(ctx->ev0, ctx->stream), "event");
       check(om_launch_lw_batch(&B.args, B.mixed, B.groups, ctx->stream), "lw batch");

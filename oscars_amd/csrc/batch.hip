@@ -527,7 +527,7 @@ lw_batch_level_kernel(BatchArgs A, int L) {
   // there is room for (16 for each of the 4096 waves; their cost depends on the
   // group's energies, so they are taken from a counter)
   long nsl = kBatchParts / n;
-  nsl = nsl < 1 ? 1 : (nsl > 256 ? 256 : nsl);
+  nsl = nsl < 1 ? 1 : (nsl > kBatchGroupSlices ? kBatchGroupSlices : nsl);
   nsl = nsl > ns / 512 ? ns / 512 : nsl;
   const int* __restrict__ ids = A.group_list + (2 * kind + (L & 1)) * A.group_cap;
   while (true) {

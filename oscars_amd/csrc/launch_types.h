@@ -205,6 +205,7 @@ constexpr int kBatchWsI = 2;
 constexpr int kBatchGroupD = 9;
 constexpr int kBatchLevels = kMaxLevel + 2;
 constexpr long kBatchParts = 65536;
+constexpr long kBatchGroupSlices = 256;  // of one group, at most
 constexpr int kBatchWsTotal = kBatchWsD * kBatchEB + (kBatchEB / 64) * 7 * 64;
 
 struct ReqDev {

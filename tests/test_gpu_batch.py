@@ -232,3 +232,35 @@ def test_hand_over_level_has_one_meaning(batch_case):
 def test_batched_mixed_levels_in_their_unit():
     """As above with every point finished in its unit, its FP64 recheck included."""
     test_batched_mixed_levels_match_fp64(-1)
+
+
+@gpu
+def test_small_batch_takes_little_memory(batch_case):
+    """The groups handed over and their partial sums are sized by what the batch
+    can hand over, and are left out where nothing is handed over, until the tuner
+    asks for a level: 70 + 384 + 10 points, 4.8 KB a group and 4 KB for each of its
+    256 slices, once (tiled: 10 groups, 10 MB); beside them 17 MB of wave scratch,
+    1 MB of rows and a margin of 16 MB for allocation in blocks."""
+    import torch
+    from oscars_amd import _lib
+    from oscars_amd import multiparticle as M
+    from oscars_amd.sr import sr
+    parts, windows, reqs, req_of, weights, ref = batch_case
+    s = sr()
+    s.add_bfield_undulator(**UNDULATOR)
+    parts, windows, req_of, weights = parts[:3], windows[:3], req_of[:3], weights[:3]
+    for deep, most in ((-1, 34e6), (0, 45e6)):
+        dev = _lib.Device(0)
+        dev.trajectories(s._fields, M.om_particles(parts, windows))
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info(0)[0]
+        dev.batch_setup(reqs, req_of, weights, [0.0] * 6, dev.conv(mode="tiled"), 1, 10, deep)
+        used = free - torch.cuda.mem_get_info(0)[0]
+        print("deep_level %d: %.1f MB" % (deep, used / 1e6))
+        assert used < most
+        first, _ = dev.batch_run(False)
+        best, _ = dev.batch_tune_deep((9, 12))
+        outs, st = dev.batch_run(False)
+        assert st["n_unconverged"] == 0
+        assert all(rel_err(a, b, 1e-6) < 1e-11 for a, b in zip(outs, first))
+        assert dev.batch_profile(False)[1]["handed_over"] > 0 or best == 12
