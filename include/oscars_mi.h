@@ -309,6 +309,10 @@ typedef struct {
 
 int om_batch_setup(om_context* ctx, const om_request* req, int n_req, const int* req_of, const double* weight,
                    const double* pol6, const om_conv* conv, const om_batch_opts* opts);
+/* Limit of the next om_batch_setup in this context: groups of up to 64 energies
+ * that may leave their work units (each holds 4.8 KB); the energies that find no
+ * group are finished in their unit.  -1: the default, by the batch's size. */
+int om_batch_limits(om_context* ctx, long groups);
 /* One step: [RK4 + spline when recompute_trajectories] + level samples + all
  * sums, replayed from a captured HIP graph; out[r] receives request r's grid
  * (n_obs x n_e, energy fastest). */

@@ -66,7 +66,8 @@ EXPORTS = ["om_device_count", "om_device_info", "om_context_create", "om_context
            "om_spectrum", "om_power_density", "om_batch_setup", "om_batch_run", "om_batch_tune",
            "om_batch_profile",
            "om_adjoint_forward", "om_adjoint_backward", "om_flux_dev", "om_spectrum_dev", "om_power_density_dev",
-           "om_flux_dev_noalloc", "om_adjoint_forward_dev", "om_adjoint_backward_dev", "om_batch_tune_deep"]
+           "om_flux_dev_noalloc", "om_adjoint_forward_dev", "om_adjoint_backward_dev", "om_batch_tune_deep",
+           "om_batch_limits"]
 
 _lib = None
 
@@ -130,6 +131,7 @@ def lib():
                                  C.POINTER(om_batch_opts)]
     L.om_batch_run.argtypes = [C.c_void_p, C.c_int, C.POINTER(_dp), C.POINTER(om_stats)]
     L.om_batch_tune.argtypes = [C.c_void_p, _ip, C.c_int, C.c_long, _ip, _dp]
+    L.om_batch_limits.argtypes = [C.c_void_p, C.c_long]
     L.om_batch_tune_deep.argtypes = [C.c_void_p, _ip, C.c_int, _ip, _dp]
     L.om_batch_profile.argtypes = [C.c_void_p, C.c_int, _dp, C.POINTER(C.c_ulonglong), C.POINTER(om_stats)]
     L.om_adjoint_forward.argtypes = [C.c_void_p, C.POINTER(om_field), C.c_int, C.c_int, C.POINTER(om_particle),
@@ -435,6 +437,10 @@ class Device:
         self._chk(self.L.om_batch_setup(self.h, ra, len(requests), _ptr(ro, _ip), _ptr(w), _ptr(pol),
                                         C.byref(conv), C.byref(opts)))
         self._batch_shapes = shapes
+
+    def batch_limits(self, groups=-1):
+        """Limit of the next batch_setup (om_batch_limits)."""
+        self._chk(self.L.om_batch_limits(self.h, int(groups)))
 
     def batch_run(self, recompute_trajectories=False):
         outs = [np.zeros(n * m) for n, m in self._batch_shapes]

@@ -259,6 +259,7 @@ struct om_context {
   // device samples of a grid field whose om_field carries no host samples (om_adjoint_forward_dev)
   const double* dev_grid_samples = nullptr;
   int batch_wpc = 0;  // persistent batch kernel: waves per CU chosen by om_batch_tune (0: default)
+  long batch_groups = -1;  // om_batch_limits
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::string err;
@@ -1884,8 +1885,10 @@ constexpr long kBatchFixCap = 1L << 27;
 constexpr long kBatchGroupCap = 1L << 17;  // groups handed over (4.8 KB each)
 constexpr int kBatchNoHandOver = 99;  // a hand-over level above every level: none
 // Default hand-over level, by the work units: as low as the groups that leave
-// (2.2 per unit at level 12, 0.8 at 14, 0.12 at 17 with 128 to 1024 energies a
-// point) find room for, since a unit that finds none keeps its slow energies.
+// (2.2 per unit at level 12, 0.8 at 14, 0.04 to 0.05 at 17 with 128 to 1024
+// energies a point) find room for, since a unit that finds none keeps its slow
+// energies.  At level 17 the room ends at some 2.5 M units: 1.76 M hand over
+// 489 k energies in 86 k groups, 2.70 M 617 k in 115 k.
 // 13664 units, levels 0 (none) / 11 / 12 / 13 / 14 / 16: 183 / 43.9 / 40.8 / 40.6 /
 // 42.8 / 51.7 ms; 304032 units, 0 / 12 / 14 / 16 / 17 / 18: 993 / 1159 / 1139 / 888 /
 // 886 / 889 ms; 1755904 units, 0 / 14 / 16 / 17 / 18: 5096 / 5482 / 5709 / 4845 / 4848.
@@ -1919,6 +1922,7 @@ void batch_groups(om_context* ctx, om::BatchArgs& A) {
   // its points one by one
   const long most = B.mixed ? 2 * B.total_groups + B.total_points : B.total_groups;
   A.group_cap = std::min({kBatchGroupCap, std::max(4096L, 3 * B.total_items), most});
+  if (ctx->batch_groups > 0) A.group_cap = std::min(A.group_cap, ctx->batch_groups);
   B.group_list.ensure(4 * A.group_cap);
   B.group_item.ensure(A.group_cap);
   B.group_n.ensure(A.group_cap);
@@ -1937,6 +1941,13 @@ void batch_groups(om_context* ctx, om::BatchArgs& A) {
   A.part = B.part.p;
 }
 }  // namespace
+
+int om_batch_limits(om_context* ctx, long groups) {
+  return guarded(ctx, [&] {
+    if (groups < -1 || groups == 0) throw std::out_of_range("groups must be -1 or at least 1");
+    ctx->batch_groups = groups;
+  });
+}
 
 int om_batch_setup(om_context* ctx, const om_request* req, int n_req, const int* req_of, const double* weight,
                    const double* pol6, const om_conv* conv, const om_batch_opts* opts) {

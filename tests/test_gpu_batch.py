@@ -264,3 +264,43 @@ def test_small_batch_takes_little_memory(batch_case):
         assert st["n_unconverged"] == 0
         assert all(rel_err(a, b, 1e-6) < 1e-11 for a, b in zip(outs, first))
         assert dev.batch_profile(False)[1]["handed_over"] > 0 or best == 12
+
+
+@gpu
+@pytest.mark.parametrize("mode", ["tiled", "mixed"])
+@pytest.mark.parametrize("groups", [4, 40, 1416])
+def test_batch_groups_run_out(mode, groups):
+    """Fewer groups than the units ask for at the hand-over level: those that find
+    none keep their energies; and just enough for them (12 x 25 x 4 + 12 x 9 x 2),
+    so that the points of the recomputation list go on in its kernel.  Equal evaluation counts and, over several replays, the same values as
+    with everything left in its unit (the sums' order: 2^16 terms, 1e-11; mixed
+    sums carry 4.8e-9 in their sines and cosines, 1e-6)."""
+    from oscars_amd import multiparticle as M
+    from oscars_amd.sr import sr
+    parts, windows, _, _, _ = scenario(n_particles=24, seed=7)
+    grid = np.array([[x, y, 30.0] for x in np.linspace(-0.002, 0.002, 5) for y in np.linspace(-0.001, 0.001, 5)])
+    reqs = [(grid, np.linspace(140.0, 600.0, 256)), (grid[::3], np.linspace(440.0, 470.0, 100))]
+    req_of, weights = M.assign_round_robin(len(parts), len(reqs))
+    s = sr()
+    s.add_bfield_undulator(**UNDULATOR)
+    dev = s._device()
+
+    def batch(deep, limit):
+        dev.batch_limits(limit)
+        try:
+            return M.BatchedFlux(dev, s._fields, parts, windows, reqs, req_of, weights, mode=mode, deep_level=deep)
+        finally:
+            dev.batch_limits()
+    ref, st = batch(-1, -1).run(recompute_trajectories=False)
+    batch(9, -1)
+    all_handed = dev.batch_profile(False)[1]["handed_over"]
+    b = batch(9, groups)
+    cnt = dev.batch_profile(False)[1]
+    print("%s, %d groups: handed over %d of %d, listed for the recheck kernel %d, rechecked in unit %d"
+          % (mode, groups, cnt["handed_over"], all_handed, cnt["fix_listed"], cnt["rechecked_in_unit"]))
+    assert 0 < cnt["handed_over"] <= 64 * groups and (cnt["handed_over"] < all_handed) == (groups < 1416)
+    assert (cnt["fix_listed"] > 0) == (mode == "mixed" and groups == 1416)
+    for k in range(3):
+        outs, st1 = b.run(recompute_trajectories=k == 2)
+        assert st1["evals"] == st["evals"] and st1["n_unconverged"] == st["n_unconverged"] == 0
+        assert all(rel_err(x, y, 1e-6) < (1e-11 if mode == "tiled" else 1e-6) for x, y in zip(outs, ref))
