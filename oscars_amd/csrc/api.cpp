@@ -233,6 +233,10 @@ struct LaunchTimer {
 // Levels 0..kBlockLevel of a trajectory are one block of rows, built in one
 // launch (1.3 MB); deeper ones have buffers of their own.
 constexpr int kBlockLevel = 13;
+// ... but of more particles than this only the levels a sum has to have (41 KB),
+// the deeper ones as they are asked for: 1.3 MB, 2.1 as allocated, for each of
+// 100000 would be most of the memory.
+constexpr size_t kBlockParticles = 2048;
 
 // The reverse pass goes through the RK4 steps in at most this many segments
 // (eight lanes each in the map kernel: one workgroup per CU), of at least 4
@@ -1013,13 +1017,15 @@ int lw_sums(om_context* ctx, int ip, const double* obs_xyz, long n_obs, const do
     // Levels 0..8 (no point can stop before level 9) in one dense launch, then
     // one launch per level over the points still active, compacted into full
     // waves (tiles of one observation point for the tiled kernels).  Requests
-    // small enough to go on by themselves take levels 0..13 before the host looks.
-    int Lb = std::min(stop_ext, sliced || waves ? kBlockLevel : kListFrom - 1);
+    // small enough to go on by themselves take levels 0..13 before the host looks
+    // (of very many particles 0..8, the rows every particle has).
+    const int top = ctx->levels.size() > kBlockParticles ? kListFrom - 1 : kBlockLevel;
+    int Lb = std::min(stop_ext, sliced || waves ? top : kListFrom - 1);
     if (capped) Lb = stop_ext;
     long ntiles = 0;
     long n_recheck = 0;
     int Ldone = 0;  // deepest level summed so far (its samples exist)
-    const int block = ar && !(sliced || waves) ? kListFrom - 1 : kBlockLevel;
+    const int block = ar && !(sliced || waves) ? kListFrom - 1 : top;
     om::SliceArgs X;
     std::memset(&X, 0, sizeof(X));
     if (sliced) {

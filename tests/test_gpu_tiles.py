@@ -290,3 +290,40 @@ def test_adjoint_segments(npts):
         fd = (-at(2e-7) + 8 * at(1e-7) - 8 * at(-1e-7) + at(-2e-7)) / 1.2e-6
         print("npts %d angle %d: adjoint %.10e differences %.10e" % (npts, k, ga[k], fd))
         assert abs(ga[k] - fd) < 1e-4 * abs(fd)
+
+
+@gpu
+@pytest.mark.parametrize("mode", ["plain", "tiled"])
+def test_level_rows_of_many_particles(mode):
+    """Of more than 2048 particles a sum keeps the level rows it needs, here to level
+    9 or 10 of most (1023 or 2047 rows of 80 bytes; 250 KB a particle on average
+    with the deeper ones and the allocations rounded up), and not 1.3 MB.  The
+    same sums as of a particle alone, whose levels to 13 are summed before the
+    host looks (the same additions, so equal but for the sums of slices: 1e-12)."""
+    import torch
+    from oscars_amd import _lib
+    from oscars_amd.sr import sr
+    from tests.common import UNDULATOR
+    s = sr()
+    s.set_particle_beam(energy_GeV=3, x0=[0, 0, -0.1], d0=[0, 0, 1], current=0.5)
+    s.add_bfield_undulator(**UNDULATOR)
+    r = np.random.default_rng(1)
+    parts = []
+    for i in range(2100):
+        s.set_particle([1e-5 * r.standard_normal(), 0, -0.1], [2e-5 * r.standard_normal(), 0, 0.99999998])
+        parts.append(s._om_particle(s._particle, ctstart=0, ctstop=0.2, npoints=301))
+    obs, e = np.array([[1e-4, 0.0, 30.0]]), np.linspace(100.0, 400.0, 3)
+    dev, one = _lib.Device(0), _lib.Device(0)
+    dev.trajectories(s._fields, parts)
+    conv = dev.conv(precision=0.05, mode=mode)
+    dev.flux(0, obs, e, [0.0] * 6, conv)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info(0)[0]
+    res = [dev.flux(i, obs, e, [0.0] * 6, conv) for i in range(2100)]
+    used = free - torch.cuda.mem_get_info(0)[0]
+    print("%s: %.0f KB a particle" % (mode, used / 2099e3))
+    assert np.median([x[1].max() for x in res]) <= 10 and used < 2100 * 500e3
+    for i in (0, 1049, 2099):
+        one.trajectories(s._fields, [parts[i]])
+        v, lev, cv, _, _ = one.flux(0, obs, e, [0.0] * 6, conv)
+        assert np.array_equal(lev, res[i][1]) and np.array_equal(cv, res[i][2]) and rel_err(res[i][0], v) < 1e-12
