@@ -327,3 +327,52 @@ def test_level_rows_of_many_particles(mode):
         one.trajectories(s._fields, [parts[i]])
         v, lev, cv, _, _ = one.flux(0, obs, e, [0.0] * 6, conv)
         assert np.array_equal(lev, res[i][1]) and np.array_equal(cv, res[i][2]) and rel_err(res[i][0], v) < 1e-12
+
+
+def _spline(t, y):
+    """Second derivatives of the clamped spline (include/TOMATH.h:141-203), the
+    sweep in order, in the device's order of operations."""
+    n = len(t)
+    sig = (t[1:-1] - t[:-2]) / (t[2:] - t[:-2])
+    w = ((y[2:] - y[1:-1]) / (t[2:] - t[1:-1])[:, None] - (y[1:-1] - y[:-2]) / (t[1:-1] - t[:-2])[:, None])
+    w = w * 6. / (t[2:] - t[:-2])[:, None]
+    pv, u, out = np.full(n, -0.5), np.zeros_like(y), np.zeros_like(y)
+    for i in range(1, n - 1):
+        p = sig[i - 1] * pv[i - 1] + 2.0
+        pv[i] = (sig[i - 1] - 1.) / p
+        u[i] = (w[i - 1] - sig[i - 1] * u[i - 1]) / p
+    out[n - 1] = (0.0 - u[n - 2] * 0.5) / (pv[n - 2] * 0.5 + 1.)
+    for i in range(n - 2, -1, -1):
+        out[i] = pv[i] * out[i + 1] + u[i]
+    return out
+
+
+@gpu
+@pytest.mark.parametrize("total,run", [(7000, 1), (14000, 2), (28000, 4), (240000, 32)])
+def test_spline_runs(total, run):
+    """The splines of many particles, whose knots a lane takes in runs of 1 to 32:
+    runs that end inside a particle and go on in the next, or hold several whole
+    ones, and particles of 3 knots up to many runs.  Against the sweep in order:
+    the run-ups of 64 knots leave 0.27^64 = 4e-37 of a channel's scale, so that
+    only entries of that size and their roundings differ (1e-19 of the scale)."""
+    from oscars_amd.sr import sr
+    s = sr()
+    planar(s, 301)
+    lengths = [3, 4, 5, 31, 32, 33, 63, 64, 65, 66, 129, 301, 3, 3, 1400, 34]
+    while sum(lengths) < total - 1400:
+        lengths.append(lengths[(len(lengths) * 7) % 16])
+    assert min(32, -(-9 * sum(lengths) // 65536)) == run
+    r = np.random.default_rng(total)
+    parts = []
+    for n in lengths:
+        s.set_particle([1e-5 * r.standard_normal(), 0, -1], [2e-5 * r.standard_normal(), 1e-5, 0.9999999])
+        parts.append(s._om_particle(s._particle, ctstart=0, ctstop=2.0, npoints=n))
+    dev = s._device()
+    dev.trajectories(s._fields, parts)
+    n_knots = 0
+    for i in list(range(min(48, len(parts)))) + [len(parts) - 1]:
+        t, p, ypp = dev.trajectory(i)
+        ref = _spline(t, p)
+        n_knots += len(t)
+        assert np.all(np.abs(ypp - ref) <= 1e-19 * np.abs(ref).max(axis=0)), (i, len(t))
+    print("%d particles, %d knots, %d compared" % (len(parts), sum(lengths), n_knots))
