@@ -515,7 +515,9 @@ __device__ __forceinline__ void pd_term(const PdArgs& A, V3 obs, V3 nrm, const d
   V3 R = sub(obs, X);
   if (!MIXED) {
     double r2 = mag2(R);
-    double m = sqrt(r2);
+    // (where |R|^2 overflows, the term is divided by infinity whatever N is; div_by
+    // would make N a NaN of R / infinity)
+    double m = fmin(sqrt(r2), 1.79769313486231570815e308);
     double im = 1.0 / m;  // correctly rounded, so div_by gives the IEEE quotients
     V3 N1 = v3(div_by(R.x, m, im), div_by(R.y, m, im), div_by(R.z, m, im));
     // src/OSCARSSR.cc:2908: a surface without normals takes N1.normal as 1

@@ -48,6 +48,23 @@ def test_power_density_sizes(epu_pair, n):
     assert rel_err(vm, v, 1e-6) < 1e-5
 
 
+@gpu
+@pytest.mark.parametrize("z", [1e120, 1e153, 2e154, 1e160, 1e300])
+def test_power_density_far_away(epu_pair, z):
+    """Points so far that |R|^2 is near the largest double or overflows: the
+    oracle's value (0 where it overflows, as the term is divided by infinity) and
+    its level, in a few points and in as many as take several to a wave."""
+    o, dev = epu_pair
+    obs = np.column_stack([np.zeros((5000, 2)), np.full(5000, z)])
+    obs[:, 0] = 1e-3 * z * np.linspace(-1, 1, 5000)
+    ov, olev, oconv = o.power_density_surface(obs[:2], np.array([[0, 0, 1.0]] * 2), directional=True, precision=0.01,
+                                              carry_quirk=False)
+    for n in (2, 5000):
+        v, lev, cv, _ = dev.power_density(0, obs[:n], [0.0, 0.0, 1.0], True, dev.conv(precision=0.01))
+        assert np.isfinite(v).all() and np.allclose(v[:2], ov, rtol=1e-9, atol=0)
+        assert np.array_equal(lev[:2], olev) and np.array_equal(cv[:2], np.asarray(oconv, dtype=cv.dtype))
+
+
 def _field(x, name):
     from tests.common import EPU, UNDULATOR
     if name == "epu":
