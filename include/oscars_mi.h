@@ -184,9 +184,9 @@ int om_trajectory_status(om_context* ctx, int i);
 int om_trajectory_rounds(om_context* ctx, int i, int* rounds);
 /* Limits of the segmented integration in this context, from the next
  * integration on: rounds before a trajectory is integrated in order instead
- * (0: always in order; at most 32), and polls of 0.4 us that one of its
- * workgroups waits for the others (0: no wait).  -1: the default (32 rounds, a
- * poll per step).  The trajectory is the same within the last bits
+ * (0: always in order; at most 96), and polls of 0.4 us that one of its
+ * workgroups waits for the others (0: no wait).  -1: the default (32 rounds, or
+ * one for 128 steps up to 96; a poll per step).  The trajectory is the same within the last bits
  * whichever way it is integrated. */
 int om_trajectory_limits(om_context* ctx, int rounds, int polls);
 

@@ -282,7 +282,7 @@ struct om_context {
   // (nblocks 0) where the steps are taken in order
   struct Shoot {
     int nchains = 0, nblocks = 0;
-    int rounds = om::kShootRounds, polls = -1;  // om_trajectory_limits
+    int rounds = -1, polls = -1;  // om_trajectory_limits
     std::vector<om::ShootChain> chain;
     std::vector<int> block_chain, flags;
     DevBuf<om::ShootChain> d_chain;
@@ -851,7 +851,7 @@ void shoot_setup(om_context* ctx, int np) {
     longest = std::max(longest, std::max(ctx->desc[i].nf, ctx->desc[i].nb));
     total += ctx->desc[i].nf + ctx->desc[i].nb;
   }
-  if (ctx->nefields > 0 || longest < kShootMinSteps || total > kShootMaxRatio * longest || S.rounds < 1) return;
+  if (ctx->nefields > 0 || longest < kShootMinSteps || total > kShootMaxRatio * longest || S.rounds == 0) return;
   om::FieldDev none;
   std::memset(&none, 0, sizeof(none));
   const long per_step = 8L * om::kShootWaves;  // segments of a workgroup
@@ -1399,9 +1399,9 @@ int om_trajectory_status(om_context* ctx, int i) {
 
 int om_trajectory_limits(om_context* ctx, int rounds, int polls) {
   return guarded(ctx, [&] {
-    if (rounds < -1 || rounds > om::kShootRounds) throw std::out_of_range("rounds must be -1 .. 32");
+    if (rounds < -1 || rounds > om::kShootRoundsMax) throw std::out_of_range("rounds must be -1 .. 96");
     if (polls < -1) throw std::out_of_range("polls must be -1 or more");
-    ctx->shoot.rounds = rounds < 0 ? om::kShootRounds : rounds;
+    ctx->shoot.rounds = rounds;
     ctx->shoot.polls = polls;
     ctx->batch.drop_graphs();
   });

@@ -120,7 +120,7 @@ struct SliceArgs {
 
 // ---- trajectories in parallel segments (shoot.hip)
 constexpr int kShootWaves = 4;   // waves per workgroup, eight segments each
-constexpr int kShootRounds = 32;  // a chain that has not settled then is integrated in order
+constexpr int kShootRounds = 32, kShootRoundsMax = 96;  // see shoot.hip
 constexpr int kShootWalk = 64;   // maps of other workgroups held in LDS at a time
 
 // One particle's forward or backward chain of steps.
@@ -140,7 +140,7 @@ struct ShootArgs {
   int nblocks;
   double* Mb;      // 2 x 42 per workgroup: composed map of its segments, by the round's parity
   int* block_ok;   // 2 per workgroup: its joins agree
-  int rounds;      // at most
+  int rounds;      // at most; -1: by the chain's length
   int polls;       // of a wait, at most; -1: one per step of the chain
   // per chain (two per particle: forward, backward); all zero before the launch,
   // and zeroed again by rk4_kernel once it has read them

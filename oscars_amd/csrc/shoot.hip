@@ -24,7 +24,7 @@
 // Every step is the reference's, in the operation order of rk4_kernel (derivs
 // and rk4_try of rk4_common.h).  A segment in which |beta| >= 1 is met is never
 // accepted (its steps would have to be halved), nor is a chain whose joins
-// still differ after A.rounds rounds: rk4_kernel then integrates that
+// still differ after its rounds: rk4_kernel then integrates that
 // particle in order, as it does for short chains.
 //
 // Layout: one wave holds eight segments of eight lanes.  Lane 0 of a segment
@@ -64,9 +64,14 @@ namespace om {
 // rad, is sensitive to the last bit of z, and a join off by less than a bit
 // there is off by one further on.  Across, two units of the coordinate's own last
 // place: the joins' mismatches add up along the chain.  The random walk of the
-// last bits can keep a chain from settling for long: 1920 electrons through five
-// settings of fields with 3001 to 40001 points took 12 rounds at the median, 25
-// at most, and z and beta_z were those of the integration in order in every bit.
+// last bits can keep a chain from settling for long: 1920 electrons of 3 GeV
+// through five settings of fields with 3001 to 40001 points took 12 rounds at the
+// median, 25 at most, and z and beta_z were those of the integration in order in
+// every bit.  Strong fields take longer: 100 MeV in 0.3 T, 8001 points, 85; 3 GeV
+// in a 10 T wiggler, 60001 points, 60.  So a chain has kShootRounds rounds, and up
+// to kShootRoundsMax if it is long: one for 128 steps, about a quarter of the time
+// in order takes, which is what a chain that does not settle loses (coarse steps
+// of 7 cm, 3001 points: 3.2 -> 3.7 ms; the 10 T wiggler, settled, 47 -> 3.1 ms).
 constexpr double kShootPos = 1.3552527156068805e-20;      // 2^-66
 constexpr double kShootVelAlong = 5.551115123125783e-17;  // 2^-54
 constexpr double kShootVel = 2.168404344971009e-19;       // 2^-62
@@ -179,7 +184,9 @@ __global__ void __launch_bounds__(64 * kShootWaves) shoot_kernel(const ShootArgs
   double* tk = A.t + D->knot_offset;
   double* pk = A.p + 9 * D->knot_offset;
   const long nb = D->nb;
-  for (int round = 0; round < A.rounds; ++round) {
+  const long by_length = n / 128 < kShootRoundsMax ? n / 128 : kShootRoundsMax;
+  const int rounds = A.rounds >= 0 ? A.rounds : by_length > kShootRounds ? (int) by_length : kShootRounds;
+  for (int round = 0; round < rounds; ++round) {
     // lanes 1..6: the start moved along coordinate q - 1, by 2^-26 m or 2^-24 c
     // (any step between the roundings and the fields' scale serves: the
     // differences only steer the corrections)

@@ -62,6 +62,34 @@ def test_accepted_joins_are_exact_along(field, npoints, span):
     assert in_order == [(0, 0)] * 3 and all(r[0] > 1 and r[1] == 0 for r in rounds)
 
 
+@gpu
+def test_strong_fields_settle():
+    """Chains that take more rounds than an ordinary one has: 3 GeV in a 10 T
+    wiggler and 100 MeV in 0.3 T, with points for 60 and 96 rounds.  Equal to the
+    integration in order as above."""
+    from oscars_amd.sr import sr
+    more = 0
+    for energy, b, period, n_periods in ((3.0, 10.0, 0.5, 3), (0.1, 0.3, 0.049, 31)):
+        s = sr()
+        s.set_particle_beam(energy_GeV=energy, x0=[1e-5, 0, -1], d0=[1e-5, 2e-5, 1], current=0.5)
+        s.add_bfield_undulator(bfield=[0, b, 0], period=[0, 0, period], nperiods=n_periods)
+        dev = s._device()
+        for npoints in (8001, 12001, 40001, 60001):
+            part = s._om_particle(s._particle, ctstart=0, ctstop=2.0, npoints=npoints)
+            dev.trajectory_limits(rounds=0)
+            dev.trajectories(s._fields, [part])
+            t, p = knots(dev, 0)
+            dev.trajectory_limits()
+            dev.trajectories(s._fields, [part])
+            t1, p1 = knots(dev, 0)
+            rounds = dev.trajectory_rounds(0)
+            print("%g GeV, %g T, %d points: %d rounds" % (energy, b, npoints, rounds[0]))
+            more += rounds[0] > 32
+            assert np.array_equal(t1, t) and np.max(np.abs(p1[:, 2] - p[:, 2])) < 1e-19
+            assert np.array_equal(p1[:, 5], p[:, 5]) and np.max(np.abs(p1[:, :2] - p[:, :2])) < 2e-15
+    assert more > 0
+
+
 def knots(dev, i):
     return dev.trajectory(i)[:2]
 
@@ -99,7 +127,7 @@ def test_chains_given_up_are_integrated_in_order(limits):
     finally:
         dev.trajectory_limits()
     with pytest.raises(Exception):
-        dev.trajectory_limits(rounds=33)
+        dev.trajectory_limits(rounds=97)
 
 
 @gpu
