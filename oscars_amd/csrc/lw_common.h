@@ -319,7 +319,11 @@ __device__ __forceinline__ void add_replicas(double ps[6], double& maxd, double&
 // Partial sums that another XCD's wave reads in the same launch (8 x 64 doubles
 // per slice): stores that bypass the caches, with no write-back, waited for, so
 // the caller's arrival count follows them; the reader drops its caches' copies
-// once and loads them plainly, many at a time.
+// once and loads them plainly, many at a time.  The order of the stores before the
+// count rests on gfx950 (stores at agent scope are written through, vmcnt(0) waits
+// until they are where every XCD reads, the count is a later instruction of the
+// same wave), not on the language's memory model, in which nothing orders relaxed
+// accesses; a release would write the whole L2 back.
 __device__ __forceinline__ void part_publish(double* p, int lane, bool mine, const double ps[6], double maxd,
                                              double an) {
   if (mine) {

@@ -262,8 +262,13 @@ __global__ void __launch_bounds__(64 * kShootWaves) shoot_kernel(const ShootArgs
             __hip_atomic_store(Mb + 42L * ib + 7 * k + lane, v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (lane == 0) __hip_atomic_store(okb + ib, done ? 1 : 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // the map and the flag are past the caches before the arrival is; a fence
-        // here would write the knots back from L2 in every round
+        // The map and the flag are past the caches before the arrival is.  This rests
+        // on gfx950, not on the language's memory model, in which the relaxed stores
+        // are not ordered before the relaxed arrival: stores at agent scope are
+        // written through to what the XCDs share, vmcnt(0) waits until they are there,
+        // the arrival is a later instruction of the same wave, and the readers drop
+        // their caches' copies (the acquire fence below) after they have seen it.  A
+        // release fence here would write the knots back from L2 in every round.
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (lane == 0) {
           int* cnt = A.arrived + A.block_chain[ib];

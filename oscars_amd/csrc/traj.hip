@@ -364,9 +364,10 @@ __global__ void __launch_bounds__(64) rk4_kernel(const UndParams f_arg, const Gr
 // include/TOMATH.h:141-203.  spline_pre_kernel computes, in parallel, the
 // parts of the tridiagonal sweep that do not depend on the previous knot:
 // sig_i, sig_i - 1 and w_i = (secant difference) * 6 / (t[i+1] - t[i-1]) per
-// channel.  spline_kernel then runs the sequential recurrences
+// channel.  spline_p_kernel and spline_u_kernel then run the recurrences
 //   p = sig*ypp[i-1] + 2,  ypp[i] = (sig-1)/p,  u[i] = (w_i - sig*u[i-1])/p
-// and the back substitution, one lane per (particle, channel).
+// and spline_b_kernel the back substitution, each knot (or run of knots) from
+// kSplineWin knots before it.
 __global__ void __launch_bounds__(256) spline_pre_kernel(const TrajDesc* __restrict__ desc, int np,
                                                          const double* __restrict__ t, const double* __restrict__ p,
                                                          double* __restrict__ sig, double* __restrict__ sm1,

@@ -146,9 +146,9 @@ def test_sr_nparticles_batched_matches_particle_loop():
 @gpu
 @pytest.mark.parametrize("mode,tol", [("tiled", 1e-9), ("mixed", 1e-5)])
 def test_batched_hand_over_matches_oracle(batch_case, mode, tol):
-    """deep_level=10: every point still active at level 10 is finished by the
-    workgroup-per-point kernel from its handed-over state (and, mixed, its
-    borderline points by the FP64 recheck kernel) instead of inside its unit.
+    """deep_level=10: every point still active at level 10 leaves its unit in a
+    group and goes on level by level (and, mixed, its borderline points by the
+    FP64 recheck kernel) instead of inside its unit.
     Same bar against the oracle, same evaluation count as the default."""
     from oscars_amd import multiparticle as M
     from oscars_amd.sr import sr
@@ -176,8 +176,8 @@ def test_batched_hand_over_matches_oracle(batch_case, mode, tol):
 def test_batched_mixed_levels_match_fp64(deep_level):
     """Mixed batch against the FP64 batch on a denser case: identical levels
     (equal evaluation counts: borderline points are recomputed in FP64 inside
-    the same graph, in their unit or, for points handed over at deep_level, by
-    the recheck kernel) and per-point agreement to 1e-5."""
+    the same graph, in their unit or, for points handed over at deep_level (0: at
+    level 12 here), by the recheck kernel) and per-point agreement to 1e-5."""
     from oscars_amd import multiparticle as M
     from oscars_amd.sr import sr
     parts, windows, _, _, _ = scenario(n_particles=24, seed=7)

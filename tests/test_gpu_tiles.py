@@ -84,7 +84,8 @@ def _field(x, name):
 def test_trajectory_in_segments(field):
     """Chains cut into segments and joined, one to 53 workgroups long, with
     remainders, T0 at the start, inside and at the end of the window, beside
-    chains too short to be cut.  Against the oracle's integration in order: times equal; positions
+    chains of one step; every one accepted, none left to the integration in order.
+    Against the oracle's integration in order: times equal; positions
     along the trajectory within two units in the last place of 1 m (2^-52: the
     joins agree to a fraction of one), transverse ones and velocities to 1e-12 of
     their largest value (the device's sine differs from the C library's in the
@@ -109,6 +110,8 @@ def test_trajectory_in_segments(field):
         o.set_npoints_trajectory(n)
         T = o.calculate_trajectory()
         t, p, _ = dev.trajectory(i)
+        rounds = dev.trajectory_rounds(i)
+        assert rounds[0] > 0 and (rounds[1] > 0) == (a < 0), (a, b, n, rounds)
         scale = np.max(np.abs(T.p), axis=0)
         scale[scale == 0] = 1
         err = np.max(np.abs(p - T.p) / scale, axis=0)
@@ -135,6 +138,7 @@ def test_many_trajectories_in_segments():
     dev = s._device()
     dev.trajectories(s._fields, parts)
     many = [dev.trajectory(i) for i in (0, 74, 149)]
+    assert all(min(dev.trajectory_rounds(i)) > 0 for i in range(150))
     for (t, p, _), i in zip(many, (0, 74, 149)):
         dev.trajectories(s._fields, [parts[i]])
         t1, p1, _ = dev.trajectory(0)
