@@ -186,8 +186,8 @@ int om_trajectory_rounds(om_context* ctx, int i, int* rounds);
  * integration on: rounds before a trajectory is integrated in order instead
  * (0: always in order; at most 96), and polls of 0.4 us that one of its
  * workgroups waits for the others (0: no wait).  -1: the default (32 rounds, or
- * one for 128 steps up to 96; a poll per step).  The trajectory is the same within the last bits
- * whichever way it is integrated. */
+ * one for 128 steps of the longest trajectory up to 96; a poll per step).  The
+ * trajectory is the same within the last bits whichever way it is integrated. */
 int om_trajectory_limits(om_context* ctx, int rounds, int polls);
 
 /* Flux on n_obs observation points x n_e photon energies (point index

@@ -283,6 +283,7 @@ struct om_context {
   struct Shoot {
     int nchains = 0, nblocks = 0;
     int rounds = -1, polls = -1;  // om_trajectory_limits
+    int by_length = om::kShootRounds;  // rounds where rounds is -1
     std::vector<om::ShootChain> chain;
     std::vector<int> block_chain, flags;
     DevBuf<om::ShootChain> d_chain;
@@ -852,6 +853,7 @@ void shoot_setup(om_context* ctx, int np) {
     total += ctx->desc[i].nf + ctx->desc[i].nb;
   }
   if (ctx->nefields > 0 || longest < kShootMinSteps || total > kShootMaxRatio * longest || S.rounds == 0) return;
+  S.by_length = (int) std::max((long) om::kShootRounds, std::min((long) om::kShootRoundsMax, longest / 128));
   om::FieldDev none;
   std::memset(&none, 0, sizeof(none));
   const long per_step = 8L * om::kShootWaves;  // segments of a workgroup
@@ -912,7 +914,7 @@ void launch_trajectories(om_context* ctx, int np) {
     A.block_chain = S.d_block_chain.p;
     A.nblocks = S.nblocks;
     A.Mb = S.maps.p;
-    A.rounds = S.rounds;
+    A.rounds = S.rounds >= 0 ? S.rounds : S.by_length;
     A.polls = S.polls;
     A.done = S.d_flags.p;
     A.arrived = S.d_flags.p + S.nchains;

@@ -140,7 +140,7 @@ struct ShootArgs {
   int nblocks;
   double* Mb;      // 2 x 42 per workgroup: composed map of its segments, by the round's parity
   int* block_ok;   // 2 per workgroup: its joins agree
-  int rounds;      // at most; -1: by the chain's length
+  int rounds;      // at most
   int polls;       // of a wait, at most; -1: one per step of the chain
   // per chain (two per particle: forward, backward); all zero before the launch,
   // and zeroed again by rk4_kernel once it has read them

@@ -68,10 +68,11 @@ namespace om {
 // through five settings of fields with 3001 to 40001 points took 12 rounds at the
 // median, 25 at most, and z and beta_z were those of the integration in order in
 // every bit.  Strong fields take longer: 100 MeV in 0.3 T, 8001 points, 85; 3 GeV
-// in a 10 T wiggler, 60001 points, 60.  So a chain has kShootRounds rounds, and up
-// to kShootRoundsMax if it is long: one for 128 steps, about a quarter of the time
-// in order takes, which is what a chain that does not settle loses (coarse steps
-// of 7 cm, 3001 points: 3.2 -> 3.7 ms; the 10 T wiggler, settled, 47 -> 3.1 ms).
+// in a 10 T wiggler, 60001 points, 60.  So there are kShootRounds rounds, and up
+// to kShootRoundsMax where a chain is long: one for 128 steps, about a quarter of
+// the time in order takes, which is what a chain that does not settle loses (steps
+// of 7 cm, 3001 points: 3.3 -> 4.1 ms; 100 MeV in 0.3 T, 2001 points: 1.4 -> 2.1;
+// the 10 T wiggler, settled, 39 -> 3.1 ms).
 constexpr double kShootPos = 1.3552527156068805e-20;      // 2^-66
 constexpr double kShootVelAlong = 5.551115123125783e-17;  // 2^-54
 constexpr double kShootVel = 2.168404344971009e-19;       // 2^-62
@@ -184,9 +185,7 @@ __global__ void __launch_bounds__(64 * kShootWaves) shoot_kernel(const ShootArgs
   double* tk = A.t + D->knot_offset;
   double* pk = A.p + 9 * D->knot_offset;
   const long nb = D->nb;
-  const long by_length = n / 128 < kShootRoundsMax ? n / 128 : kShootRoundsMax;
-  const int rounds = A.rounds >= 0 ? A.rounds : by_length > kShootRounds ? (int) by_length : kShootRounds;
-  for (int round = 0; round < rounds; ++round) {
+  for (int round = 0; round < A.rounds; ++round) {
     // lanes 1..6: the start moved along coordinate q - 1, by 2^-26 m or 2^-24 c
     // (any step between the roundings and the fields' scale serves: the
     // differences only steer the corrections)
