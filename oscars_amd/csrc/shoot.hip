@@ -36,9 +36,10 @@
 // workgroups of a chain wait for each other once a round, and each walks the
 // compositions before its own.  One launch for everything (as two launches a
 // round, segments and walk, the 20001-point planar chain took 0.30 ms of kernels
-// and 36 launches).  Measured: planar 20001 points 12.4 -> 0.17 ms, EPU 40001
-// points 37.5 -> 0.44 ms, 1-D map 20001 points 18.1 -> 0.3 ms, undulator and
-// Gaussian 8001 points 23.7 -> 0.5 ms.
+// and 36 launches).  Measured, by the rounds an electron takes: planar 20001 points
+// 12.4 -> 0.16 to 0.24 ms, EPU 40001 points 37.5 -> 0.39 to 0.55 ms, 1-D map 20001
+// points 18.1 -> 0.40 to 0.57 ms, undulator and Gaussian 8001 points 23.7 -> 0.4 to
+// 1.05 ms (8 to 24 rounds).
 //
 // The wait is bounded: if the workgroups of a chain cannot all be resident,
 // because other work fills the GPU, the first whose wait runs out gives the chain
